@@ -22,14 +22,29 @@
 // Reference: triangle_attn/module.py:57-125 and benchmarks/references.py:174-205 (the op),
 // triangle_attn/kernel.py:230-238 (-1e9 pair mask), :282-290 (D = 16 keeps separate K / V
 // weights), tests/test_triangle_attn.py:137-192 (the Apo shape).
+#include <initializer_list>
+
 #include "capi.hpp"
 #include "common.hpp"
 #include "generic.hpp"
+#include "tile_mma.hpp"
 
 namespace tops {
 
 constexpr int kGenTok = 16;  // tokens per block; 16 lanes per token for the LayerNorm sums
 constexpr int kTK = 32;      // k-tile of the weights the tiled kernels stage through LDS
+
+// Conditions of a kernel's 16-byte accesses (a null pointer is not accessed).
+static bool aligned16(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if ((uintptr_t)p % 16 != 0) return false;
+  return true;
+}
+static bool multiples_of(int n, std::initializer_list<int64_t> vs) {
+  for (int64_t v : vs)
+    if (v % n != 0) return false;
+  return true;
+}
 
 // LayerNorm of kGenTok token rows held in LDS (fp32, row length C, row stride ld): 16
 // consecutive lanes per token, two-pass statistics.  Writes normalised rows back in place.
@@ -248,58 +263,74 @@ __global__ __launch_bounds__(256, 2) void tri_generic_attn_kernel(const T* __res
 }
 
 // ---------------------------------------------------------------------------------------------
-// Gate + output projection, any (C_in, HD, C_out): 256 threads per kGenTok tokens.
+// Gate + output projection, any (C_in, HD, C_out): 32 tokens per block of NW waves.  Both input
+// tiles are staged in LDS; each wave takes 32-feature chunks of the two products in turn (weights
+// from L2 as the A operand, tokens as B), so a lane ends up with 16 consecutive features of one
+// token: the gated activations overwrite the o tile in place and the output is stored in 16-byte
+// pieces.  Few tokens are bound by the latency of the weight reads (600 tokens, C = HD = 384, bf16:
+// 373 -> 20 us against a thread per output), many by the matrix cores in fp32 (262144 tokens, C = HD =
+// 128: 206 us, 83 TFLOP/s) and by memory otherwise (the same in bf16: 771 -> 79 us).  32 tokens per
+// block: 64 were 2 % faster at C = 128 and 15 % slower at C = 64 (fewer blocks per CU).
 // ---------------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void gate_generic_kernel(const T* __restrict__ o, int64_t so0, int64_t so1,
-                                                          const T* __restrict__ gin, int64_t sg0, int64_t sg1,
-                                                          const T* __restrict__ w_ln, const T* __restrict__ b_ln,
-                                                          float eps, int apply_ln, const T* __restrict__ Wg,
-                                                          const T* __restrict__ bg, const T* __restrict__ Wo,
-                                                          const T* __restrict__ bo, const T* __restrict__ res,
-                                                          int64_t sr0, int64_t sr1, T* __restrict__ out, int64_t sd0,
-                                                          int64_t sd1, int64_t M1, int64_t M2, int Cin, int HD,
-                                                          int Cout) {
-  extern __shared__ float sm[];
-  float* gs = sm;                   // [kGenTok][Cin]  gate input (normalised)
-  float* ys = sm + kGenTok * Cin;   // [kGenTok][HD]   o, then the gated activations
-  const int tid = threadIdx.x;
-  const int64_t M = M1 * M2, tok0 = (int64_t)blockIdx.x * kGenTok;
-  for (int e = tid; e < kGenTok * Cin; e += 256) {
-    const int64_t tok = tok0 + e / Cin;
-    float v = 0.f;
-    if (tok < M) v = (float)gin[(tok / M2) * sg0 + (tok % M2) * sg1 + e % Cin];
-    gs[e] = v;
-  }
-  for (int e = tid; e < kGenTok * HD; e += 256) {
-    const int64_t tok = tok0 + e / HD;
-    float v = 0.f;
-    if (tok < M) v = (float)o[(tok / M2) * so0 + (tok % M2) * so1 + e % HD];
-    ys[e] = v;
-  }
-  __syncthreads();
-  if (apply_ln) gen_layer_norm<T>(gs, Cin, Cin, w_ln, b_ln, eps);
-  __syncthreads();
-  for (int e = tid; e < kGenTok * HD; e += 256) {
-    const int t = e / HD, j = e % HD;
-    const float* g = gs + t * Cin;
-    const T* w = Wg + (int64_t)j * Cin;
-    float acc = bg ? (float)bg[j] : 0.f;
-    for (int c = 0; c < Cin; ++c) acc = fmaf((float)(T)g[c], (float)w[c], acc);
-    ys[e] = (float)(T)(ys[e] * sigmoid(acc));
+template <typename T, int NW, bool VEC>
+__global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restrict__ o, int64_t so0, int64_t so1,
+                                                              const T* __restrict__ gin, int64_t sg0, int64_t sg1,
+                                                              const T* __restrict__ w_ln, const T* __restrict__ b_ln,
+                                                              float eps, int apply_ln, const T* __restrict__ Wg,
+                                                              const T* __restrict__ bg, const T* __restrict__ Wo,
+                                                              const T* __restrict__ bo, const T* __restrict__ res,
+                                                              int64_t sr0, int64_t sr1, T* __restrict__ out,
+                                                              int64_t sd0, int64_t sd1, int64_t M1, int64_t M2,
+                                                              int Cin, int HD, int Cout) {
+  constexpr int TT = 32, TPT = 64 * NW / TT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int rg = tile_row<T>(Cin), ry = tile_row<T>(HD);
+  T* gs = reinterpret_cast<T*>(smem);  // [TT][rg] gate input (normalised)
+  T* ys = gs + TT * rg;                // [TT][ry] o, then the gated activations
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const int64_t M = M1 * M2, tok0 = (int64_t)blockIdx.x * TT;
+  {
+    const int t = tid / TPT, part = tid % TPT;
+    const bool ok = tok0 + t < M;
+    const int64_t tok = ok ? tok0 + t : M - 1, m1 = tok / M2, m2 = tok - m1 * M2;
+    stage_row<T, TPT, VEC>(gs + t * rg, gin + m1 * sg0 + m2 * sg1, ok, part, Cin, tile_kp(Cin));
+    stage_row<T, TPT, VEC>(ys + t * ry, o + m1 * so0 + m2 * so1, ok, part, HD, tile_kp(HD));
+    if (apply_ln) {
+      float mean, rstd;
+      row_stats<T, TPT>(gs + t * rg, part, Cin, eps, mean, rstd);
+      normalise_row<T, TPT>(gs + t * rg, part, Cin, mean, rstd, w_ln, b_ln);
+    }
   }
   __syncthreads();
-  for (int e = tid; e < kGenTok * Cout; e += 256) {
-    const int t = e / Cout, c = e % Cout;
-    const int64_t tok = tok0 + t;
-    if (tok >= M) continue;
-    const float* y = ys + t * HD;
-    const T* w = Wo + (int64_t)c * HD;
-    float acc = bo ? (float)bo[c] : 0.f;
-    for (int j = 0; j < HD; ++j) acc = fmaf(y[j], (float)w[j], acc);
-    const int64_t m1 = tok / M2, m2 = tok % M2;
-    // with a residual: out = res + result, the result rounded first as a separate add would see it
-    out[m1 * sd0 + m2 * sd1 + c] = res ? (T)((float)res[m1 * sr0 + m2 * sr1 + c] + (float)(T)acc) : (T)acc;
+  // gate: ys = io(o * sigmoid(g . Wg + bg)), each element rewritten by the lane that reads it
+  for (int f0 = 32 * wave; f0 < HD; f0 += 32 * NW) {
+    const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
+    f32x16 acc[1] = {};
+    tile_gemm<T, 1, true, VEC>(acc, gs, rg, col, Wg + (int64_t)(row < HD ? row : HD - 1) * Cin, Cin);
+    const f32x16 b = load16<T, VEC>(bg && fl < HD ? bg + fl : nullptr, HD - fl);
+    T* y = ys + col * ry + fl;
+    store16<T, true>(y, 16, [&](int v) __attribute__((always_inline)) {
+      return (T)((float)y[v] * sigmoid(acc[0][v] + b[v]));
+    });
+  }
+  __syncthreads();
+  // output projection; with a residual, the result is rounded first as a separate add would see it
+  const int64_t tok = tok0 + col < M ? tok0 + col : M - 1, m1 = tok / M2, m2 = tok - m1 * M2;
+  for (int f0 = 32 * wave; f0 < Cout; f0 += 32 * NW) {
+    const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
+    f32x16 acc[1] = {};
+    tile_gemm<T, 1, true, VEC>(acc, ys, ry, col, Wo + (int64_t)(row < Cout ? row : Cout - 1) * HD, HD);
+    if (tok0 + col >= M || fl >= Cout) continue;
+    const f32x16 b = load16<T, VEC>(bo ? bo + fl : nullptr, Cout - fl);
+    T* dst = out + m1 * sd0 + m2 * sd1 + fl;
+    if (res) {
+      const f32x16 r = load16<T, VEC>(res + m1 * sr0 + m2 * sr1 + fl, Cout - fl);
+      store16<T, VEC>(dst, Cout - fl,
+                      [&](int v) __attribute__((always_inline)) { return (T)(r[v] + (float)(T)(acc[0][v] + b[v])); });
+    } else {
+      store16<T, VEC>(dst, Cout - fl, [&](int v) __attribute__((always_inline)) { return (T)(acc[0][v] + b[v]); });
+    }
   }
 }
 
@@ -487,47 +518,6 @@ __global__ __launch_bounds__(256) void tri_gen_prep_tiled_kernel(const T* __rest
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void gate_gen_tiled_kernel(const T* __restrict__ o, int64_t so0, int64_t so1,
-                                                            const T* __restrict__ gin, int64_t sg0, int64_t sg1,
-                                                            const T* __restrict__ w_ln, const T* __restrict__ b_ln,
-                                                            float eps, int apply_ln, const T* __restrict__ Wg,
-                                                            const T* __restrict__ bg, const T* __restrict__ Wo,
-                                                            const T* __restrict__ bo, const T* __restrict__ res,
-                                                            int64_t sr0, int64_t sr1, T* __restrict__ out,
-                                                            int64_t sd0, int64_t sd1, int64_t M1, int64_t M2, int Cin,
-                                                            int HD, int Cout) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CinK = (Cin + kTK - 1) / kTK * kTK, HDK = (HD + kTK - 1) / kTK * kTK;
-  float* gs = sm;                  // [CinK][kGRow] gate input (normalised), k-major
-  float* ys = gs + CinK * kGRow;   // [HDK][kGRow]  o, then the gated activations
-  float* ws = ys + HDK * kGRow;    // [kTK][kGRow]
-  const int tid = threadIdx.x;
-  const int64_t M = M1 * M2, tok0 = (int64_t)blockIdx.x * kGT;
-  const int ntok = (int)(M - tok0 < kGT ? M - tok0 : kGT);
-  tiled_load_rows<T>(gs, gin, Cin, CinK, ntok, [=](int t) {
-    const int64_t tok = tok0 + t;
-    return (tok / M2) * sg0 + (tok % M2) * sg1;
-  });
-  tiled_load_rows<T>(ys, o, HD, HDK, ntok, [=](int t) {
-    const int64_t tok = tok0 + t;
-    return (tok / M2) * so0 + (tok % M2) * so1;
-  });
-  __syncthreads();
-  if (apply_ln) tiled_ln_affine<T>(gs, Cin, CinK, w_ln, b_ln, eps);
-  // gate: ys[j][t] = io(o * sigmoid(io(g) . Wg[j] + bg[j])), each element rewritten by the thread that reads it
-  tiled_gemm64<T, true, 1>(gs, Cin, CinK, Wg, HD, ws, kGT, [=](int t, int j, float v) {
-    const float g = v + (bg ? (float)bg[j] : 0.f);
-    ys[j * kGRow + t] = (float)(T)(ys[j * kGRow + t] * sigmoid(g));
-  });
-  // output projection of the gated tile; with a residual, the result is rounded first
-  tiled_gemm64<T, false, 1>(ys, HD, HDK, Wo, Cout, ws, ntok, [=](int t, int c, float v) {
-    const T r = (T)(v + (bo ? (float)bo[c] : 0.f));
-    const int64_t tok = tok0 + t, m1 = tok / M2, m2 = tok % M2;
-    out[m1 * sd0 + m2 * sd1 + c] = res ? (T)((float)res[m1 * sr0 + m2 * sr1 + c] + (float)r) : r;
-  });
-}
-
-template <typename T>
 static int tri_generic_prep_t(const void* x, int64_t sx0, int64_t sx1, const void* w_ln, const void* b_ln,
                               int apply_ln, const void* wqkv, const void* WZ, const float* BZ, void* xln, void* q,
                               void* k, void* v, float* bias, int64_t N, int C, int H, int D, float eps,
@@ -578,23 +568,35 @@ static int gate_generic_t(const void* o, int64_t so0, int64_t so1, const void* g
                           const void* Wo, const void* bo, const void* res, int64_t sr0, int64_t sr1, void* out,
                           int64_t sd0, int64_t sd1, int64_t M1, int64_t M2, int Cin, int HD, int Cout,
                           hipStream_t st) {
-  const int64_t tiles = (M1 * M2 + kGT - 1) / kGT;
-  if (Cin <= 256 && HD <= 256 && tiles >= num_cus()) {  // tiled kernel: 64 tokens per block
-    const int CinK = (Cin + kTK - 1) / kTK * kTK, HDK = (HD + kTK - 1) / kTK * kTK;
-    const size_t lds = (size_t)(CinK + HDK + kTK) * kGRow * sizeof(float);
-    hipFuncSetAttribute((const void*)gate_gen_tiled_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((gate_gen_tiled_kernel<T>), dim3((unsigned)tiles), dim3(256), lds, st, (const T*)o, so0, so1,
-                       (const T*)gin, sg0, sg1, (const T*)w_ln, (const T*)b_ln, eps, apply_ln, (const T*)Wg,
-                       (const T*)bg, (const T*)Wo, (const T*)bo, (const T*)res, sr0, sr1, (T*)out, sd0, sd1, M1, M2,
-                       Cin, HD, Cout);
-    return launched(res ? "tops_gate_out_generic_residual" : "tops_gate_out_generic");
+  const int64_t M = M1 * M2;
+  if (M == 0) return TOPS_OK;
+  using V = TileMma<T>;
+  const bool vec = aligned16({gin, o, Wg, bg, Wo, bo, res, out}) &&
+                   multiples_of(V::VE, {sg0, sg1, so0, so1, sr0, sr1, sd0, sd1, Cin, HD, Cout});
+  const size_t lds = (size_t)32 * (tile_row<T>(Cin) + tile_row<T>(HD)) * sizeof(T);
+#define TOPS_GEN_GATE(NW, VEC)                                                                                      \
+  do {                                                                                                              \
+    const void* fn = (const void*)gate_generic_kernel<T, NW, VEC>;                                                  \
+    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                            \
+    hipLaunchKernelGGL((gate_generic_kernel<T, NW, VEC>), dim3((unsigned)((M + 31) / 32)), dim3(64 * NW), lds, st,  \
+                       (const T*)o, so0, so1, (const T*)gin, sg0, sg1, (const T*)w_ln, (const T*)b_ln, eps,         \
+                       apply_ln, (const T*)Wg, (const T*)bg, (const T*)Wo, (const T*)bo, (const T*)res, sr0, sr1,    \
+                       (T*)out, sd0, sd1, M1, M2, Cin, HD, Cout);                                                   \
+  } while (0)
+  // 16 waves per block while every block has a CU to itself (bf16 / fp32, 6000 tokens x 384: 21 / 49 us
+  // against 23 / 57 with 4; 8000 x 128: equal), 4 beyond (16000 x 128: 10 / 16 against 11 / 19)
+  if ((M + 31) / 32 <= num_cus()) {
+    if (vec)
+      TOPS_GEN_GATE(16, true);
+    else
+      TOPS_GEN_GATE(16, false);
+  } else {
+    if (vec)
+      TOPS_GEN_GATE(4, true);
+    else
+      TOPS_GEN_GATE(4, false);
   }
-  const int64_t blocks = (M1 * M2 + kGenTok - 1) / kGenTok;
-  if (blocks == 0) return TOPS_OK;
-  hipLaunchKernelGGL((gate_generic_kernel<T>), dim3((unsigned)blocks), dim3(256),
-                     (size_t)kGenTok * (Cin + HD) * sizeof(float), st, (const T*)o, so0, so1, (const T*)gin, sg0, sg1,
-                     (const T*)w_ln, (const T*)b_ln, eps, apply_ln, (const T*)Wg, (const T*)bg, (const T*)Wo,
-                     (const T*)bo, (const T*)res, sr0, sr1, (T*)out, sd0, sd1, M1, M2, Cin, HD, Cout);
+#undef TOPS_GEN_GATE
   return launched(res ? "tops_gate_out_generic_residual" : "tops_gate_out_generic");
 }
 
