@@ -26,8 +26,8 @@ def _within(out, ref, bound, name):
     assert worst <= 1.0, f"{name}: {worst:.2f} of the bound, max |d| {d.max().item():.2e}"
 
 
-# tokens: one, one short of and past a 32- and a 64-token tile, past the one-tile-per-CU rule
-# (32 * 256 tokens) and past the 64-token rule (64 * 8 * 256 tokens)
+# tokens: one, one short of and past a 32-token tile and past two, past the one-tile-per-CU rule
+# (32 * 256 tokens), and thousands of blocks
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("M,Cin,HD,Cout", [(1, 64, 64, 64), (31, 384, 384, 384), (65, 33, 40, 7), (8225, 96, 72, 100),
                                            (8225, 24, 24, 24), (131137, 32, 32, 32), (33, 512, 512, 130)])
@@ -50,7 +50,7 @@ def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
     slack = 0.0
     if extras:
         gd = torch.nn.functional.layer_norm(gd, (Cin,), w_ln.double(), b_ln.double(), 1e-5).to(dtype).double()
-        slack = gd.abs() @ wg.double().T.abs() / 4  # the sigmoid's slope
+        slack = (gd.abs() + 1e-2) @ wg.double().T.abs() / 4  # the sigmoid's slope; see size below for small values
     z = gd @ wg.double().T + (bg.double() if extras else 0.0)
     y = (od * torch.sigmoid(z)).to(dtype).double()
     ref = y @ wo.double().T + (bo.double() if extras else 0.0)
@@ -60,3 +60,61 @@ def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
         ref = res.double() + ref
         bound = bound + EPS[dtype] * ref.abs()
     _within(out, ref, bound, f"gate {dtype} {M} {Cin} {HD} {Cout}")
+
+
+# grids of one token, one short of and past a 32-token tile, a few thousand blocks;
+# head widths of every store width, C of one and several k batches and with a tail
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("N,C,H,D", [(1, 64, 2, 64), (6, 24, 3, 24), (9, 40, 5, 10), (13, 33, 2, 12), (21, 200, 9, 16),
+                                     (33, 1024, 4, 64), (130, 128, 4, 32)])
+@pytest.mark.parametrize("ln", [False, True])
+def test_tri_prep_any_shape(device, dtype, N, C, H, D, ln):
+    """LN(x), Q / K / V and the pair bias of a transposed view (ln) or of a channel slice."""
+    from triangleops_amd.triangle_attn.kernel import generic_prep_forward
+
+    g = torch.Generator().manual_seed(N + C)
+    x = _rnd(g, dtype, N, N, C).transpose(0, 1) if ln else _rnd(g, dtype, N, N, C + 1)[..., :C]
+    w, wz = _rnd(g, dtype, H, 3, D, C, scale=C**-0.5), _rnd(g, dtype, H, C, scale=C**-0.5)
+    w_ln, b_ln, bz = _rnd(g, dtype, C), _rnd(g, dtype, C), _rnd(g, torch.float32, H)
+    xd = x.to(device) if not ln else x.transpose(0, 1).contiguous().to(device).transpose(0, 1)
+    out = generic_prep_forward(xd, w_ln.to(device), b_ln.to(device), w.to(device), wz.to(device), bz.to(device),
+                               apply_ln=ln)
+    xn = x.double()
+    size = xn.abs()  # of what an element is summed from: x and the mean, the scaled result and the bias may cancel
+    if ln:
+        mean, std = xn.mean(-1, keepdim=True), (xn.var(-1, correction=0, keepdim=True) + 1e-5).sqrt()
+        size = (xn.abs() + mean.abs()) / std * w_ln.double().abs() + b_ln.double().abs()
+        xn = torch.nn.functional.layer_norm(xn, (C,), w_ln.double(), b_ln.double(), 1e-5)
+    xr = xn.to(dtype).double()
+    _within(out[0], xr, EPS[dtype] * xr.abs() + EPS[torch.float32] * size, "xln")
+    for i, name in enumerate("qkv"):
+        wi = w[:, i].double().reshape(H * D, C)
+        ref = (xr @ wi.T).view(N, N, H, D)
+        bound = EPS[dtype] * (ref.abs() + (xr.abs() @ wi.abs().T).view(N, N, H, D) + 1e-3)
+        _within(out[1 + i], ref, bound, name)
+    ref = (xn @ wz.double().T + bz.double()).permute(2, 0, 1)
+    bound = EPS[torch.float32] * ((xn.abs() @ wz.double().abs().T).permute(2, 0, 1) + 1.0)
+    _within(out[4], ref, bound, "bias")
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("M,C,H,D", [(1, 8, 1, 8), (31, 384, 16, 24), (33, 30, 3, 10), (65, 512, 2, 64), (64, 520, 3, 20),
+                                     (40, 1100, 5, 16)])
+def test_apb_qkv_any_shape(device, dtype, M, C, H, D):
+    """Q / K / V at one, exactly one and several 512-channel stages, odd channel counts and head widths."""
+    from triangleops_amd import _native
+    from triangleops_amd._common.dtype import any_shape_dtype_code
+
+    g = torch.Generator().manual_seed(M + C)
+    x, w = _rnd(g, dtype, M, C), _rnd(g, dtype, H, 3, D, C, scale=C**-0.5)
+    xd, wd, z = x.to(device), w.to(device), torch.zeros(M, M, 8, device=device, dtype=dtype)
+    wc, bc = torch.zeros(H, 8, device=device), torch.zeros(H, device=device)
+    out = torch.empty(3, M, H * D, device=device, dtype=dtype)  # rows of odd sizes: misaligned k and v
+    bias = torch.empty(H, M, M, device=device)
+    _native.call("tops_apb_generic_prep", xd.data_ptr(), wd.data_ptr(), z.data_ptr(), M * 8, 8, wc.data_ptr(),
+                 bc.data_ptr(), *(o.data_ptr() for o in out), bias.data_ptr(), M, C, 8, H, D, 1e-5,
+                 any_shape_dtype_code(dtype), _native.stream_of(xd))
+    for i, name in enumerate("qkv"):
+        wi = w[:, i].double().reshape(H * D, C)
+        ref = x.double() @ wi.T
+        _within(out[i], ref, EPS[dtype] * (ref.abs() + x.double().abs() @ wi.abs().T + 1e-3), name)

@@ -23,6 +23,7 @@
 // triangle_attn/kernel.py:230-238 (-1e9 pair mask), :282-290 (D = 16 keeps separate K / V
 // weights), tests/test_triangle_attn.py:137-192 (the Apo shape).
 #include <initializer_list>
+#include <type_traits>
 
 #include "capi.hpp"
 #include "common.hpp"
@@ -64,10 +65,56 @@ __device__ void gen_layer_norm(float* rows, int ld, int C, const T* w_ln, const 
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Pre-pass: 256 threads per kGenTok tokens.  xs holds the fp32 rows, LN'd in place.
-// ---------------------------------------------------------------------------------------------
+// Writes 16 consecutive rows f0 .. f0 + 15 (f(v), v < n) of the (H, 3, D) projection of one token to
+// its q, k and v rows, in pieces of pw elements.
+template <typename T, typename F>
+__device__ __attribute__((always_inline)) inline void store_qkv16(T* qo, T* ko, T* vo, int64_t row, int f0, int n,
+                                                                  int D, int pw, F f) {
+  // the destination is picked by integer selects on address offsets (a pointer choice among the three
+  // becomes a table in private memory)
+  const uint64_t aq = (uint64_t)qo, dk = (uint64_t)ko - aq, dv = (uint64_t)vo - aq;
+  auto dst = [&](int fr) __attribute__((always_inline)) {
+    const int h = fr / (3 * D), r = fr - h * 3 * D, which = r / D;
+    return reinterpret_cast<T*>(aq + (which == 1 ? dk : 0) + (which == 2 ? dv : 0)) + row + h * D + (r - which * D);
+  };
+  auto pieces = [&](auto tag) __attribute__((always_inline)) {
+    constexpr int W = decltype(tag)::value;
+#pragma unroll
+    for (int c = 0; c < 16; c += W) {
+      if (c >= n) continue;
+      vec<T, W> r;
+#pragma unroll
+      for (int e = 0; e < W; ++e) r[e] = (T)f(c + e);
+      *reinterpret_cast<vec<T, W>*>(dst(f0 + c)) = r;
+    }
+  };
+  if (pw == TileMma<T>::VE)
+    pieces(std::integral_constant<int, TileMma<T>::VE>{});
+  else if (pw == 4)
+    pieces(std::integral_constant<int, 4>{});
+  else
+    pieces(std::integral_constant<int, 1>{});
+}
+
+// The widest piece (VE, 4 or 1 elements) that divides D and that the three outputs are aligned to.
 template <typename T>
+static int qkv_piece(int D, const void* q, const void* k, const void* v) {
+  for (int w : {TileMma<T>::VE, 4})
+    if (D % w == 0 && ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % (w * sizeof(T)) == 0) return w;
+  return 1;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Pre-pass: 32 tokens per block of 4 waves.  LN(x) in LDS (rounded to the I/O type, also written out
+// as xln), Q / K / V of all heads on the matrix cores (a wave takes 32-row chunks of the weight in
+// turn), the row-shared pair bias from the unrounded LN(x) in fp32 FMAs by the threads that normalise
+// the rows (H is small: an MFMA chunk of 32 features would be mostly empty).  Bound by the matrix
+// cores and the weight reads; N = 200, C = 128, H = 4, D = 32: fp32 130 -> 60 us, bf16 193 -> 29 us
+// against VALU block products; N = 320, C = 256, H = 8 in bf16 3815 -> 210 us.  64 tokens per block
+// (each weight row read half as often) measured slower up to C = 128 (68 and 36 us) and 9 % faster
+// at C = 256.
+// ---------------------------------------------------------------------------------------------
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restrict__ x, int64_t sx0, int64_t sx1,
                                                               const T* __restrict__ w_ln, const T* __restrict__ b_ln,
                                                               int apply_ln, const T* __restrict__ wqkv,
@@ -75,44 +122,86 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
                                                               T* __restrict__ xln, T* __restrict__ qo,
                                                               T* __restrict__ ko, T* __restrict__ vo,
                                                               float* __restrict__ bias, int64_t N, int C, int H, int D,
-                                                              float eps) {
-  extern __shared__ float xs[];  // [kGenTok][C]
-  const int tid = threadIdx.x;
-  const int64_t ntok = N * N, tok0 = (int64_t)blockIdx.x * kGenTok;
-  for (int e = tid; e < kGenTok * C; e += 256) {
-    const int t = e / C, c = e % C;
-    const int64_t tok = tok0 + t;
-    float v = 0.f;
-    if (tok < ntok) v = (float)x[(tok / N) * sx0 + (tok % N) * sx1 + c];
-    xs[e] = v;
-  }
-  __syncthreads();
-  if (apply_ln) gen_layer_norm<T>(xs, C, C, w_ln, b_ln, eps);
-  __syncthreads();
-  const int HD = H * D, F = 3 * HD + H;
-  for (int e = tid; e < kGenTok * F; e += 256) {
-    const int t = e / F, f = e % F;
-    const int64_t tok = tok0 + t;
-    if (tok >= ntok) continue;
-    const float* r = xs + t * C;
-    if (f < 3 * HD) {  // head h, which (0 = Q, 1 = K, 2 = V), d
-      const int h = f / (3 * D), which = (f / D) % 3, d = f % D;
-      const T* w = wqkv + (int64_t)f * C;  // (H, 3, D, C): row f
-      float acc = 0.f;
-      for (int c = 0; c < C; ++c) acc = fmaf((float)(T)r[c], (float)w[c], acc);
-      T* dst = which == 0 ? qo : which == 1 ? ko : vo;
-      dst[tok * HD + h * D + d] = (T)acc;
-    } else {
-      const int h = f - 3 * HD;
-      const T* w = WZ + (int64_t)h * C;
-      float acc = 0.f;
-      for (int c = 0; c < C; ++c) acc = fmaf(r[c], (float)w[c], acc);
-      bias[(int64_t)h * ntok + tok] = acc + (BZ ? BZ[h] : 0.f);
+                                                              int pw, float eps) {
+  using M = TileMma<T>;
+  using V = typename M::V;
+  constexpr int TT = 32, TPT = 256 / TT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int rx = tile_row<T>(C);
+  T* xs = reinterpret_cast<T*>(smem);  // [TT][rx]  x, then LN(x)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31, HD = H * D, F = 3 * HD;
+  const int64_t ntok = N * N, tok0 = (int64_t)blockIdx.x * TT;
+  {
+    const int t = tid / TPT, part = tid % TPT;
+    const bool ok = tok0 + t < ntok;
+    const int64_t tok = ok ? tok0 + t : ntok - 1, i = tok / N;
+    T* row = xs + t * rx;
+    stage_row<T, TPT, VEC>(row, x + i * sx0 + (tok - i * N) * sx1, ok, part, C, tile_kp(C));
+    float mean = 0.f, rstd = 1.f;
+    if (apply_ln) row_stats<T, TPT>(row, part, C, eps, mean, rstd);
+    // pair bias, 4 heads at a time
+    for (int h0 = 0; h0 < H; h0 += 4) {
+      float acc[4] = {};
+      for (int k = part * M::VE; k < C; k += TPT * M::VE) {
+        const V v = *reinterpret_cast<const V*>(row + k);
+        V wz[4], w = {}, b = {};
+        if constexpr (VEC) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) wz[j] = ldg<V>(WZ + (int64_t)(h0 + j < H ? h0 + j : H - 1) * C + k);
+          if (apply_ln) {
+            w = ldg<V>(w_ln + k);
+            if (b_ln) b = ldg<V>(b_ln + k);
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < M::VE; ++e) {
+            const bool in = k + e < C;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) wz[j][e] = in ? WZ[(int64_t)(h0 + j < H ? h0 + j : H - 1) * C + k + e] : (T)0.f;
+            if (apply_ln) {
+              w[e] = in ? w_ln[k + e] : (T)0.f;
+              b[e] = in && b_ln ? b_ln[k + e] : (T)0.f;
+            }
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < M::VE; ++e) {
+          float n = (float)v[e];
+          if (apply_ln) n = (n - mean) * rstd * (float)w[e] + (float)b[e];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[j] = fmaf(n, (float)wz[j][e], acc[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float s = token_sum<TPT>(acc[j]);
+        if (part == j && ok && h0 + j < H) bias[(int64_t)(h0 + j) * ntok + tok] = s + (BZ ? BZ[h0 + j] : 0.f);
+      }
+    }
+    if (apply_ln) normalise_row<T, TPT>(row, part, C, mean, rstd, w_ln, b_ln);
+    if (ok) {
+      T* dst = xln + tok * C;
+      for (int k = part * M::VE; k < C; k += TPT * M::VE) {
+        const V v = *reinterpret_cast<const V*>(row + k);
+        if constexpr (VEC) {
+          *reinterpret_cast<V*>(dst + k) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < M::VE; ++e)
+            if (k + e < C) dst[k + e] = v[e];
+        }
+      }
     }
   }
-  for (int e = tid; e < kGenTok * C; e += 256) {
-    const int64_t tok = tok0 + e / C;
-    if (tok < ntok) xln[tok * C + e % C] = (T)xs[e];
+  __syncthreads();
+  for (int f0 = 32 * wave; f0 < F; f0 += 128) {
+    const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
+    f32x16 acc[1] = {};
+    tile_gemm<T, 1, true, VEC>(acc, xs, rx, col, wqkv + (int64_t)(row < F ? row : F - 1) * C, C);
+    if (tok0 + col < ntok)
+      store_qkv16<T>(qo, ko, vo, (tok0 + col) * HD, fl, F - fl, D, pw,
+                     [&](int v) __attribute__((always_inline)) { return acc[0][v]; });
   }
 }
 
@@ -343,82 +432,6 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
 // ---------------------------------------------------------------------------------------------
 constexpr int kGT = 64, kGRow = kGT + 4;  // tokens per tile, LDS row of the k-major tiles
 
-// out[t][f] = sum_k a[k][t] * W[f][k] (a: k-major LDS tile of kGT tokens, K valid rows of CK;
-// W: F x K row-major in global memory), handed to epi(t, f, value) for t < ntok, f < F.  With
-// ROUND the activations are rounded to T as the products' operand.  The (64-feature chunk,
-// 32-deep k-tile) steps run as one sequence; each step's weights go k-major into LDS (ws: NBUF x
-// kTK x kGRow floats) from registers loaded during the previous step, so the loads' latency
-// overlaps the products.  One block barrier per step with two buffers, two with one (which
-// leaves more LDS for the caller's tiles and more blocks per CU).
-template <typename T, bool ROUND, int NBUF = 2, typename Epi>
-__device__ __attribute__((always_inline)) inline void tiled_gemm64(const float* a, int K, int CK,
-                                                                   const T* __restrict__ W, int F, float* ws,
-                                                                   int ntok, Epi epi) {
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  const int nk = CK / kTK, nsteps = ((F + 63) / 64) * nk;
-  // staging: thread tid moves weights (f, k) = (e / kTK, e % kTK), e = tid + 256 i, i < 8
-  float wr[8];
-  auto wload = [&](int step) __attribute__((always_inline)) {
-    const int f0 = (step / nk) * 64, k0 = (step % nk) * kTK;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + 256 * i, ff = f0 + e / kTK, kk = k0 + e % kTK;
-      wr[i] = ff < F && kk < K ? (float)W[(int64_t)ff * K + kk] : 0.f;
-    }
-  };
-  auto wstore = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + 256 * i;
-      ws[(buf * kTK + e % kTK) * kGRow + e / kTK] = wr[i];
-    }
-  };
-  __syncthreads();  // the caller's tile is complete; ws is free
-  wload(0);
-  wstore(0);
-  float acc[4][4] = {};
-  for (int step = 0; step < nsteps; ++step) {
-    if constexpr (NBUF == 1) {
-      if (step > 0) {
-        __syncthreads();  // every thread is done with the previous step's weights
-        wstore(0);
-      }
-    }
-    __syncthreads();  // this step's buffer is filled (two buffers: the other one is no longer read)
-    if (step + 1 < nsteps) wload(step + 1);
-    const int k0 = (step % nk) * kTK;
-    const float* wb = ws + (NBUF == 1 ? 0 : (step & 1)) * kTK * kGRow;
-#pragma unroll 8
-    for (int k = 0; k < kTK; ++k) {
-      f32x4 x = *reinterpret_cast<const f32x4*>(&a[(k0 + k) * kGRow + 4 * ty]);
-      if constexpr (ROUND) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) x[u] = (float)(T)x[u];
-      }
-      const f32x4 w = *reinterpret_cast<const f32x4*>(&wb[k * kGRow + 4 * tx]);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = fmaf(x[u], w[v], acc[u][v]);
-    }
-    if constexpr (NBUF == 2) {
-      if (step + 1 < nsteps) wstore((step + 1) & 1);
-    }
-    if (step % nk == nk - 1) {  // the chunk's last k-tile: epilogue, fresh accumulators
-      const int f0 = (step / nk) * 64;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int t = 4 * ty + u, f = f0 + 4 * tx + v;
-          if (t < ntok && f < F) epi(t, f, acc[u][v]);
-          acc[u][v] = 0.f;
-        }
-    }
-  }
-  __syncthreads();  // ws and the caller's tile may be reused after return
-}
-
 // LayerNorm (optionally with the affine w, b) of the kGT token columns of a k-major tile, in place
 // (fp32, two-pass, 4 threads per token); rows [C, CK) are set to zero.
 template <typename T>
@@ -476,68 +489,27 @@ __device__ __attribute__((always_inline)) inline void tiled_load_rows(float* dst
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void tri_gen_prep_tiled_kernel(const T* __restrict__ x, int64_t sx0, int64_t sx1,
-                                                                const T* __restrict__ w_ln, const T* __restrict__ b_ln,
-                                                                int apply_ln, const T* __restrict__ wqkv,
-                                                                const T* __restrict__ WZ, const float* __restrict__ BZ,
-                                                                T* __restrict__ xln, T* __restrict__ qo,
-                                                                T* __restrict__ ko, T* __restrict__ vo,
-                                                                float* __restrict__ bias, int64_t N, int C, int H, int D,
-                                                                float eps) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CK = (C + kTK - 1) / kTK * kTK;
-  float* xs = sm;                  // [CK][kGRow]  (LN(x)), k-major
-  float* ws = xs + CK * kGRow;     // [2][kTK][kGRow] staged weights
-  const int tid = threadIdx.x;
-  const int64_t ntokall = N * N, tok0 = (int64_t)blockIdx.x * kGT;
-  const int ntok = (int)(ntokall - tok0 < kGT ? ntokall - tok0 : kGT);
-  tiled_load_rows<T>(xs, x, C, CK, ntok, [=](int t) {
-    const int64_t tok = tok0 + t;
-    return (tok / N) * sx0 + (tok % N) * sx1;
-  });
-  __syncthreads();
-  if (apply_ln) tiled_ln_affine<T>(xs, C, CK, w_ln, b_ln, eps);
-  __syncthreads();
-  for (int e = tid; e < kGT * C; e += 256) {
-    const int t = e / C, c = e % C;
-    if (t < ntok) xln[(tok0 + t) * C + c] = (T)xs[c * kGRow + t];
-  }
-  const int HD = H * D;
-  // Q / K / V of all heads from LN(x) rounded to the I/O type; weight row f = (h, which, d).  The
-  // destination is picked by integer selects on address offsets (a pointer choice among the three
-  // becomes a table in private memory)
-  const uint64_t aq = (uint64_t)qo, dk = (uint64_t)ko - aq, dv = (uint64_t)vo - aq;
-  tiled_gemm64<T, true>(xs, C, CK, wqkv, 3 * HD, ws, ntok, [=](int t, int f, float v) {
-    const int h = f / (3 * D), which = (f / D) % 3, d = f % D;
-    const uint64_t base = aq + (which == 1 ? dk : 0) + (which == 2 ? dv : 0);
-    reinterpret_cast<T*>(base)[(tok0 + t) * HD + h * D + d] = (T)v;
-  });
-  // the row-shared pair bias from the unrounded LN(x), fp32
-  tiled_gemm64<T, false>(xs, C, CK, WZ, H, ws, ntok,
-                         [=](int t, int h, float v) { bias[(int64_t)h * ntokall + tok0 + t] = v + (BZ ? BZ[h] : 0.f); });
-}
-
-template <typename T>
 static int tri_generic_prep_t(const void* x, int64_t sx0, int64_t sx1, const void* w_ln, const void* b_ln,
                               int apply_ln, const void* wqkv, const void* WZ, const float* BZ, void* xln, void* q,
                               void* k, void* v, float* bias, int64_t N, int C, int H, int D, float eps,
                               hipStream_t st) {
-  const int64_t tiles = (N * N + kGT - 1) / kGT;
-  if (C <= 256 && tiles >= num_cus()) {  // tiled kernel: 64 tokens per block
-    const int CK = (C + kTK - 1) / kTK * kTK;
-    const size_t lds = (size_t)(CK + 2 * kTK) * kGRow * sizeof(float);
-    hipFuncSetAttribute((const void*)tri_gen_prep_tiled_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                        (int)lds);
-    hipLaunchKernelGGL((tri_gen_prep_tiled_kernel<T>), dim3((unsigned)tiles), dim3(256), lds, st, (const T*)x, sx0, sx1,
-                       (const T*)w_ln, (const T*)b_ln, apply_ln, (const T*)wqkv, (const T*)WZ, BZ, (T*)xln, (T*)q,
-                       (T*)k, (T*)v, bias, N, C, H, D, eps);
-    return launched("tops_tri_generic_prep");
-  }
-  const int64_t blocks = (N * N + kGenTok - 1) / kGenTok;
-  if (blocks == 0) return TOPS_OK;
-  hipLaunchKernelGGL((tri_generic_prep_kernel<T>), dim3((unsigned)blocks), dim3(256), kGenTok * C * sizeof(float), st,
-                     (const T*)x, sx0, sx1, (const T*)w_ln, (const T*)b_ln, apply_ln, (const T*)wqkv, (const T*)WZ,
-                     BZ, (T*)xln, (T*)q, (T*)k, (T*)v, bias, N, C, H, D, eps);
+  if (N == 0) return TOPS_OK;
+  const bool vec = aligned16({x, w_ln, b_ln, wqkv, WZ, xln}) && multiples_of(TileMma<T>::VE, {sx0, sx1, C});
+  const int pw = qkv_piece<T>(D, q, k, v);
+  const size_t lds = (size_t)32 * tile_row<T>(C) * sizeof(T);
+#define TOPS_GEN_PREP(VEC)                                                                                          \
+  do {                                                                                                              \
+    (void)hipFuncSetAttribute((const void*)tri_generic_prep_kernel<T, VEC>,                                         \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                                \
+    hipLaunchKernelGGL((tri_generic_prep_kernel<T, VEC>), dim3((unsigned)((N * N + 31) / 32)), dim3(256), lds, st,   \
+                       (const T*)x, sx0, sx1, (const T*)w_ln, (const T*)b_ln, apply_ln, (const T*)wqkv, (const T*)WZ, \
+                       BZ, (T*)xln, (T*)q, (T*)k, (T*)v, bias, N, C, H, D, pw, eps);                                 \
+  } while (0)
+  if (vec)
+    TOPS_GEN_PREP(true);
+  else
+    TOPS_GEN_PREP(false);
+#undef TOPS_GEN_PREP
   return launched("tops_tri_generic_prep");
 }
 
@@ -606,22 +578,37 @@ static int gate_generic_t(const void* o, int64_t so0, int64_t so1, const void* g
 //   apb_generic_bias_kernel  per pair (q, k): bias[h][q][k] = zn . Wc[h] + Bc[h], zn = (z - mean) * rstd
 //                            of z = Z[q, k, :] (the LN affine is folded into Wc / Bc)
 // ---------------------------------------------------------------------------------------------
-template <typename T>
+// 32 tokens and 128 weight rows per block, one 32-row chunk per wave; X rows go through LDS kQkvC
+// channels at a time.  Few tokens: bound by latency (600 tokens, C = 384, 16 heads of 24 in bf16: 1031
+// -> 8 us against a thread per output).
+constexpr int kQkvC = 512;
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void apb_generic_qkv_kernel(const T* __restrict__ X, const T* __restrict__ wqkv,
                                                              T* __restrict__ qo, T* __restrict__ ko,
-                                                             T* __restrict__ vo, int64_t M, int C, int H, int D) {
-  const int HD = H * D;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= M * 3 * HD) return;
-  const int64_t m = idx / (3 * HD);
-  const int f = (int)(idx % (3 * HD));  // row of the (H, 3, D, C) weight
-  const int h = f / (3 * D), which = (f / D) % 3, d = f % D;
-  const T* xr = X + m * C;
-  const T* w = wqkv + (int64_t)f * C;
-  float acc = 0.f;
-  for (int c = 0; c < C; ++c) acc = fmaf((float)xr[c], (float)w[c], acc);
-  T* dst = which == 0 ? qo : which == 1 ? ko : vo;
-  dst[m * HD + h * D + d] = (T)acc;
+                                                             T* __restrict__ vo, int64_t M, int C, int H, int D,
+                                                             int pw) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  T* xs = reinterpret_cast<T*>(smem);  // [32][tile_row(min(C, kQkvC))]
+  const int rx = tile_row<T>(C < kQkvC ? C : kQkvC), HD = H * D, F = 3 * HD;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const int64_t tok0 = (int64_t)blockIdx.x * 32;
+  const int f0 = 128 * blockIdx.y + 32 * wave, row = f0 + tile_perm(col), fl = f0 + 16 * hl;
+  const T* w = wqkv + (int64_t)(row < F ? row : F - 1) * C;
+  const int t = tid >> 3, part = tid & 7;
+  const bool ok = tok0 + t < M;
+  const T* src = X + (ok ? tok0 + t : M - 1) * C;
+  f32x16 acc[1] = {};
+  for (int c0 = 0; c0 < C; c0 += kQkvC) {
+    const int kc = C - c0 < kQkvC ? C - c0 : kQkvC;
+    if (c0 > 0) __syncthreads();
+    stage_row<T, 8, VEC>(xs + t * rx, src + c0, ok, part, kc, tile_kp(kc));
+    __syncthreads();
+    if (f0 < F) tile_gemm<T, 1, true, VEC, 8>(acc, xs, rx, col, w + c0, kc);
+  }
+  if (tok0 + col < M && f0 < F)
+    store_qkv16<T>(qo, ko, vo, (tok0 + col) * HD, fl, F - fl, D, pw,
+                   [&](int v) __attribute__((always_inline)) { return acc[0][v]; });
 }
 
 template <typename T>
@@ -651,32 +638,8 @@ __global__ __launch_bounds__(256) void apb_generic_bias_kernel(const T* __restri
   }
 }
 
-// Tiled apb pre-pass kernels (C_s, C_z <= 256): Q / K / V as a block GEMM over 64 tokens and 64
-// weight rows; the pair bias as a LayerNorm of 64 pairs in LDS, then per head (one wave each) the
-// dot products of its 64 pairs (lanes) with the head's weights (wave-uniform: scalar loads).
-template <typename T>
-__global__ __launch_bounds__(256) void apb_gen_qkv_tiled_kernel(const T* __restrict__ X, const T* __restrict__ wqkv,
-                                                               T* __restrict__ qo, T* __restrict__ ko,
-                                                               T* __restrict__ vo, int64_t M, int C, int H, int D) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CK = (C + kTK - 1) / kTK * kTK;
-  float* xs = sm;               // [CK][kGRow]  X, k-major
-  float* ws = xs + CK * kGRow;  // [2][kTK][kGRow]
-  const int tid = threadIdx.x;
-  const int64_t tok0 = (int64_t)blockIdx.x * kGT;
-  const int ntok = (int)(M - tok0 < kGT ? M - tok0 : kGT);
-  tiled_load_rows<T>(xs, X, C, CK, ntok, [=](int t) { return (tok0 + t) * (int64_t)C; });
-  const int HD = H * D;
-  const uint64_t aq = (uint64_t)qo, dk = (uint64_t)ko - aq, dv = (uint64_t)vo - aq;
-  // this block's 64 weight rows (blockIdx.y): more blocks than tokens / 64 alone would give
-  const int fb = 64 * (int)blockIdx.y, nf = 3 * HD - fb < 64 ? 3 * HD - fb : 64;
-  tiled_gemm64<T, false>(xs, C, CK, wqkv + (int64_t)fb * C, nf, ws, ntok, [=](int t, int fl, float v) {
-    const int f = fb + fl, h = f / (3 * D), which = (f / D) % 3, d = f % D;
-    const uint64_t base = aq + (which == 1 ? dk : 0) + (which == 2 ? dv : 0);
-    reinterpret_cast<T*>(base)[(tok0 + t) * HD + h * D + d] = (T)v;
-  });
-}
-
+// Tiled form for C_z <= 256: a LayerNorm of 64 pairs in LDS, then per head (one wave each) the dot
+// products of its 64 pairs (lanes) with the head's weights (wave-uniform: scalar loads).
 template <typename T>
 __global__ __launch_bounds__(256) void apb_gen_bias_tiled_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
                                                                 const float* __restrict__ Wc,
@@ -713,18 +676,24 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
                               const float* Wc, const float* Bc, void* q, void* k, void* v, float* bias, int64_t M,
                               int C, int Cz, int H, int D, float eps, hipStream_t st) {
   // the tiled bias kernel takes 64 pairs per block: used where that still gives every CU a block
-  const int64_t t1 = (M + kGT - 1) / kGT, t2 = (M * M + kGT - 1) / kGT;
-  if (t1 == 0) return TOPS_OK;
-  if (C <= 256) {
-    const int CK = (C + kTK - 1) / kTK * kTK;
-    const size_t l1 = (size_t)(CK + 2 * kTK) * kGRow * sizeof(float);
-    hipFuncSetAttribute((const void*)apb_gen_qkv_tiled_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l1);
-    hipLaunchKernelGGL((apb_gen_qkv_tiled_kernel<T>), dim3((unsigned)t1, (unsigned)((3 * H * D + 63) / 64)), dim3(256),
-                       l1, st, (const T*)X, (const T*)wqkv, (T*)q, (T*)k, (T*)v, M, C, H, D);
-  } else {
-    const int64_t b1 = (M * 3 * H * D + 255) / 256;
-    hipLaunchKernelGGL((apb_generic_qkv_kernel<T>), dim3((unsigned)b1), dim3(256), 0, st, (const T*)X,
-                       (const T*)wqkv, (T*)q, (T*)k, (T*)v, M, C, H, D);
+  const int64_t t2 = (M * M + kGT - 1) / kGT;
+  if (M == 0) return TOPS_OK;
+  const int pw = qkv_piece<T>(D, q, k, v);
+  {
+    const bool vec = aligned16({X, wqkv}) && C % TileMma<T>::VE == 0;
+    const size_t lds = (size_t)32 * tile_row<T>(C < kQkvC ? C : kQkvC) * sizeof(T);
+    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)((3 * H * D + 127) / 128));
+    if (vec) {
+      (void)hipFuncSetAttribute((const void*)apb_generic_qkv_kernel<T, true>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL((apb_generic_qkv_kernel<T, true>), grid, dim3(256), lds, st, (const T*)X, (const T*)wqkv,
+                         (T*)q, (T*)k, (T*)v, M, C, H, D, pw);
+    } else {
+      (void)hipFuncSetAttribute((const void*)apb_generic_qkv_kernel<T, false>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL((apb_generic_qkv_kernel<T, false>), grid, dim3(256), lds, st, (const T*)X, (const T*)wqkv,
+                         (T*)q, (T*)k, (T*)v, M, C, H, D, pw);
+    }
   }
   if (Cz <= 256 && t2 >= num_cus()) {
     const int CzK = (Cz + kTK - 1) / kTK * kTK;
