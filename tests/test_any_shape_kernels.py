@@ -118,3 +118,47 @@ def test_apb_qkv_any_shape(device, dtype, M, C, H, D):
         wi = w[:, i].double().reshape(H * D, C)
         ref = x.double() @ wi.T
         _within(out[i], ref, EPS[dtype] * (ref.abs() + x.double().abs() @ wi.abs().T + 1e-3), name)
+
+
+# key chunks of 32: one key, one chunk less one, one, one more, several; 128-query blocks; D at and below
+# 32 and 64, with and without 16-byte rows; few blocks (keys split over the waves) and many
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("N,H,D", [(1, 2, 32), (31, 3, 24), (32, 2, 64), (33, 1, 10), (129, 4, 32), (70, 9, 40),
+                                   (100, 8, 64), (160, 4, 6)])
+@pytest.mark.parametrize("mask", ["none", "random", "rows", "inf"])
+def test_attention_any_shape(device, dtype, N, H, D, mask):
+    """Triangle attention (a random pair mask; whole rows masked) and attention over one row (mask
+    "inf": masked keys -inf, some chunks wholly masked)."""
+    from triangleops_amd import _native
+    from triangleops_amd._common.dtype import any_shape_dtype_code
+    from triangleops_amd.triangle_attn.kernel import generic_attention
+
+    g = torch.Generator().manual_seed(N + D)
+    R = 1 if mask == "inf" else N
+    q, k, v = (_rnd(g, dtype, R, N, H, D) for _ in range(3))
+    bias = _rnd(g, torch.float32, H, N, N)
+    scale = D**-0.5
+    m = None
+    if mask != "none":
+        m = torch.rand(R, N, generator=g) < 0.8
+        m[:, : min(40, N // 2)] = False
+        m[:, N - 1] = True
+        if mask == "rows":
+            m[::3] = False
+    dev = [t.to(device) for t in (q, k, v, bias)]
+    md = None if m is None else m.to(device)
+    out = torch.empty(R, N, H * D, device=device, dtype=dtype)
+    if mask == "inf":
+        _native.call("tops_apb_generic_attention", *(t.data_ptr() for t in dev), md.view(torch.int8).data_ptr(),
+                     out.data_ptr(), N, H, D, scale, any_shape_dtype_code(dtype), _native.stream_of(out))
+    else:
+        generic_attention(*dev, out, scale=scale, mask=md)
+    s = torch.einsum("iqhd,ikhd->ihqk", q.double(), k.double()) * scale + bias.double()
+    if m is not None:
+        s = s.masked_fill(~m[:, None, None, :], float("-inf")) if mask == "inf" else \
+            (s + torch.where(m, 0.0, -1e9)[:, None, None, :]).float().double()  # the fp32 add rounds to 64s
+    p = torch.softmax(s, -1)
+    ref = torch.einsum("ihqk,ikhd->iqhd", p, v.double()).reshape(R, N, H * D)
+    size = torch.einsum("ihqk,ikhd->iqhd", p, v.double().abs()).reshape(R, N, H * D)
+    # fp32 scores of a few units are off by some 2^-22, the weights relatively so; one rounding of the result
+    _within(out, ref, 0.5 * EPS[dtype] * ref.abs() + EPS[torch.float32] * size + 1e-7, f"{dtype} {N} {H} {D} {mask}")

@@ -206,147 +206,192 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 }
 
 // ---------------------------------------------------------------------------------------------
-// Attention over R rows of N queries and N keys, any H, D <= DM.  A block takes 64 queries of
-// one (row i, head h), lane = query; its 4 waves split the keys into 32-key chunks (chunk c to
-// wave c % 4).  Per chunk a wave stages the chunk's K and V in LDS (fp32; every lane then reads
-// the same element, a broadcast), computes the 32 scores of its queries (q . k * scale + bias;
-// masked keys (mask[i*sm0 + k*sm1] == 0) get "+ (-1e9)" in fp32 (triangle attention) or -inf
-// (MASK_INF, attention_pair_bias: a row without valid keys gives NaN, as torch's softmax does);
-// keys >= N are left out), rescales its running (o, l) once to the chunk's maximum and adds
-// exp(s - m) and exp(s - m) v.  The 4 waves' (m, l, o) are merged through LDS at the end.
+// Attention over R rows of N queries and N keys, any H, D <= DP (16, 32 or 64).  A wave holds 32 queries of one
+// (row i, head h) and walks the keys in chunks of 32: S^T = K . Q^T (a lane: one query, the 16 keys
+// k0 + 16 hl + v), scores q . k * scale + bias with masked keys (mask[i*sm0 + k*sm1] == 0) getting
+// "+ (-1e9)" in fp32 (triangle attention) or -inf (MASK_INF, attention_pair_bias: a row without valid
+// keys gives NaN, as torch's softmax does) and keys >= N left out, online softmax in fp32, and
+// O^T += V^T . P^T with the score registers as the operand.  fp32 I/O runs the fp32 MFMA throughout;
+// with 16-bit I/O the fp32 weights enter as two 16-bit terms (hi + lo, two MFMAs: 16 bits of each
+// weight or more, as fp16 weights are scaled by 2^10 to stay clear of its denormals).
+// K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
+// per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block's
+// 4 waves take 4 query tiles and share the key reads through L1; with KSPL = 4 they take every 4th chunk
+// of one query tile and merge (m, l, o) through LDS.  Bound by the fp32 MFMAs in fp32 (N = 200, 4 heads
+// of 32: 247 -> 75 us against a query per lane on the VALU, half of the fp32 matrix rate), by the
+// exponentials and the split of the weights in 16 bits (the same in bf16: 245 -> 44 us).
 // ---------------------------------------------------------------------------------------------
-constexpr int kGenKC = 32, kGenAW = 4;  // keys per chunk, waves (key splits) per block
-
-template <typename T, int DM, bool MASK_INF>
-__global__ __launch_bounds__(256, 2) void tri_generic_attn_kernel(const T* __restrict__ qi_, const T* __restrict__ ki_,
-                                                              const T* __restrict__ vi_, const float* __restrict__ bias,
-                                                              const int8_t* __restrict__ mask, int64_t sm0, int64_t sm1,
-                                                              T* __restrict__ out, int64_t so0, int64_t so1, int64_t R,
-                                                              int64_t N, int H, int D, float scale) {
-  __shared__ __attribute__((aligned(16))) float kvs[kGenAW][2][kGenKC][DM];  // per wave: K, V of its chunk
-  __shared__ float madd[kGenAW][kGenKC];                                     // per key: 0, -1e9, -inf
-  __shared__ float mls[kGenAW][64][2];                                       // per wave and query: m, l
-  const int64_t nqb = (N + 63) / 64, qb = blockIdx.x % nqb, ih = blockIdx.x / nqb;
-  const int h = (int)(ih % H);
-  const int64_t i = ih / H;
-  (void)R;
+template <typename T, int DP, int KSPL, bool MASK_INF, bool VEC>
+__global__ __launch_bounds__(256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel(
+    const T* __restrict__ qi_, const T* __restrict__ ki_, const T* __restrict__ vi_, const float* __restrict__ bias,
+    const int8_t* __restrict__ mask, int64_t sm0, int64_t sm1, T* __restrict__ out, int64_t so0, int64_t so1, int N,
+    int H, int D, float scale) {
+  using M = TileMma<T>;
+  using V = typename M::V;
+  constexpr int ND = (DP + 31) / 32;               // 32-channel tiles of O
+  constexpr int NQ = DP / M::KS, NV = 16 / M::VE;  // k-steps of q . k, 16-byte pieces of 16 keys
+  constexpr int QB = 128 / KSPL;                          // queries per block
+  constexpr float kShift = std::is_same<T, _Float16>::value ? 10.f : 0.f;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t q = qb * 64 + lane, qq = q < N ? q : N - 1;
-  const int HD = H * D;
-  float qv[DM], o[DM];
-  const T* qp = qi_ + (i * N + qq) * HD + h * D;
+  const int hl = lane >> 5, col = lane & 31;
+  const uint32_t nqb = (N + QB - 1) / QB, ih = blockIdx.x / nqb, qb = blockIdx.x - ih * nqb;
+  const int i = ih / (uint32_t)H, h = ih - i * H;
+  const int q0 = qb * QB + (KSPL == 1 ? 32 * wave : 0);
+  if (KSPL == 1 && q0 >= N) return;
+  // all reads go through buffers of the row's keys and of the tile's bias rows: a lane keeps 32-bit byte
+  // offsets (64-bit addresses of every element would take the registers of two more waves per SIMD),
+  // and keys past N read 0.  kOut is past any buffer's end.
+  constexpr uint32_t ES = sizeof(T), kOut = 0x80000000u;
+  const uint32_t HDB = H * D * ES;
+  const int64_t base = (int64_t)i * N * H * D + h * D;
+  const int q = q0 + col < N ? q0 + col : N - 1;
+  const uint32_t rbytes = (uint32_t)N * HDB - (uint32_t)h * D * ES;
+  const Rsrc qr = buffer_of(qi_ + base, rbytes), kr = buffer_of(ki_ + base, rbytes), vr = buffer_of(vi_ + base, rbytes);
+  const int qrows = N - q0 < 32 ? N - q0 : 32;
+  const Rsrc br = buffer_of(bias + ((int64_t)h * N + q0) * N, (uint32_t)qrows * N * 4);
+  const int8_t* mrow = mask ? mask + i * sm0 : nullptr;
+  auto load_row = [&](V(&r)[NQ], Rsrc src, uint32_t row) __attribute__((always_inline)) {  // zero past D
 #pragma unroll
-  for (int d = 0; d < DM; ++d) {
-    qv[d] = d < D ? (float)qp[d] * scale : 0.f;
-    o[d] = 0.f;
+    for (int s = 0; s < NQ; ++s) {
+      const int d = s * M::KS + hl * M::VE;
+      if constexpr (VEC) {
+        r[s] = buffer_load<V>(src, row + (d < D ? d * ES : kOut));
+      } else {
+#pragma unroll
+        for (int e = 0; e < M::VE; ++e) r[s][e] = buffer_load<T>(src, row + (d + e < D ? (d + e) * ES : kOut));
+      }
+    }
+  };
+  V qf[NQ], kf[NQ];
+  load_row(qf, qr, (uint32_t)q * HDB);
+  uint32_t vd[ND];  // this lane's V element of a key: channel tile_perm(col) of each 32, so o holds 16 hl + v
+#pragma unroll
+  for (int n = 0; n < ND; ++n) {
+    const int d = 32 * n + tile_perm(col);
+    vd[n] = 16 * hl * HDB + (d < D ? d : D - 1) * ES;  // channels past D are computed and not stored
   }
-  const float* brow = bias + ((int64_t)h * N + qq) * N;
+  const uint32_t bd = (uint32_t)(q - q0) * N * 4 + 64 * hl, kd = tile_perm(col) * HDB;
+  f32x16 o[ND] = {};
   float m = -INFINITY, l = 0.f;
-  const int64_t nch = (N + kGenKC - 1) / kGenKC;
-  for (int64_t c = wave; c < nch; c += kGenAW) {
-    const int64_t k0 = c * kGenKC;
-    for (int e = lane; e < kGenKC * DM; e += 64) {
-      const int kk = e / DM, d = e % DM;
-      const int64_t key = k0 + kk;
-      const bool ok = key < N && d < D;
-      const int64_t off = (i * N + key) * HD + h * D + d;
-      kvs[wave][0][kk][d] = ok ? (float)ki_[off] : 0.f;
-      kvs[wave][1][kk][d] = ok ? (float)vi_[off] : 0.f;
-    }
-    if (lane < kGenKC) {
-      const int64_t key = k0 + lane;
-      madd[wave][lane] = key >= N ? -INFINITY
-                         : (mask && mask[i * sm0 + key * sm1] == 0) ? (MASK_INF ? -INFINITY : -1e9f)
-                                                                     : 0.f;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // 8-key sub-chunks, each with its own maximum and one rescale of (o, l)
-#pragma unroll 1
-    for (int k8 = 0; k8 < kGenKC; k8 += 8) {
-      float sc[8] = {};
-      // q . k for the 8 keys, 4 channels per step; at most 32 K values live (the pins end a step's
-      // products, the empty asm with a memory clobber keeps the next step's LDS reads after them)
+  const int nch = (N + 31) / 32;
+  int c = KSPL == 1 ? 0 : wave;
+  if (c < nch) load_row(kf, kr, kd + 32 * c * HDB);
+  for (; c < nch; c += KSPL) {
+    const int k0 = 32 * c;
+    // this chunk's V, bias and mask, used after the scores
+    V vf[ND][NV];
+    f32x16 b;
 #pragma unroll
-      for (int d0 = 0; d0 < DM; d0 += 4) {
+    for (int v = 0; v < 16; ++v)
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          const f32x4 kq = *reinterpret_cast<const f32x4*>(&kvs[wave][0][k8 + kk][d0]);
+      for (int n = 0; n < ND; ++n) vf[n][v / M::VE][v % M::VE] = buffer_load<T>(vr, vd[n] + (k0 + v) * HDB);
+    if (k0 + 32 <= N) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sc[kk] = fmaf(qv[d0 + e], kq[e], sc[kk]);
-        }
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 t = buffer_load<f32x4>(br, bd + k0 * 4 + 16 * g);
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) pin(sc[kk]);  // this step's products are done here
-        asm volatile("" ::: "memory");                 // and the next step's reads follow
+        for (int e = 0; e < 4; ++e) b[4 * g + e] = t[e];
       }
-      float cm = -INFINITY;
+    } else {  // (past the end of a row: the next row or 0, replaced by -inf below)
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const float a = sc[kk];
-        const float ma = madd[wave][k8 + kk];
-        const int64_t key = k0 + k8 + kk;
-        const float sk = a + (key < N ? brow[key] : 0.f);
-        sc[kk] = ma == 0.f ? sk : (ma == -INFINITY ? -INFINITY : sk + ma);
-        cm = fmaxf(cm, sc[kk]);
+      for (int v = 0; v < 16; ++v) b[v] = buffer_load<float>(br, bd + k0 * 4 + 4 * v);
+    }
+    const bool in = k0 + col < N;
+    const bool on = in && (!mrow || mrow[(int64_t)(k0 + col) * sm1] != 0);
+    const uint32_t inb = (uint32_t)__builtin_amdgcn_ballot_w64(in), onb = (uint32_t)__builtin_amdgcn_ballot_w64(on);
+    f32x16 s = {};
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
+    if (c + KSPL < nch) load_row(kf, kr, kd + 32 * (c + KSPL) * HDB);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], scale, b[v]);
+    if (onb != 0xffffffffu) {  // some key is masked or past the end
+      const uint32_t ib = inb >> (16 * hl), ob = onb >> (16 * hl);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        s[v] = (ob >> v) & 1 ? s[v] : (MASK_INF ? -INFINITY : s[v] - 1e9f);
+        s[v] = (ib >> v) & 1 ? s[v] : -INFINITY;
       }
-      const float mn = fmaxf(m, cm);
-      // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
-      // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
-      const float sh = mn == -INFINITY ? 0.f : mn;
-      const float corr = __expf(m - sh);
+    }
+    float cm = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) cm = fmaxf(cm, s[v]);
+    const float mn = fmaxf(m, halves_max(cm));
+    // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
+    // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
+    const float sh = mn == -INFINITY ? 0.f : mn;
+    if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {
+      const float corr = fast_exp2((m - sh) * kLog2e);
       l *= corr;
 #pragma unroll
-      for (int d = 0; d < DM; ++d) o[d] *= corr;
+      for (int n = 0; n < ND; ++n)
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const float p = __expf(sc[kk] - sh);
-        l += p;
-#pragma unroll
-        for (int d = 0; d < DM; d += 4) {
-          const f32x4 vq = *reinterpret_cast<const f32x4*>(&kvs[wave][1][k8 + kk][d]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[d + e] = fmaf(p, vq[e], o[d + e]);
-        }
-#pragma unroll
-        for (int d = 0; d < DM; ++d) pin(o[d]);
-        asm volatile("" ::: "memory");
-      }
+        for (int v = 0; v < 16; ++v) o[n][v] *= corr;
       m = mn;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the chunk's K / V are read before the next chunk overwrites them
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    V p[NV], pl[NV];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float w = fast_exp2(fmaf(s[v] - sh, kLog2e, kShift));
+      l += w;
+      const T hi = (T)w;
+      p[v / M::VE][v % M::VE] = hi;
+      pl[v / M::VE][v % M::VE] = (T)(w - (float)hi);
+    }
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        o[n] = M::mma(vf[n][j], p[j], o[n]);
+        if constexpr (sizeof(T) == 2) o[n] = M::mma(vf[n][j], pl[j], o[n]);
+      }
   }
-  // ---- merge the 4 waves' partial states (o goes through the K / V staging area) ----
-  __syncthreads();
-  float* ob = &kvs[0][0][0][0];  // [kGenAW][64][DM]
+  l = halves_sum(l);
+  if constexpr (KSPL == 1) {
+    const float inv = 1.f / l;
+    if (q0 + col >= N) return;
+    T* dst = out + i * so0 + (int64_t)q * so1 + h * D;
 #pragma unroll
-  for (int d = 0; d < DM; ++d) ob[(wave * 64 + lane) * DM + d] = o[d];
-  mls[wave][lane][0] = m;
-  mls[wave][lane][1] = l;
-  __syncthreads();
-  float mw[kGenAW], mx = -INFINITY;
+    for (int n = 0; n < ND; ++n) {
+      const int d = 32 * n + 16 * hl;
+      store16<T, VEC>(dst + d, D - d, [&](int v) __attribute__((always_inline)) { return (T)(o[n][v] * inv); });
+    }
+  } else {
+    // ---- merge the waves' partial states ----
+    constexpr int OR = 32 * ND + 4;
+    __shared__ __attribute__((aligned(16))) float ob[KSPL][32][OR];
+    __shared__ float mls[KSPL][32][2];
 #pragma unroll
-  for (int w = 0; w < kGenAW; ++w) {
-    mw[w] = mls[w][lane][0];
-    mx = fmaxf(mx, mw[w]);
-  }
-  const float sh = mx == -INFINITY ? 0.f : mx;
-  float sw[kGenAW], lt = 0.f;
+    for (int n = 0; n < ND; ++n)
 #pragma unroll
-  for (int w = 0; w < kGenAW; ++w) {
-    sw[w] = __expf(mw[w] - sh);
-    lt += sw[w] * mls[w][lane][1];
-  }
-  const float inv = 1.f / lt;
-  if (q < N) {
-    T* dst = out + i * so0 + q * so1 + h * D;
-    for (int d = wave; d < D; d += kGenAW) {  // each wave writes every 4th element of the row
-      float acc = 0.f;
+      for (int v = 0; v < 16; ++v) ob[wave][col][32 * n + 16 * hl + v] = o[n][v];
+    mls[wave][col][0] = m;
+    mls[wave][col][1] = l;
+    __syncthreads();
+    const int t = threadIdx.x >> 3, d0 = (threadIdx.x & 7) * 4 * ND;  // 8 threads per query, 4 ND channels each
+    float mw[KSPL], mx = -INFINITY;
 #pragma unroll
-      for (int w = 0; w < kGenAW; ++w) acc += sw[w] * ob[(w * 64 + lane) * DM + d];
-      dst[d] = (T)(acc * inv);
+    for (int w = 0; w < KSPL; ++w) {
+      mw[w] = mls[w][t][0];
+      mx = fmaxf(mx, mw[w]);
+    }
+    const float sh = mx == -INFINITY ? 0.f : mx;
+    float sw[KSPL], lt = 0.f;
+#pragma unroll
+    for (int w = 0; w < KSPL; ++w) {
+      sw[w] = fast_exp2((mw[w] - sh) * kLog2e);
+      lt += sw[w] * mls[w][t][1];
+    }
+    const float inv = 1.f / lt;
+    if (q0 + t < N) {
+      T* dst = out + i * so0 + (q0 + t) * so1 + h * D;
+#pragma unroll
+      for (int d = 0; d < 4 * ND; ++d) {
+        float acc = 0.f;
+#pragma unroll
+        for (int w = 0; w < KSPL; ++w) acc += sw[w] * ob[w][t][d0 + d];
+        if (d0 + d < D) dst[d0 + d] = (T)(acc * inv);
+      }
     }
   }
 }
@@ -513,25 +558,46 @@ static int tri_generic_prep_t(const void* x, int64_t sx0, int64_t sx1, const voi
   return launched("tops_tri_generic_prep");
 }
 
-template <typename T>
-static int tri_generic_attention_t(const void* q, const void* k, const void* v, const float* bias, const void* mask,
-                                   int64_t sm0, int64_t sm1, void* out, int64_t so0, int64_t so1, int64_t N, int H,
-                                   int D, float scale, hipStream_t st) {
-  const int64_t blocks = N * H * ((N + 63) / 64);
-  if (blocks == 0) return TOPS_OK;
-  TOPS_REQUIRE(blocks < (1LL << 31), "tops_tri_generic_attention: too many query blocks");
-#define TOPS_GEN_ATTN(DMV)                                                                                           \
-  hipLaunchKernelGGL((tri_generic_attn_kernel<T, DMV, false>), dim3((unsigned)blocks), dim3(256), 0, st,            \
-                     (const T*)q, (const T*)k, (const T*)v, bias, (const int8_t*)mask, sm0, sm1, (T*)out, so0, so1, \
-                     N, N, H, D, scale)
-  if (D <= 16)
-    TOPS_GEN_ATTN(16);
+// Attention of R rows (q, k, v: (R, N, H, D) contiguous; mask rows sm0 apart, out rows so0 apart).
+template <typename T, bool MASK_INF>
+static int generic_attention_t(const char* name, const void* q, const void* k, const void* v, const float* bias,
+                               const void* mask, int64_t sm0, int64_t sm1, void* out, int64_t so0, int64_t so1,
+                               int64_t R, int64_t N, int H, int D, float scale, hipStream_t st) {
+  if (R * N == 0) return TOPS_OK;
+  const int64_t rh = R * H;
+  // keys split over the waves while 128-query blocks are fewer than the CUs (80 blocks, 600 tokens x 16
+  // heads of 24, bf16: 14 us against 31; 192 blocks, 1500 tokens: 41 against 75; 400 blocks, N = 100 x 4
+  // heads: 13 against 10)
+  const bool split = rh * ((N + 127) / 128) < num_cus();
+  const int64_t blocks = rh * (split ? (N + 31) / 32 : (N + 127) / 128);
+  TOPS_REQUIRE(blocks < (1LL << 31), "%s: too many query blocks", name);
+  const bool vec = aligned16({q, k, v, out}) && multiples_of(TileMma<T>::VE, {D, so0, so1});
+#define TOPS_GEN_ATTN(DP, KS, VEC)                                                                                  \
+  hipLaunchKernelGGL((tri_generic_attn_kernel<T, DP, KS, MASK_INF, VEC>), dim3((unsigned)blocks), dim3(256), 0, st, \
+                     (const T*)q, (const T*)k, (const T*)v, bias, (const int8_t*)mask, sm0, sm1, (T*)out, so0, so1,  \
+                     (int)N, H, D, scale)
+#define TOPS_GEN_ATTN_V(DP, KS) \
+  do {                          \
+    if (vec)                    \
+      TOPS_GEN_ATTN(DP, KS, true);  \
+    else                        \
+      TOPS_GEN_ATTN(DP, KS, false); \
+  } while (0)
+  if (split && D <= 16)
+    TOPS_GEN_ATTN_V(16, 4);
+  else if (split && D <= 32)
+    TOPS_GEN_ATTN_V(32, 4);
+  else if (split)
+    TOPS_GEN_ATTN_V(64, 4);
+  else if (D <= 16)
+    TOPS_GEN_ATTN_V(16, 1);
   else if (D <= 32)
-    TOPS_GEN_ATTN(32);
+    TOPS_GEN_ATTN_V(32, 1);
   else
-    TOPS_GEN_ATTN(64);
+    TOPS_GEN_ATTN_V(64, 1);
+#undef TOPS_GEN_ATTN_V
 #undef TOPS_GEN_ATTN
-  return launched("tops_tri_generic_attention");
+  return launched(name);
 }
 
 template <typename T>
@@ -708,26 +774,6 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
                        (size_t)kGenTok * Cz * sizeof(float), st, (const T*)Z, sz0, sz1, Wc, Bc, bias, M, Cz, H, eps);
   }
   return launched("tops_apb_generic_prep");
-}
-
-template <typename T>
-static int apb_generic_attention_t(const void* q, const void* k, const void* v, const float* bias, const void* mask,
-                                   void* Og, int64_t M, int H, int D, float scale, hipStream_t st) {
-  const int64_t blocks = H * ((M + 63) / 64);
-  if (blocks == 0) return TOPS_OK;
-  const int64_t HD = (int64_t)H * D;
-#define TOPS_GEN_APB(DMV)                                                                                         \
-  hipLaunchKernelGGL((tri_generic_attn_kernel<T, DMV, true>), dim3((unsigned)blocks), dim3(256), 0, st,          \
-                     (const T*)q, (const T*)k, (const T*)v, bias, (const int8_t*)mask, 0, 1, (T*)Og, 0, HD, 1, M, \
-                     H, D, scale)
-  if (D <= 16)
-    TOPS_GEN_APB(16);
-  else if (D <= 32)
-    TOPS_GEN_APB(32);
-  else
-    TOPS_GEN_APB(64);
-#undef TOPS_GEN_APB
-  return launched("tops_apb_generic_attention");
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1169,13 +1215,14 @@ extern "C" int tops_tri_generic_attention(const void* q, const void* k, const vo
                (long long)H, (long long)D);
   hipStream_t st = (hipStream_t)stream;
   if (dtype == TOPS_DTYPE_BF16)
-    return tri_generic_attention_t<__bf16>(q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, (int)H, (int)D, scale,
-                                           st);
+    return generic_attention_t<__bf16, false>("tops_tri_generic_attention", q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, N,
+                                      (int)H, (int)D, scale, st);
   if (dtype == TOPS_DTYPE_F16)
-    return tri_generic_attention_t<_Float16>(q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, (int)H, (int)D, scale,
-                                             st);
+    return generic_attention_t<_Float16, false>("tops_tri_generic_attention", q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, N,
+                                      (int)H, (int)D, scale, st);
   if (dtype == TOPS_DTYPE_F32)
-    return tri_generic_attention_t<float>(q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, (int)H, (int)D, scale, st);
+    return generic_attention_t<float, false>("tops_tri_generic_attention", q, k, v, bias, mask, sm0, sm1, out, so0, so1, N, N,
+                                      (int)H, (int)D, scale, st);
   return fail(TOPS_EUNSUPPORTED, "tops_tri_generic_attention: unsupported dtype code %d", dtype);
 }
 
@@ -1211,11 +1258,14 @@ extern "C" int tops_apb_generic_attention(const void* q, const void* k, const vo
                (long long)H, (long long)D);
   hipStream_t st = (hipStream_t)stream;
   if (dtype == TOPS_DTYPE_BF16)
-    return apb_generic_attention_t<__bf16>(q, k, v, bias, mask, Og, M, (int)H, (int)D, scale, st);
+    return generic_attention_t<__bf16, true>("tops_apb_generic_attention", q, k, v, bias, mask, 0, 1, Og, 0, H * D, 1, M, (int)H,
+                                     (int)D, scale, st);
   if (dtype == TOPS_DTYPE_F16)
-    return apb_generic_attention_t<_Float16>(q, k, v, bias, mask, Og, M, (int)H, (int)D, scale, st);
+    return generic_attention_t<_Float16, true>("tops_apb_generic_attention", q, k, v, bias, mask, 0, 1, Og, 0, H * D, 1, M, (int)H,
+                                     (int)D, scale, st);
   if (dtype == TOPS_DTYPE_F32)
-    return apb_generic_attention_t<float>(q, k, v, bias, mask, Og, M, (int)H, (int)D, scale, st);
+    return generic_attention_t<float, true>("tops_apb_generic_attention", q, k, v, bias, mask, 0, 1, Og, 0, H * D, 1, M, (int)H,
+                                     (int)D, scale, st);
   return fail(TOPS_EUNSUPPORTED, "tops_apb_generic_attention: unsupported dtype code %d", dtype);
 }
 

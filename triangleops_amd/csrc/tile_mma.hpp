@@ -27,6 +27,21 @@ struct TileMma<float> {
   }
 };
 
+// Raw buffer loads: 32-bit byte offsets from one base, reads at or past `bytes` return 0.
+using Rsrc = __amdgpu_buffer_rsrc_t;
+__device__ inline Rsrc buffer_of(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+template <typename V>
+__device__ inline V buffer_load(Rsrc r, uint32_t off) {
+  if constexpr (sizeof(V) == 16)
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  else if constexpr (sizeof(V) == 4)
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  else
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+}
+
 // Channels of an LDS token row: C rounded up to 32, the tail zero.  Rows are 16 bytes longer than
 // that, an odd number of 16-byte slots, so 16 rows read together hit 16 distinct bank groups.
 __host__ __device__ inline int tile_kp(int C) { return (C + 31) / 32 * 32; }
