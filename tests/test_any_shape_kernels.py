@@ -162,3 +162,32 @@ def test_attention_any_shape(device, dtype, N, H, D, mask):
     size = torch.einsum("ihqk,ikhd->iqhd", p, v.double().abs()).reshape(R, N, H * D)
     # fp32 scores of a few units are off by some 2^-22, the weights relatively so; one rounding of the result
     _within(out, ref, 0.5 * EPS[dtype] * ref.abs() + EPS[torch.float32] * size + 1e-7, f"{dtype} {N} {H} {D} {mask}")
+
+
+# pairs: one, below and past a 16-pair step, several steps per wave; C_z of every chunk count with tails;
+# one, exactly 16 and more heads
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("M,Cz,H", [(1, 128, 4), (3, 8, 1), (5, 33, 17), (40, 64, 16), (67, 250, 3), (260, 128, 16),
+                                    (33, 256, 5), (20, 300, 2)])
+@pytest.mark.parametrize("offset", [0.0, 30.0])
+def test_apb_bias_any_shape(device, dtype, M, Cz, H, offset):
+    """The pair bias LN(z) . Wc + Bc of a Z slice with odd strides (offset 0) or of contiguous Z whose
+    values share an offset (the statistics must not cancel)."""
+    from triangleops_amd import _native
+    from triangleops_amd._common.dtype import any_shape_dtype_code
+
+    g = torch.Generator().manual_seed(M + Cz)
+    z = (_rnd(g, torch.float64, M, M, Cz + (1 if offset == 0 else 0)) + offset).to(dtype)
+    zd = z.to(device)[..., :Cz]
+    z = z[..., :Cz].double()
+    wc, bc = _rnd(g, torch.float32, H, Cz, scale=Cz**-0.5), _rnd(g, torch.float32, H)
+    wd, bd = wc.to(device), bc.to(device)
+    x, w = torch.zeros(M, 8, device=device, dtype=dtype), torch.zeros(H, 3, 8, 8, device=device, dtype=dtype)
+    scratch, out = torch.empty(3, M, H * 8, device=device, dtype=dtype), torch.empty(H, M, M, device=device)
+    _native.call("tops_apb_generic_prep", x.data_ptr(), w.data_ptr(), zd.data_ptr(), zd.stride(0), zd.stride(1),
+                 wd.data_ptr(), bd.data_ptr(), *(t.data_ptr() for t in scratch), out.data_ptr(), M, 8, Cz, H, 8, 1e-5,
+                 any_shape_dtype_code(dtype), _native.stream_of(x))
+    mean, std = z.mean(-1, keepdim=True), (z.var(-1, correction=0, keepdim=True) + 1e-5).sqrt()
+    ref = ((z - mean) / std @ wc.double().T + bc.double()).permute(2, 0, 1)
+    size = ((z.abs() + mean.abs()) / std @ wc.double().abs().T + bc.double().abs()).permute(2, 0, 1)
+    _within(out, ref, EPS[torch.float32] * size, f"bias {dtype} {M} {Cz} {H}")

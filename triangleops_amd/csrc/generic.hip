@@ -468,71 +468,6 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Tiled pre-pass and gate for C_in <= 256 (and H * D <= 256 for the gate): 64 tokens per block,
-// 256 threads.  Activations go to LDS k-major ([channel][token], fp32); every product is a block
-// GEMM over that tile (tiled_gemm64: weights of 64 output features at a time staged k-major
-// through LDS in 32-deep k-tiles, 4 tokens x 4 features per thread in registers).  Rounding
-// points are those of the per-token kernels above.
-// ---------------------------------------------------------------------------------------------
-constexpr int kGT = 64, kGRow = kGT + 4;  // tokens per tile, LDS row of the k-major tiles
-
-// LayerNorm (optionally with the affine w, b) of the kGT token columns of a k-major tile, in place
-// (fp32, two-pass, 4 threads per token); rows [C, CK) are set to zero.
-template <typename T>
-__device__ __attribute__((always_inline)) inline void tiled_ln_affine(float* xs, int C, int CK, const T* __restrict__ w, const T* __restrict__ b,
-                                       float eps) {
-  const int t = threadIdx.x >> 2, part = threadIdx.x & 3;
-  float s = 0.f;
-  for (int k = part; k < C; k += 4) s += xs[k * kGRow + t];
-  const float mean = group_sum<4>(s) / (float)C;
-  float q = 0.f;
-  for (int k = part; k < C; k += 4) {
-    const float d = xs[k * kGRow + t] - mean;
-    q = fmaf(d, d, q);
-  }
-  const float rstd = rsqrtf(group_sum<4>(q) / (float)C + eps);
-  for (int k = part; k < CK; k += 4) {
-    float v = 0.f;
-    if (k < C) {
-      v = (xs[k * kGRow + t] - mean) * rstd;
-      if (w) v = v * (float)w[k] + (b ? (float)b[k] : 0.f);
-    }
-    xs[k * kGRow + t] = v;
-  }
-}
-
-// Loads the rows of kGT tokens into a k-major tile dst[c][t] (c < C; rows [C, CK) and tokens
-// t >= ntok are zeros; CK <= 256): wave w takes tokens w, w + 4, ..., its lanes consecutive
-// channels, and row(t) gives the element offset of token t's row (once per token, wave-uniform).
-// Four tokens' loads are issued before their LDS stores, so their latencies overlap.
-template <typename T, typename Row>
-__device__ __attribute__((always_inline)) inline void tiled_load_rows(float* dst, const T* __restrict__ src, int C,
-                                                                      int CK, int ntok, Row row) {
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int t0 = wave; t0 < kGT; t0 += 16) {
-    float v[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int t = t0 + 4 * a;
-      const bool ok = t < ntok;
-      const int64_t r0 = ok ? row(t) : 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int c = lane + 64 * b;
-        v[a][b] = ok && c < C ? (float)src[r0 + c] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int c = lane + 64 * b;
-        if (c < CK) dst[c * kGRow + t0 + 4 * a] = v[a][b];
-      }
-  }
-}
-
 template <typename T>
 static int tri_generic_prep_t(const void* x, int64_t sx0, int64_t sx1, const void* w_ln, const void* b_ln,
                               int apply_ln, const void* wqkv, const void* WZ, const float* BZ, void* xln, void* q,
@@ -704,36 +639,92 @@ __global__ __launch_bounds__(256) void apb_generic_bias_kernel(const T* __restri
   }
 }
 
-// Tiled form for C_z <= 256: a LayerNorm of 64 pairs in LDS, then per head (one wave each) the dot
-// products of its 64 pairs (lanes) with the head's weights (wave-uniform: scalar loads).
-template <typename T>
-__global__ __launch_bounds__(256) void apb_gen_bias_tiled_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
-                                                                const float* __restrict__ Wc,
-                                                                const float* __restrict__ Bc, float* __restrict__ bias,
-                                                                int64_t M, int Cz, int H, float eps) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CzK = (Cz + kTK - 1) / kTK * kTK;
-  float* zs = sm;  // [CzK][kGRow]  LN(Z) of 64 pairs, k-major
-  const int tid = threadIdx.x;
-  const int64_t npair = M * M, p0 = (int64_t)blockIdx.x * kGT;
-  const int np = (int)(npair - p0 < kGT ? npair - p0 : kGT);
-  tiled_load_rows<T>(zs, Z, Cz, CzK, np, [=](int t) {
-    const int64_t pr = p0 + t;
-    return (pr / M) * sz0 + (pr % M) * sz1;
-  });
-  __syncthreads();
-  tiled_ln_affine<T>(zs, Cz, CzK, nullptr, nullptr, eps);
-  __syncthreads();
-  const int lane = tid & 63;
-  for (int h = __builtin_amdgcn_readfirstlane(tid >> 6); h < H; h += 4) {
-    const float* w = Wc + (int64_t)h * Cz;
-    float acc[4] = {Bc[h], 0.f, 0.f, 0.f};
-    int c = 0;
-    for (; c + 4 <= Cz; c += 4)
+// C_z <= 4 VE NKC: 16 pairs and 16 heads (blockIdx.y) per wave and step.  Lane quarter qd holds the
+// 16-byte chunks 4 j + qd of pair lane % 16, takes the two-pass LayerNorm in registers and feeds the
+// normalised fp32 values to v_mfma_f32_16x16x4_f32 against the fp32 folded weights, which stay in
+// registers over all steps.  The next step's loads are issued before this step's arithmetic.  Bound by
+// the read of Z and the matrix cores together (600 tokens, 16 heads, C_z = 128, bf16: 148 -> 39 us
+// against LDS tiles and FMAs, 2.9 TB/s).
+template <typename T, int NKC, bool VEC>
+__global__ __launch_bounds__(256) void apb_gen_bias_mma_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
+                                                              const float* __restrict__ Wc,
+                                                              const float* __restrict__ Bc, float* __restrict__ bias,
+                                                              uint32_t M, int Cz, int H, float eps) {
+  using TM = TileMma<T>;
+  using V = typename TM::V;
+  constexpr int VE = TM::VE;
+  const int lane = threadIdx.x & 63, qd = lane >> 4, col = lane & 15;
+  const int h0 = 16 * blockIdx.y, hr = h0 + col < H ? h0 + col : H - 1;
+  const uint32_t npair = M * M, nstep = (npair + 15) / 16;
+  const uint32_t nw = gridDim.x * 4, w0 = blockIdx.x * 4 + (threadIdx.x >> 6);
+  float wr[NKC][VE], bc[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = fmaf(zs[(c + j) * kGRow + lane], w[c + j], acc[j]);
-    for (; c < Cz; ++c) acc[0] = fmaf(zs[c * kGRow + lane], w[c], acc[0]);
-    if (lane < np) bias[(int64_t)h * npair + p0 + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  for (int j = 0; j < NKC; ++j)
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+      const int k = (4 * j + qd) * VE + e;
+      wr[j][e] = k < Cz ? Wc[(int64_t)hr * Cz + k] : 0.f;
+    }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) bc[v] = h0 + 4 * qd + v < H ? Bc[h0 + 4 * qd + v] : 0.f;
+  auto load = [&](V(&z)[NKC], uint32_t step) __attribute__((always_inline)) {
+    uint32_t p = step * 16 + col;
+    p = p < npair ? p : npair - 1;
+    const uint32_t a = p / M, b = p - a * M;
+    const T* src = Z + a * sz0 + b * sz1;
+#pragma unroll
+    for (int j = 0; j < NKC; ++j) {
+      const int k = (4 * j + qd) * VE;
+      if constexpr (VEC) {
+        z[j] = ldg<V>(src + (k < Cz ? k : 0));
+        if (k >= Cz) z[j] = V{};
+      } else {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) z[j][e] = k + e < Cz ? src[k + e] : (T)0.f;
+      }
+    }
+  };
+  auto quarters = [&](float v) __attribute__((always_inline)) {  // sum over the pair's four lanes
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return halves_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  };
+  auto compute = [&](const V(&z)[NKC], uint32_t step) __attribute__((always_inline)) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NKC; ++j)
+#pragma unroll
+      for (int e = 0; e < VE; ++e) s += (float)z[j][e];
+    const float mean = quarters(s) / (float)Cz;
+    float q = 0.f, d[NKC][VE];
+#pragma unroll
+    for (int j = 0; j < NKC; ++j)
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        d[j][e] = (4 * j + qd) * VE + e < Cz ? (float)z[j][e] - mean : 0.f;
+        q = fmaf(d[j][e], d[j][e], q);
+      }
+    const float rstd = rsqrtf(quarters(q) / (float)Cz + eps);
+    f32x4 acc = {};
+#pragma unroll
+    for (int j = 0; j < NKC; ++j)
+#pragma unroll
+      for (int e = 0; e < VE; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[j][e], d[j][e] * rstd, acc, 0, 0, 0);
+    const uint32_t p = step * 16 + col;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int h = h0 + 4 * qd + v;
+      if (p < npair && h < H) bias[(int64_t)h * npair + p] = acc[v] + bc[v];
+    }
+  };
+  V za[NKC], zb[NKC];
+  uint32_t t = w0;
+  if (t < nstep) load(za, t);
+  for (; t < nstep; t += 2 * nw) {
+    if (t + nw < nstep) load(zb, t + nw);
+    compute(za, t);
+    if (t + nw >= nstep) break;
+    if (t + 2 * nw < nstep) load(za, t + 2 * nw);
+    compute(zb, t + nw);
   }
 }
 
@@ -741,8 +732,6 @@ template <typename T>
 static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, int64_t sz0, int64_t sz1,
                               const float* Wc, const float* Bc, void* q, void* k, void* v, float* bias, int64_t M,
                               int C, int Cz, int H, int D, float eps, hipStream_t st) {
-  // the tiled bias kernel takes 64 pairs per block: used where that still gives every CU a block
-  const int64_t t2 = (M * M + kGT - 1) / kGT;
   if (M == 0) return TOPS_OK;
   const int pw = qkv_piece<T>(D, q, k, v);
   {
@@ -761,13 +750,35 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
                          (T*)q, (T*)k, (T*)v, M, C, H, D, pw);
     }
   }
-  if (Cz <= 256 && t2 >= num_cus()) {
-    const int CzK = (Cz + kTK - 1) / kTK * kTK;
-    const size_t l2 = (size_t)CzK * kGRow * sizeof(float);
-    hipFuncSetAttribute((const void*)apb_gen_bias_tiled_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                        (int)l2);
-    hipLaunchKernelGGL((apb_gen_bias_tiled_kernel<T>), dim3((unsigned)t2), dim3(256), l2, st, (const T*)Z, sz0, sz1, Wc,
-                       Bc, bias, M, Cz, H, eps);
+  if (Cz <= 256 && M < 65536) {
+    const bool vec = aligned16({Z}) && multiples_of(TileMma<T>::VE, {sz0, sz1, Cz});
+    const int64_t steps = (M * M + 63) / 64;  // of 4 waves
+    // 2 blocks per CU: 600 tokens x 16 heads, C_z = 128 in bf16 39 us against 42 with 4 and 52 with 8 (whose
+    // waves take 3 and 1.5 steps each, unevenly), 500 tokens x 2 heads, C_z = 32 equal within 1 us
+    const dim3 grid((unsigned)(steps < 2 * num_cus() ? steps : 2 * num_cus()), (unsigned)((H + 15) / 16));
+#define TOPS_GEN_BIAS(NKC, VEC)                                                                                     \
+  hipLaunchKernelGGL((apb_gen_bias_mma_kernel<T, NKC, VEC>), grid, dim3(256), 0, st, (const T*)Z, sz0, sz1, Wc, Bc, \
+                     bias, (uint32_t)M, Cz, H, eps)
+#define TOPS_GEN_BIAS_V(NKC)    \
+  do {                          \
+    if (vec)                    \
+      TOPS_GEN_BIAS(NKC, true); \
+    else                        \
+      TOPS_GEN_BIAS(NKC, false);\
+  } while (0)
+    constexpr int W = 4 * TileMma<T>::VE;  // channels per chunk of the four lanes
+    if (Cz <= W)
+      TOPS_GEN_BIAS_V(1);
+    else if (Cz <= 2 * W)
+      TOPS_GEN_BIAS_V(2);
+    else if (Cz <= 4 * W)
+      TOPS_GEN_BIAS_V(4);
+    else if (Cz <= 8 * W)
+      TOPS_GEN_BIAS_V(8);
+    else if constexpr (sizeof(T) == 4)
+      TOPS_GEN_BIAS_V(16);
+#undef TOPS_GEN_BIAS_V
+#undef TOPS_GEN_BIAS
   } else {
     const int64_t b2 = (M * M + kGenTok - 1) / kGenTok;
     hipLaunchKernelGGL((apb_generic_bias_kernel<T>), dim3((unsigned)b2), dim3(256),
