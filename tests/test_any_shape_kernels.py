@@ -191,3 +191,51 @@ def test_apb_bias_any_shape(device, dtype, M, Cz, H, offset):
     ref = ((z - mean) / std @ wc.double().T + bc.double()).permute(2, 0, 1)
     size = ((z.abs() + mean.abs()) / std @ wc.double().abs().T + bc.double().abs()).permute(2, 0, 1)
     _within(out, ref, EPS[torch.float32] * size, f"bias {dtype} {M} {Cz} {H}")
+
+
+# one and several 64-token tiles per row with every kind of tail; C of one k-step, with tails, of one
+# and several weight batches, wider than the 64-token tile fits; few and many 32-feature chunks
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("B,L,C", [(1, 1, 8), (2, 33, 64), (1, 64, 96), (1, 65, 33), (1, 100, 256), (1, 20, 500),
+                                   (1, 200, 32)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_tmu_phases_any_shape(device, dtype, B, L, C, transpose):
+    """Input phase (masked, padded columns zero) and output phase (with a residual when transpose)."""
+    from triangleops_amd.triangle_mul.kernel import input_phase, output_phase
+
+    g = torch.Generator().manual_seed(L + C)
+    x, res = _rnd(g, dtype, B, L, L, C), _rnd(g, dtype, B, L, L, C)
+    mask = torch.rand(B, L, L, generator=g) < 0.8
+    ld = (L + 63) // 64 * 64
+    y = _rnd(g, dtype, C, B, L, ld)
+    y[..., L:] = float("nan")  # never part of a result
+    (wp, wg), (bp, bg) = (_rnd(g, dtype, 2, 2 * C, C, scale=C**-0.5), _rnd(g, torch.float32, 2, 2 * C))
+
+    def norm(t):
+        t = t.double()
+        return torch.nn.functional.layer_norm(t, (C,), eps=1e-5).to(dtype).double()
+
+    def gated(a, b, n):
+        w, v = wp[:n].double(), wg[:n].double()
+        p, s = a @ w.T + bp[:n].double(), torch.sigmoid(b @ v.T + bg[:n].double())
+        # rounding of the normalised operands (some 2e-2 of them close to a rounding step of x - mean)
+        slack = (a.abs() + 1e-2) @ w.T.abs() * s + p.abs() * s * (1 - s) * ((b.abs() + 1e-2) @ v.T.abs())
+        return p * s, EPS[dtype] * ((p * s).abs() + slack + 1e-3)
+
+    sums = torch.zeros(2 * C, device=device)
+    dev = [t.to(device) for t in (x, mask, wp, wg, bp, bg, y, res)]
+    ab = input_phase(dev[0], dev[1], dev[2], dev[3], sums, sums, dev[4], dev[5], 1e-5, transpose=transpose, ld=ld)
+    ref, bound = gated(norm(x), norm(x), 2 * C)
+    ref = ref * mask[..., None]
+    if transpose:
+        ref, bound = ref.transpose(1, 2), bound.transpose(1, 2)
+    assert ab.shape == (2 * C, B, L, ld) and not ab[..., L:].any()
+    _within(ab[..., :L], ref.permute(3, 0, 1, 2), bound.permute(3, 0, 1, 2), f"input phase {dtype} {L} {C}")
+
+    out = output_phase(dev[6], dev[0], dev[2][:C], dev[3][:C], sums[:C], sums[:C], dev[4][:C], dev[5][:C], 1e-5, ldy=ld,
+                       residual=dev[7] if transpose else None)
+    ref, bound = gated(norm(y[..., :L].permute(1, 2, 3, 0)), norm(x), C)
+    if transpose:
+        ref = res.double() + ref
+        bound = bound + EPS[dtype] * ref.abs()
+    _within(out, ref, bound, f"output phase {dtype} {L} {C}")

@@ -1,19 +1,17 @@
-// Any-shape kernels for the triangle-attention op and the gate / output projection: the
-// shapes the tuned kernels do not cover (C_in != 128, D != 32, H != 4, C_out != 128, e.g. the
-// D = 16, C_in = 64 "Apo" configuration).  Plain fp32 VALU arithmetic (no MFMA), written for
-// correctness at small and medium sizes, and the path of fp32 I/O (then every value stays fp32);
-// with 16-bit I/O the rounding points follow the tuned path:
+// Any-shape kernels: the shapes the tuned kernels do not cover, and fp32 I/O (then every value stays
+// fp32).  Products run on the matrix cores, 32x32x16 MFMAs in 16-bit types and 32x32x2 fp32 MFMAs
+// in fp32 (tile_mma.hpp); with 16-bit I/O the rounding points follow the tuned path:
 //   LN(x) is rounded to the I/O type before the Q / K / V and gate products, Q / K / V and the
-//   gated activations are rounded to the I/O type, the pair bias stays fp32.
+//   gated activations are rounded to the I/O type, the pair bias and the attention weights stay fp32.
 //
-//   tri_generic_prep_kernel   per token: LN(x) (fp32, two-pass), Q / K / V of all heads and
-//                             the row-shared pair bias bias[h][a][b] = LN(x[a, b]) . Wz[h] + bz[h]
-//   tri_generic_attn_kernel   64 queries of one (row i, head h) per block, keys split over 4 waves
-//                             in 32-key chunks staged in LDS: online softmax in fp32, scores
+//   tri_generic_prep_kernel   LN(x), Q / K / V of all heads and the row-shared pair bias
+//                             bias[h][a][b] = LN(x[a, b]) . Wz[h] + bz[h]
+//   tri_generic_attn_kernel   32 queries of one (row i, head h) per wave: online softmax in fp32, scores
 //                             q . k * scale + bias, masked keys get the reference's fp32 "+ (-1e9)"
-//   gate_generic_kernel       per token: y = (o * sigmoid(g . Wg^T + bg)) -> io, out = y . Wo^T + bo
+//   gate_generic_kernel       y = (o * sigmoid(g . Wg^T + bg)) -> io, out = y . Wo^T + bo
 //                             with g = LN(gin) or gin
-//
+//   apb_generic_qkv_kernel, apb_gen_bias_mma_kernel (C_z <= 256), apb_generic_bias_kernel (wider; fp32
+//                             FMAs): attention_pair_bias's projections and pair bias
 //   tmu_generic_in_kernel     triangle_multiplicative_update input phase at any C / C_out:
 //                             ab[f] = (xn . Wp[f] + Bp[f]) * sigmoid(xn . Wg[f] + Bg[f]) * mask,
 //                             xn = (x - mean) * rstd (the LN affine is folded into Wp / Wg)
@@ -33,7 +31,6 @@
 namespace tops {
 
 constexpr int kGenTok = 16;  // tokens per block; 16 lanes per token for the LayerNorm sums
-constexpr int kTK = 32;      // k-tile of the weights the tiled kernels stage through LDS
 
 // Conditions of a kernel's 16-byte accesses (a null pointer is not accessed).
 static bool aligned16(std::initializer_list<const void*> ps) {
@@ -197,11 +194,11 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
   __syncthreads();
   for (int f0 = 32 * wave; f0 < F; f0 += 128) {
     const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
-    f32x16 acc[1] = {};
+    f32x16 acc[1][1] = {};
     tile_gemm<T, 1, true, VEC>(acc, xs, rx, col, wqkv + (int64_t)(row < F ? row : F - 1) * C, C);
     if (tok0 + col < ntok)
       store_qkv16<T>(qo, ko, vo, (tok0 + col) * HD, fl, F - fl, D, pw,
-                     [&](int v) __attribute__((always_inline)) { return acc[0][v]; });
+                     [&](int v) __attribute__((always_inline)) { return acc[0][0][v]; });
   }
 }
 
@@ -440,12 +437,12 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
   // gate: ys = io(o * sigmoid(g . Wg + bg)), each element rewritten by the lane that reads it
   for (int f0 = 32 * wave; f0 < HD; f0 += 32 * NW) {
     const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
-    f32x16 acc[1] = {};
+    f32x16 acc[1][1] = {};
     tile_gemm<T, 1, true, VEC>(acc, gs, rg, col, Wg + (int64_t)(row < HD ? row : HD - 1) * Cin, Cin);
     const f32x16 b = load16<T, VEC>(bg && fl < HD ? bg + fl : nullptr, HD - fl);
     T* y = ys + col * ry + fl;
     store16<T, true>(y, 16, [&](int v) __attribute__((always_inline)) {
-      return (T)((float)y[v] * sigmoid(acc[0][v] + b[v]));
+      return (T)((float)y[v] * sigmoid(acc[0][0][v] + b[v]));
     });
   }
   __syncthreads();
@@ -453,7 +450,7 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
   const int64_t tok = tok0 + col < M ? tok0 + col : M - 1, m1 = tok / M2, m2 = tok - m1 * M2;
   for (int f0 = 32 * wave; f0 < Cout; f0 += 32 * NW) {
     const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
-    f32x16 acc[1] = {};
+    f32x16 acc[1][1] = {};
     tile_gemm<T, 1, true, VEC>(acc, ys, ry, col, Wo + (int64_t)(row < Cout ? row : Cout - 1) * HD, HD);
     if (tok0 + col >= M || fl >= Cout) continue;
     const f32x16 b = load16<T, VEC>(bo ? bo + fl : nullptr, Cout - fl);
@@ -461,9 +458,9 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
     if (res) {
       const f32x16 r = load16<T, VEC>(res + m1 * sr0 + m2 * sr1 + fl, Cout - fl);
       store16<T, VEC>(dst, Cout - fl,
-                      [&](int v) __attribute__((always_inline)) { return (T)(r[v] + (float)(T)(acc[0][v] + b[v])); });
+                      [&](int v) __attribute__((always_inline)) { return (T)(r[v] + (float)(T)(acc[0][0][v] + b[v])); });
     } else {
-      store16<T, VEC>(dst, Cout - fl, [&](int v) __attribute__((always_inline)) { return (T)(acc[0][v] + b[v]); });
+      store16<T, VEC>(dst, Cout - fl, [&](int v) __attribute__((always_inline)) { return (T)(acc[0][0][v] + b[v]); });
     }
   }
 }
@@ -599,7 +596,7 @@ __global__ __launch_bounds__(256) void apb_generic_qkv_kernel(const T* __restric
   const int t = tid >> 3, part = tid & 7;
   const bool ok = tok0 + t < M;
   const T* src = X + (ok ? tok0 + t : M - 1) * C;
-  f32x16 acc[1] = {};
+  f32x16 acc[1][1] = {};
   for (int c0 = 0; c0 < C; c0 += kQkvC) {
     const int kc = C - c0 < kQkvC ? C - c0 : kQkvC;
     if (c0 > 0) __syncthreads();
@@ -609,7 +606,7 @@ __global__ __launch_bounds__(256) void apb_generic_qkv_kernel(const T* __restric
   }
   if (tok0 + col < M && f0 < F)
     store_qkv16<T>(qo, ko, vo, (tok0 + col) * HD, fl, F - fl, D, pw,
-                   [&](int v) __attribute__((always_inline)) { return acc[0][v]; });
+                   [&](int v) __attribute__((always_inline)) { return acc[0][0][v]; });
 }
 
 template <typename T>
@@ -789,308 +786,254 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
 
 // ---------------------------------------------------------------------------------------------
 // triangle_multiplicative_update, any C (triangle_mul/module.py:8-12: x is (B, L, L, D), any D;
-// triangle_mul/kernel.py:235-326).  Tokens t = (b, i, j) in row-major order.
+// triangle_mul/kernel.py:235-326).  Both phases take 32 NB tokens per block of 4 waves, normalised in LDS
+// (rounded to the I/O type as the products' operand); a wave takes units of one 32-feature chunk of
+// the weights and 32 NU tokens in turn.
+//   input phase:  the tile is part of one row r of the (B, L, ld) store grid (tokens (r, c) or,
+//                 transposed, (c, r), c = c0 ..; c >= L stores zeros).  Tokens are the A operand, so a
+//                 lane holds 16 consecutive tokens of one feature of P and of G; the gated values go
+//                 through a per-wave LDS tile, so each store instruction writes whole 64 NB-byte (fp32:
+//                 128 NB) pieces of the features' rows.
+//   output phase: tokens (b, i, j0 ..); y, channel-major, is transposed on its way into LDS.  Weights are
+//                 the A operand, so a lane holds 16 consecutive features of one token.
+// Bound by the fp32 MFMAs in fp32 (L = 256, C = 128: input / output phase 174 / 181 -> 91 / 66 us against
+// VALU block products, 94 and 65 TFLOP/s) and by memory and the weight reads in 16-bit types (bf16 L = 512,
+// C = 64: 174 / 320 -> 41 / 39 us, 2.5 TB/s).  Three waves per SIMD: left to itself the compiler takes the
+// registers of one more (46 / 45 us), four spill (63 / 38).
 // ---------------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void tmu_generic_in_kernel(const T* __restrict__ x, const int8_t* __restrict__ mask,
+template <typename T, int NB, int NU, bool VEC>
+__global__ __launch_bounds__(256, 3) void tmu_generic_in_kernel(const T* __restrict__ x, const int8_t* __restrict__ mask,
                                                             const T* __restrict__ Wp, const T* __restrict__ Wg,
                                                             const float* __restrict__ Bp, const float* __restrict__ Bg,
-                                                            T* __restrict__ ab, int64_t B, int64_t L, int C, int Cout,
-                                                            int64_t ld, int transpose, float eps) {
-  extern __shared__ float xs[];  // [kGenTok][C]
-  const int tid = threadIdx.x;
-  const int64_t ntok = B * L * L, tok0 = (int64_t)blockIdx.x * kGenTok;
-  for (int e = tid; e < kGenTok * C; e += 256) {
-    const int64_t tok = tok0 + e / C;
-    xs[e] = tok < ntok ? (float)x[tok * C + e % C] : 0.f;
+                                                            T* __restrict__ ab, uint32_t L, int C, int Cout, uint32_t ld,
+                                                            int64_t fstride, int transpose, float eps) {
+  using M = TileMma<T>;
+  using V = typename M::V;
+  constexpr int TT = 32 * NB, TPT = 256 / TT, UT = 32 * NU, OR = UT + M::VE;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int rx = tile_row<T>(C);
+  T* xs = reinterpret_cast<T*>(smem);          // [TT][rx] normalised tokens
+  T* ost = xs + TT * rx;                       // [4 waves][32][OR] output features x tokens
+  float* msk = reinterpret_cast<float*>(ost + 4 * 32 * OR);  // [TT] 1 for a valid, unmasked token
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const uint32_t tpr = ld / TT, rr = blockIdx.x / tpr, c0 = (blockIdx.x - rr * tpr) * TT, bb = rr / L, r = rr - bb * L;
+  {
+    const int t = tid / TPT, part = tid % TPT;
+    const uint32_t c = c0 + t < L ? c0 + t : L - 1;
+    const int64_t tok = transpose ? ((int64_t)bb * L + c) * L + r : ((int64_t)bb * L + r) * L + c;
+    T* row = xs + t * rx;
+    stage_row<T, TPT, VEC>(row, x + tok * C, true, part, C, tile_kp(C));
+    float mean, rstd;
+    row_stats<T, TPT>(row, part, C, eps, mean, rstd);
+    normalise_row<T, TPT>(row, part, C, mean, rstd, nullptr, nullptr);
+    if (part == 0) msk[t] = c0 + t < L && (!mask || mask[tok] != 0) ? 1.f : 0.f;
   }
   __syncthreads();
-  gen_layer_norm<T>(xs, C, C, nullptr, nullptr, eps);
-  __syncthreads();
-  for (int e = tid; e < kGenTok * C; e += 256) xs[e] = (float)(T)xs[e];  // GEMM operand in the I/O type
-  __syncthreads();
-  const int64_t fstride = B * L * ld;
-  for (int e = tid; e < kGenTok * Cout; e += 256) {
-    const int t = e / Cout, f = e % Cout;
-    const int64_t tok = tok0 + t;
-    if (tok >= ntok) continue;
-    const float* r = xs + t * C;
-    const T* wp = Wp + (int64_t)f * C;
-    const T* wg = Wg + (int64_t)f * C;
-    float p = Bp[f], g = Bg[f];
-    for (int c = 0; c < C; ++c) {
-      p = fmaf(r[c], (float)wp[c], p);
-      g = fmaf(r[c], (float)wg[c], g);
+  T* o = ost + wave * 32 * OR;
+  T* abt = ab + ((int64_t)bb * L + r) * ld + c0;
+  const int nunits = (Cout + 31) / 32 * (NB / NU);
+  for (int u = wave; u < nunits; u += 4) {
+    const int f0 = 32 * (u / (NB / NU)), t0 = UT * (u % (NB / NU));
+    const int f = f0 + col < Cout ? f0 + col : Cout - 1;
+    f32x16 acc[2][NU] = {};
+    const T* const w[2] = {Wp + (int64_t)f * C, Wg + (int64_t)f * C};
+    tile_gemm_n<T, 2, NU, false, VEC, 2>(acc, xs + t0 * rx, rx, tile_perm(col), w, C);
+    const float bp = Bp[f], bg = Bg[f];
+#pragma unroll
+    for (int n = 0; n < NU; ++n) {
+      const float* mk = msk + t0 + 32 * n + 16 * hl;
+      store16<T, true>(o + col * OR + 32 * n + 16 * hl, 16, [&](int v) __attribute__((always_inline)) {
+        return (T)((acc[0][n][v] + bp) * sigmoid(acc[1][n][v] + bg) * mk[v]);
+      });
     }
-    const float m = mask ? (mask[tok] != 0 ? 1.f : 0.f) : 1.f;
-    const int64_t b = tok / (L * L), rem = tok % (L * L), i = rem / L, j = rem % L;
-    const int64_t row = transpose ? j : i, col = transpose ? i : j;
-    T* dst = ab + f * fstride + (b * L + row) * ld;
-    dst[col] = (T)(p * sigmoid(g) * m);
-    if (col == L - 1)  // zero k-padding of this row for the einsum
-      for (int64_t c = L; c < ld; ++c) dst[c] = (T)0.f;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    constexpr int LPR = UT / M::VE, FPI = 64 / LPR;  // lanes per feature row, features per instruction
+#pragma unroll
+    for (int k = 0; k < 32 / FPI; ++k) {
+      const int fr = k * FPI + lane / LPR, tc = lane % LPR * M::VE;
+      const V v = *reinterpret_cast<const V*>(o + fr * OR + tc);
+      if (f0 + fr < Cout) {
+        T* dst = abt + (int64_t)(f0 + fr) * fstride + t0 + tc;
+        if constexpr (VEC) {
+          *reinterpret_cast<V*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < M::VE; ++e) dst[e] = v[e];
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // read before the next unit overwrites it
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void tmu_generic_out_kernel(const T* __restrict__ y, const T* __restrict__ x,
+template <typename T, int NB, int NU, bool VEC>
+__global__ __launch_bounds__(256, 3) void tmu_generic_out_kernel(const T* __restrict__ y, const T* __restrict__ x,
                                                              const T* __restrict__ Wp, const T* __restrict__ Wg,
                                                              const float* __restrict__ Bp,
                                                              const float* __restrict__ Bg, const T* __restrict__ res,
-                                                             T* __restrict__ out, int64_t B, int64_t L, int C,
-                                                             int Cout, int64_t ldy, float eps) {
-  extern __shared__ float sm[];
-  float* ys = sm;                 // [kGenTok][C]  y of the tile's tokens (token-major)
-  float* xs = sm + kGenTok * C;   // [kGenTok][C]  x
-  const int tid = threadIdx.x;
-  const int64_t ntok = B * L * L, tok0 = (int64_t)blockIdx.x * kGenTok, cstride = B * L * ldy;
-  for (int e = tid; e < kGenTok * C; e += 256) {
-    const int t = e % kGenTok, c = e / kGenTok;  // token fastest: y is channel-major
-    const int64_t tok = tok0 + t;
-    float v = 0.f;
-    if (tok < ntok) {
-      const int64_t b = tok / (L * L), rem = tok % (L * L);
-      v = (float)y[c * cstride + (b * L + rem / L) * ldy + rem % L];
-    }
-    ys[t * C + c] = v;
-  }
-  for (int e = tid; e < kGenTok * C; e += 256) {
-    const int64_t tok = tok0 + e / C;
-    xs[e] = tok < ntok ? (float)x[tok * C + e % C] : 0.f;
-  }
-  __syncthreads();
-  gen_layer_norm<T>(ys, C, C, nullptr, nullptr, eps);
-  gen_layer_norm<T>(xs, C, C, nullptr, nullptr, eps);
-  __syncthreads();
-  for (int e = tid; e < 2 * kGenTok * C; e += 256) sm[e] = (float)(T)sm[e];
-  __syncthreads();
-  for (int e = tid; e < kGenTok * Cout; e += 256) {
-    const int t = e / Cout, f = e % Cout;
-    const int64_t tok = tok0 + t;
-    if (tok >= ntok) continue;
-    const float* yr = ys + t * C;
-    const float* xr = xs + t * C;
-    const T* wp = Wp + (int64_t)f * C;
-    const T* wg = Wg + (int64_t)f * C;
-    float p = Bp[f], g = Bg[f];
-    for (int c = 0; c < C; ++c) {
-      p = fmaf(yr[c], (float)wp[c], p);
-      g = fmaf(xr[c], (float)wg[c], g);
-    }
-    const T r = (T)(p * sigmoid(g));
-    out[tok * Cout + f] = res ? (T)((float)res[tok * Cout + f] + (float)r) : r;
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Tiled forms of the two phases for C <= 256 (the kernels above remain for wider C): a block
-// takes a tile of tokens, normalises them into LDS k-major ([channel][token], fp32, rounded to
-// the I/O type as the products' operand, exactly as above), stages the weights of a chunk of
-// output features k-major through LDS in 32-deep k-tiles, and each thread accumulates 4 tokens
-// x 4 features of P and of G in registers (fp32 FMAs), then applies bias, gate and mask.
-//   input phase:  64 tokens of one row r of the (B, L, ld) store grid (tokens (r, c) or,
-//                 transposed, (c, r), c = c0 .. c0 + 63; c >= L stores zeros), 64-feature chunks,
-//                 each thread's 4 tokens stored as one vector per feature (contiguous in ab)
-//   output phase: 32 tokens (b, i, j0 .. j0 + 31), y read channel-major 32 tokens per channel,
-//                 128-feature chunks, each thread's 4 features stored as one vector per token
-// ---------------------------------------------------------------------------------------------
-constexpr int kTinTok = 64, kTinRow = kTinTok + 4;    // input phase: tokens per tile, LDS row
-constexpr int kToutTok = 32, kToutRow = kToutTok + 4;  // output phase
-constexpr int kTF = 128, kTFRow = kTF + 4;              // output phase: features per chunk, LDS row
-
-// LayerNorm of the `ntok` token columns of a k-major LDS tile (4 threads per token, two-pass),
-// rounding the normalised values to T; rows k in [C, CK) are set to zero.
-template <typename T>
-__device__ inline void tiled_layer_norm(float* xs, int row, int ntok, int C, int CK, float eps) {
-  const int t = threadIdx.x >> 2, part = threadIdx.x & 3;
-  if (t >= ntok) return;  // whole quads drop out together, so the quad sums stay exact
-  float s = 0.f;
-  for (int k = part; k < C; k += 4) s += xs[k * row + t];
-  const float mean = group_sum<4>(s) / (float)C;
-  float q = 0.f;
-  for (int k = part; k < C; k += 4) {
-    const float d = xs[k * row + t] - mean;
-    q = fmaf(d, d, q);
-  }
-  const float rstd = rsqrtf(group_sum<4>(q) / (float)C + eps);
-  for (int k = part; k < CK; k += 4) xs[k * row + t] = k < C ? (float)(T)((xs[k * row + t] - mean) * rstd) : 0.f;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void tmu_gen_in_tiled_kernel(const T* __restrict__ x, const int8_t* __restrict__ mask,
-                                                              const T* __restrict__ Wp, const T* __restrict__ Wg,
-                                                              const float* __restrict__ Bp, const float* __restrict__ Bg,
-                                                              T* __restrict__ ab, int64_t L, int C, int Cout, int64_t ld,
-                                                              int64_t fstride, int transpose, float eps) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CK = (C + kTK - 1) / kTK * kTK;
-  float* xs = sm;                     // [CK][kTinRow]  normalised tile
-  float* wps = xs + CK * kTinRow;     // [kTK][kTinRow] P weights of the chunk, k-major
-  float* wgs = wps + kTK * kTinRow;   // [kTK][kTinRow] G weights
-  float* msk = wgs + kTK * kTinRow;   // [kTinTok] 1 for a valid, unmasked token
-  const int tid = threadIdx.x;
-  const int64_t tpr = ld / kTinTok, rr = blockIdx.x / tpr, r = rr % L, b = rr / L;
-  const int64_t c0 = (blockIdx.x % tpr) * kTinTok;
-  auto token = [&](int t) -> int64_t {  // x / mask index of tile token t (t >= L - c0: position L - 1)
-    int64_t c = c0 + t;
-    c = c < L ? c : L - 1;
-    return transpose ? (b * L + c) * L + r : (b * L + r) * L + c;
-  };
-  for (int e = tid; e < kTinTok * C; e += 256) {  // row-major reads, k-major LDS
-    const int t = e / C, k = e % C;
-    xs[k * kTinRow + t] = (float)x[token(t) * C + k];
-  }
-  if (tid < kTinTok) msk[tid] = c0 + tid < L ? (mask ? (mask[token(tid)] != 0 ? 1.f : 0.f) : 1.f) : 0.f;
-  __syncthreads();
-  tiled_layer_norm<T>(xs, kTinRow, kTinTok, C, CK, eps);
-
-  const int ty = tid >> 4, tx = tid & 15;  // tokens 4 ty .. + 3, chunk features 4 tx .. + 3
-  T* abt = ab + (b * L + r) * ld + c0 + 4 * ty;
-  // (64-feature chunk, 32-deep k-tile) steps in one sequence; each step's P and G weights are
-  // loaded into registers during the previous step and stored k-major into LDS after a barrier
-  const int nk = CK / kTK, nsteps = ((Cout + 63) / 64) * nk;
-  float wr[16];  // P (0-7) and G (8-15) weights (f, k) = (e / kTK, e % kTK), e = tid + 256 i
-  auto wload = [&](int step) __attribute__((always_inline)) {
-    const int f0 = (step / nk) * 64, k0 = (step % nk) * kTK;
+                                                             T* __restrict__ out, uint32_t L, int C, int Cout,
+                                                             uint32_t ldy, int64_t cstride, float eps) {
+  using M = TileMma<T>;
+  using V = typename M::V;
+  constexpr int TT = 32 * NB, TPT = 256 / TT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int rx = tile_row<T>(C), KP = tile_kp(C);
+  T* ys = reinterpret_cast<T*>(smem);  // [TT][rx] LN_out(y)
+  T* xs = ys + TT * rx;                // [TT][rx] LN_in(x)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const uint32_t tpr = (L + TT - 1) / TT, bi = blockIdx.x / tpr, j0 = (blockIdx.x - bi * tpr) * TT;  // bi = b * L + i
+  const int ntok = (int)(L - j0 < (uint32_t)TT ? L - j0 : TT);
+  const int t = tid / TPT, part = tid % TPT;
+  stage_row<T, TPT, VEC>(xs + t * rx, x + ((int64_t)bi * L + j0 + (t < ntok ? t : ntok - 1)) * C, true, part, C, KP);
+  {
+    // y: 16 bytes (VE tokens) of KC channels per thread and step, written as KC-channel pieces of VE token
+    // rows (columns up to ldy exist; those past L are dropped at the end)
+    constexpr int KC = sizeof(T) == 2 ? 2 : 1, G = TT / M::VE, S = 256 / G * KC, U = 2;
+    const T* yr = y + (int64_t)bi * ldy + j0 + tid % G * M::VE;
+    for (int k0 = tid / G * KC; k0 < KP; k0 += U * S) {
+      V v[U][KC];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + 256 * i, ff = f0 + e / kTK, kk = k0 + e % kTK;
-      const bool ok = ff < Cout && kk < C;
-      wr[i] = ok ? (float)Wp[(int64_t)ff * C + kk] : 0.f;
-      wr[8 + i] = ok ? (float)Wg[(int64_t)ff * C + kk] : 0.f;
-    }
-  };
-  wload(0);
-  float ap[4][4] = {}, ag[4][4] = {};
-  for (int step = 0; step < nsteps; ++step) {
-    __syncthreads();  // the previous step's weights are consumed (step 0: the tile is normalised)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = tid + 256 * i;
-      wps[(e % kTK) * kTinRow + e / kTK] = wr[i];
-      wgs[(e % kTK) * kTinRow + e / kTK] = wr[8 + i];
-    }
-    __syncthreads();
-    if (step + 1 < nsteps) wload(step + 1);
-    const int k0 = (step % nk) * kTK;
-#pragma unroll 8
-    for (int k = 0; k < kTK; ++k) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(&xs[(k0 + k) * kTinRow + 4 * ty]);
-      const f32x4 wp = *reinterpret_cast<const f32x4*>(&wps[k * kTinRow + 4 * tx]);
-      const f32x4 wg = *reinterpret_cast<const f32x4*>(&wgs[k * kTinRow + 4 * tx]);
+        for (int j = 0; j < KC; ++j) {
+          const int k = k0 + u * S + j;
+          if constexpr (VEC) {
+            v[u][j] = ldg<V>(yr + (k < C ? k : 0) * cstride);
+            if (k >= C) v[u][j] = V{};
+          } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          ap[u][v] = fmaf(a[u], wp[v], ap[u][v]);
-          ag[u][v] = fmaf(a[u], wg[v], ag[u][v]);
+            for (int e = 0; e < M::VE; ++e) v[u][j][e] = k < C ? yr[k * cstride + e] : (T)0.f;
+          }
         }
-    }
-    if (step % nk != nk - 1) continue;
-    const int f0 = (step / nk) * 64;  // the chunk's last k-tile: bias, gate, mask, store
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int f = f0 + 4 * tx + v;
-      if (f < Cout) {
-        const float bp = Bp[f], bg = Bg[f];
-        vec<T, 4> o;
+      for (int u = 0; u < U; ++u) {
+        if (k0 + u * S >= KP) continue;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) o[u] = (T)((ap[u][v] + bp) * sigmoid(ag[u][v] + bg) * msk[4 * ty + u]);
-        *reinterpret_cast<vec<T, 4>*>(abt + (int64_t)f * fstride) = o;
-      }
+        for (int e = 0; e < M::VE; ++e) {
+          vec<T, KC> p;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) ap[u][v] = ag[u][v] = 0.f;
-    }
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void tmu_gen_out_tiled_kernel(const T* __restrict__ y, const T* __restrict__ x,
-                                                               const T* __restrict__ Wp, const T* __restrict__ Wg,
-                                                               const float* __restrict__ Bp,
-                                                               const float* __restrict__ Bg, const T* __restrict__ res,
-                                                               T* __restrict__ out, int64_t L, int C, int Cout,
-                                                               int64_t ldy, int64_t cstride, float eps) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int CK = (C + kTK - 1) / kTK * kTK;
-  float* ys = sm;                      // [CK][kToutRow]  LN_out(y), k-major
-  float* xs = ys + CK * kToutRow;      // [CK][kToutRow]  LN_in(x)
-  float* wps = xs + CK * kToutRow;     // [kTK][kTFRow]
-  float* wgs = wps + kTK * kTFRow;     // [kTK][kTFRow]
-  const int tid = threadIdx.x;
-  const int64_t tpr = (L + kToutTok - 1) / kToutTok, bi = blockIdx.x / tpr;  // bi = b * L + i
-  const int64_t j0 = (blockIdx.x % tpr) * kToutTok;
-  const int ntok = (int)(L - j0 < kToutTok ? L - j0 : kToutTok);
-  for (int e = tid; e < kToutTok * C; e += 256) {  // y channel-major: 32 consecutive tokens per channel
-    const int k = e / kToutTok, t = e % kToutTok;
-    ys[k * kToutRow + t] = t < ntok ? (float)y[(int64_t)k * cstride + bi * ldy + j0 + t] : 0.f;
-  }
-  for (int e = tid; e < kToutTok * C; e += 256) {  // x token-major
-    const int t = e / C, k = e % C;
-    xs[k * kToutRow + t] = t < ntok ? (float)x[(bi * L + j0 + t) * C + k] : 0.f;
-  }
-  __syncthreads();
-  tiled_layer_norm<T>(ys, kToutRow, kToutTok, C, CK, eps);
-  tiled_layer_norm<T>(xs, kToutRow, kToutTok, C, CK, eps);
-
-  const int ty = tid >> 5, tx = tid & 31;  // tokens 4 ty .. + 3, chunk features 4 tx .. + 3
-  // (128-feature chunk, 32-deep k-tile) steps in one sequence, weights prefetched into registers
-  const int nk = CK / kTK, nsteps = ((Cout + kTF - 1) / kTF) * nk;
-  float wr[32];  // P (0-15) and G (16-31) weights (f, k) = (e / kTK, e % kTK), e = tid + 256 i
-  auto wload = [&](int step) __attribute__((always_inline)) {
-    const int f0 = (step / nk) * kTF, k0 = (step % nk) * kTK;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int e = tid + 256 * i, ff = f0 + e / kTK, kk = k0 + e % kTK;
-      const bool ok = ff < Cout && kk < C;
-      wr[i] = ok ? (float)Wp[(int64_t)ff * C + kk] : 0.f;
-      wr[16 + i] = ok ? (float)Wg[(int64_t)ff * C + kk] : 0.f;
-    }
-  };
-  wload(0);
-  float ap[4][4] = {}, ag[4][4] = {};
-  for (int step = 0; step < nsteps; ++step) {
-    __syncthreads();  // the previous step's weights are consumed (step 0: the tiles are normalised)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int e = tid + 256 * i;
-      wps[(e % kTK) * kTFRow + e / kTK] = wr[i];
-      wgs[(e % kTK) * kTFRow + e / kTK] = wr[16 + i];
-    }
-    __syncthreads();
-    if (step + 1 < nsteps) wload(step + 1);
-    const int k0 = (step % nk) * kTK;
-#pragma unroll 8
-    for (int k = 0; k < kTK; ++k) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(&ys[(k0 + k) * kToutRow + 4 * ty]);
-      const f32x4 g = *reinterpret_cast<const f32x4*>(&xs[(k0 + k) * kToutRow + 4 * ty]);
-      const f32x4 wp = *reinterpret_cast<const f32x4*>(&wps[k * kTFRow + 4 * tx]);
-      const f32x4 wg = *reinterpret_cast<const f32x4*>(&wgs[k * kTFRow + 4 * tx]);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          ap[u][v] = fmaf(a[u], wp[v], ap[u][v]);
-          ag[u][v] = fmaf(g[u], wg[v], ag[u][v]);
+          for (int j = 0; j < KC; ++j) p[j] = v[u][j][e];
+          *reinterpret_cast<vec<T, KC>*>(ys + (tid % G * M::VE + e) * rx + k0 + u * S) = p;
         }
-    }
-    if (step % nk != nk - 1) continue;
-    const int f0 = (step / nk) * kTF;  // the chunk's last k-tile: bias, gate, residual, store
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int t = 4 * ty + u;
-      const int64_t o = (bi * L + j0 + t) * Cout;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int f = f0 + 4 * tx + v;
-        if (t < ntok && f < Cout) {
-          const T rv = (T)((ap[u][v] + Bp[f]) * sigmoid(ag[u][v] + Bg[f]));
-          out[o + f] = res ? (T)((float)res[o + f] + (float)rv) : rv;
-        }
-        ap[u][v] = ag[u][v] = 0.f;
       }
     }
   }
+  __syncthreads();
+  {
+    float mean, rstd;
+    row_stats<T, TPT>(ys + t * rx, part, C, eps, mean, rstd);
+    normalise_row<T, TPT>(ys + t * rx, part, C, mean, rstd, nullptr, nullptr);
+    row_stats<T, TPT>(xs + t * rx, part, C, eps, mean, rstd);
+    normalise_row<T, TPT>(xs + t * rx, part, C, mean, rstd, nullptr, nullptr);
+  }
+  __syncthreads();
+  const int nunits = (Cout + 31) / 32 * (NB / NU);
+  for (int u = wave; u < nunits; u += 4) {
+    const int f0 = 32 * (u / (NB / NU)), t0 = 32 * NU * (u % (NB / NU));
+    const int row = f0 + tile_perm(col), fr = row < Cout ? row : Cout - 1, fl = f0 + 16 * hl;
+    f32x16 ap[1][NU] = {}, ag[1][NU] = {};
+    tile_gemm<T, NU, true, VEC>(ap, ys + t0 * rx, rx, col, Wp + (int64_t)fr * C, C);
+    tile_gemm<T, NU, true, VEC>(ag, xs + t0 * rx, rx, col, Wg + (int64_t)fr * C, C);
+    if (fl >= Cout) continue;
+    const f32x16 bp = load16<float, false>(Bp + fl, Cout - fl), bg = load16<float, false>(Bg + fl, Cout - fl);
+#pragma unroll
+    for (int n = 0; n < NU; ++n) {
+      const int tk = t0 + 32 * n + col;
+      if (tk >= ntok) continue;
+      const int64_t off = ((int64_t)bi * L + j0 + tk) * Cout + fl;
+      auto val = [&](int v) __attribute__((always_inline)) {
+        return (T)((ap[0][n][v] + bp[v]) * sigmoid(ag[0][n][v] + bg[v]));
+      };
+      if (res) {
+        const f32x16 rv = load16<T, VEC>(res + off, Cout - fl);
+        store16<T, VEC>(out + off, Cout - fl,
+                        [&](int v) __attribute__((always_inline)) { return (T)(rv[v] + (float)val(v)); });
+      } else {
+        store16<T, VEC>(out + off, Cout - fl, val);
+      }
+    }
+  }
+}
+
+// Both phases take 64 tokens per block or 32 (`half`, see the callers), and one 32-token tile per unit
+// instead of all where there are fewer chunks of features than waves.
+#define TOPS_TMU_SHAPES(CALL, T, half, Cout, vec)  \
+  do {                                             \
+    if (half) {                                    \
+      if (vec)                                     \
+        CALL(T, 1, 1, true);                       \
+      else                                         \
+        CALL(T, 1, 1, false);                      \
+    } else if ((Cout) <= 96) {                     \
+      if (vec)                                     \
+        CALL(T, 2, 1, true);                       \
+      else                                         \
+        CALL(T, 2, 1, false);                      \
+    } else {                                       \
+      if (vec)                                     \
+        CALL(T, 2, 2, true);                       \
+      else                                         \
+        CALL(T, 2, 2, false);                      \
+    }                                              \
+  } while (0)
+
+template <typename T>
+static int tmu_generic_in_t(const void* x, const void* mask, const void* Wp, const void* Wg, const float* Bp,
+                            const float* Bg, void* ab, int64_t B, int64_t L, int64_t C, int64_t C_out, int64_t ld,
+                            int transpose, float eps, hipStream_t st) {
+  if (B * L == 0) return TOPS_OK;
+  TOPS_REQUIRE(B * L * (ld / 32) < (1LL << 31), "tops_tmu_input_phase: too many tokens");
+  const bool vec = aligned16({x, Wp, Wg, ab}) && C % TileMma<T>::VE == 0;
+  auto lds = [&](int nb, int nu) {
+    return (size_t)(32 * nb * tile_row<T>((int)C) + 4 * 32 * (32 * nu + TileMma<T>::VE)) * sizeof(T) + 32 * nb * 4;
+  };
+#define TOPS_TMU_IN(T, NB, NU, VEC)                                                                                 \
+  do {                                                                                                              \
+    (void)hipFuncSetAttribute((const void*)tmu_generic_in_kernel<T, NB, NU, VEC>,                                   \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds(NB, NU));                        \
+    hipLaunchKernelGGL((tmu_generic_in_kernel<T, NB, NU, VEC>), dim3((unsigned)(B * L * (ld / (32 * NB)))), dim3(256), \
+                       lds(NB, NU), st, (const T*)x, (const int8_t*)mask, (const T*)Wp, (const T*)Wg, Bp, Bg,       \
+                       (T*)ab, (uint32_t)L, (int)C, (int)C_out, (uint32_t)ld, B * L * ld, transpose, eps);           \
+  } while (0)
+  // 64 tokens (each weight row read half as often) unless they do not fit in LDS or, in fp32, give a CU
+  // fewer than 4 blocks: C = 128 fp32 L = 200 (3 per CU) 87 us, 81 with 32; L = 256 91 and 98; bf16 C = 64
+  // L = 256 13.5 and 17.6, L = 128 equal
+  const bool half = lds(2, 2) > 160 * 1024 || (sizeof(T) == 4 && B * L * (ld / 64) < 4 * num_cus());
+  TOPS_TMU_SHAPES(TOPS_TMU_IN, T, half, C_out, vec);
+#undef TOPS_TMU_IN
+  return launched("tops_tmu_input_phase");
+}
+
+template <typename T>
+static int tmu_generic_out_t(const void* y, const void* x, const void* Wp, const void* Wg, const float* Bp,
+                             const float* Bg, const void* res, void* out, int64_t B, int64_t L, int64_t C,
+                             int64_t C_out, int64_t ldy, float eps, hipStream_t st) {
+  if (B * L == 0) return TOPS_OK;
+  TOPS_REQUIRE(B * L * ((L + 31) / 32) < (1LL << 31), "tops_tmu_output_phase: too many tokens");
+  const bool vec = aligned16({y, x, Wp, Wg, res, out}) && multiples_of(TileMma<T>::VE, {C, C_out});
+  auto lds = [&](int nb) { return (size_t)2 * 32 * nb * tile_row<T>((int)C) * sizeof(T); };
+#define TOPS_TMU_OUT(T, NB, NU, VEC)                                                                                \
+  do {                                                                                                              \
+    (void)hipFuncSetAttribute((const void*)tmu_generic_out_kernel<T, NB, NU, VEC>,                                  \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds(NB));                            \
+    hipLaunchKernelGGL((tmu_generic_out_kernel<T, NB, NU, VEC>),                                                     \
+                       dim3((unsigned)(B * L * ((L + 32 * NB - 1) / (32 * NB)))), dim3(256), lds(NB), st, (const T*)y, \
+                       (const T*)x, (const T*)Wp, (const T*)Wg, Bp, Bg, (const T*)res, (T*)out, (uint32_t)L, (int)C, \
+                       (int)C_out, (uint32_t)ldy, B * L * ldy, eps);                                                 \
+  } while (0)
+  // 64 tokens unless they do not fit in LDS or, in fp32, leave a CU room for fewer than 3 blocks: fp32
+  // C = 128 L = 200 62 us, 50 with 32, L = 320 104 and 99; C = 64 L = 512 82 and 104; bf16, bound by the weight
+  // reads sooner, C = 256 L = 300 95 and 118
+  const bool half = lds(2) > 160 * 1024 || (sizeof(T) == 4 && 3 * lds(2) > 160 * 1024);
+  TOPS_TMU_SHAPES(TOPS_TMU_OUT, T, half, C_out, vec);
+#undef TOPS_TMU_OUT
+  return launched("tops_tmu_output_phase");
 }
 
 int tmu_generic_input_phase(const void* x, const void* mask, const void* Wp, const void* Wg, const float* Bp,
@@ -1099,46 +1042,13 @@ int tmu_generic_input_phase(const void* x, const void* mask, const void* Wp, con
   TOPS_REQUIRE(C >= 1 && C <= 1024 && C_out >= 1 && C_out <= 4096,
                "tops_tmu_input_phase: supports C <= 1024, C_out <= 4096 (got %lld, %lld)", (long long)C,
                (long long)C_out);
-  if (C <= 256) {  // tiled kernel
-    const int64_t tiles = B * L * (ld / kTinTok);
-    if (tiles == 0) return TOPS_OK;
-    TOPS_REQUIRE(tiles < (1LL << 31), "tops_tmu_input_phase: too many tokens");
-    const int CK = (int)((C + kTK - 1) / kTK * kTK);
-    const size_t lds = ((size_t)(CK + 2 * kTK) * kTinRow + kTinTok) * sizeof(float);
-    const int64_t fstride = B * L * ld;
-#define TOPS_GEN_IN_T(TT)                                                                                        \
-  do {                                                                                                           \
-    hipFuncSetAttribute((const void*)tmu_gen_in_tiled_kernel<TT>, hipFuncAttributeMaxDynamicSharedMemorySize,    \
-                        (int)lds);                                                                               \
-    hipLaunchKernelGGL((tmu_gen_in_tiled_kernel<TT>), dim3((unsigned)tiles), dim3(256), lds, st, (const TT*)x,     \
-                       (const int8_t*)mask, (const TT*)Wp, (const TT*)Wg, Bp, Bg, (TT*)ab, L, (int)C, (int)C_out, ld, \
-                       fstride, transpose, eps);                                                                  \
-  } while (0)
-    if (dtype == TOPS_DTYPE_BF16)
-      TOPS_GEN_IN_T(__bf16);
-    else if (dtype == TOPS_DTYPE_F16)
-      TOPS_GEN_IN_T(_Float16);
-    else if (dtype == TOPS_DTYPE_F32)
-      TOPS_GEN_IN_T(float);
-    else
-      return fail(TOPS_EUNSUPPORTED, "tops_tmu_input_phase: unsupported dtype code %d", dtype);
-#undef TOPS_GEN_IN_T
-    return launched("tops_tmu_input_phase");
-  }
-  const int64_t blocks = (B * L * L + kGenTok - 1) / kGenTok;
-  if (blocks == 0) return TOPS_OK;
-  const size_t lds = (size_t)kGenTok * C * sizeof(float);
-#define TOPS_GEN_IN(TT)                                                                                            hipLaunchKernelGGL((tmu_generic_in_kernel<TT>), dim3((unsigned)blocks), dim3(256), lds, st, (const TT*)x,                           (const int8_t*)mask, (const TT*)Wp, (const TT*)Wg, Bp, Bg, (TT*)ab, B, L, (int)C, (int)C_out,                      ld, transpose, eps)
   if (dtype == TOPS_DTYPE_BF16)
-    TOPS_GEN_IN(__bf16);
-  else if (dtype == TOPS_DTYPE_F16)
-    TOPS_GEN_IN(_Float16);
-  else if (dtype == TOPS_DTYPE_F32)
-    TOPS_GEN_IN(float);
-  else
-    return fail(TOPS_EUNSUPPORTED, "tops_tmu_input_phase: unsupported dtype code %d", dtype);
-#undef TOPS_GEN_IN
-  return launched("tops_tmu_input_phase");
+    return tmu_generic_in_t<__bf16>(x, mask, Wp, Wg, Bp, Bg, ab, B, L, C, C_out, ld, transpose, eps, st);
+  if (dtype == TOPS_DTYPE_F16)
+    return tmu_generic_in_t<_Float16>(x, mask, Wp, Wg, Bp, Bg, ab, B, L, C, C_out, ld, transpose, eps, st);
+  if (dtype == TOPS_DTYPE_F32)
+    return tmu_generic_in_t<float>(x, mask, Wp, Wg, Bp, Bg, ab, B, L, C, C_out, ld, transpose, eps, st);
+  return fail(TOPS_EUNSUPPORTED, "tops_tmu_input_phase: unsupported dtype code %d", dtype);
 }
 
 int tmu_generic_output_phase(const void* y, const void* x, const void* Wp, const void* Wg, const float* Bp,
@@ -1147,46 +1057,13 @@ int tmu_generic_output_phase(const void* y, const void* x, const void* Wp, const
   TOPS_REQUIRE(C >= 1 && C <= 512 && C_out >= 1 && C_out <= 4096,
                "tops_tmu_output_phase: supports C <= 512, C_out <= 4096 (got %lld, %lld)", (long long)C,
                (long long)C_out);
-  if (C <= 256) {  // tiled kernel
-    const int64_t tiles = B * L * ((L + kToutTok - 1) / kToutTok);
-    if (tiles == 0) return TOPS_OK;
-    TOPS_REQUIRE(tiles < (1LL << 31), "tops_tmu_output_phase: too many tokens");
-    const int CK = (int)((C + kTK - 1) / kTK * kTK);
-    const size_t lds = ((size_t)2 * CK * kToutRow + (size_t)2 * kTK * kTFRow) * sizeof(float);
-    const int64_t cstride = B * L * ldy;
-#define TOPS_GEN_OUT_T(TT)                                                                                       \
-  do {                                                                                                           \
-    hipFuncSetAttribute((const void*)tmu_gen_out_tiled_kernel<TT>, hipFuncAttributeMaxDynamicSharedMemorySize,   \
-                        (int)lds);                                                                               \
-    hipLaunchKernelGGL((tmu_gen_out_tiled_kernel<TT>), dim3((unsigned)tiles), dim3(256), lds, st, (const TT*)y,    \
-                       (const TT*)x, (const TT*)Wp, (const TT*)Wg, Bp, Bg, (const TT*)res, (TT*)out, L, (int)C,    \
-                       (int)C_out, ldy, cstride, eps);                                                            \
-  } while (0)
-    if (dtype == TOPS_DTYPE_BF16)
-      TOPS_GEN_OUT_T(__bf16);
-    else if (dtype == TOPS_DTYPE_F16)
-      TOPS_GEN_OUT_T(_Float16);
-    else if (dtype == TOPS_DTYPE_F32)
-      TOPS_GEN_OUT_T(float);
-    else
-      return fail(TOPS_EUNSUPPORTED, "tops_tmu_output_phase: unsupported dtype code %d", dtype);
-#undef TOPS_GEN_OUT_T
-    return launched("tops_tmu_output_phase");
-  }
-  const int64_t blocks = (B * L * L + kGenTok - 1) / kGenTok;
-  if (blocks == 0) return TOPS_OK;
-  const size_t lds = (size_t)2 * kGenTok * C * sizeof(float);
-#define TOPS_GEN_OUT(TT)                                                                                        hipLaunchKernelGGL((tmu_generic_out_kernel<TT>), dim3((unsigned)blocks), dim3(256), lds, st, (const TT*)y,                      (const TT*)x, (const TT*)Wp, (const TT*)Wg, Bp, Bg, (const TT*)res, (TT*)out, B, L, (int)C, (int)C_out, ldy, eps)
   if (dtype == TOPS_DTYPE_BF16)
-    TOPS_GEN_OUT(__bf16);
-  else if (dtype == TOPS_DTYPE_F16)
-    TOPS_GEN_OUT(_Float16);
-  else if (dtype == TOPS_DTYPE_F32)
-    TOPS_GEN_OUT(float);
-  else
-    return fail(TOPS_EUNSUPPORTED, "tops_tmu_output_phase: unsupported dtype code %d", dtype);
-#undef TOPS_GEN_OUT
-  return launched("tops_tmu_output_phase");
+    return tmu_generic_out_t<__bf16>(y, x, Wp, Wg, Bp, Bg, res, out, B, L, C, C_out, ldy, eps, st);
+  if (dtype == TOPS_DTYPE_F16)
+    return tmu_generic_out_t<_Float16>(y, x, Wp, Wg, Bp, Bg, res, out, B, L, C, C_out, ldy, eps, st);
+  if (dtype == TOPS_DTYPE_F32)
+    return tmu_generic_out_t<float>(y, x, Wp, Wg, Bp, Bg, res, out, B, L, C, C_out, ldy, eps, st);
+  return fail(TOPS_EUNSUPPORTED, "tops_tmu_output_phase: unsupported dtype code %d", dtype);
 }
 
 }  // namespace tops

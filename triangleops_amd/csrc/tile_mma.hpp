@@ -140,38 +140,42 @@ __device__ __attribute__((always_inline)) inline void normalise_row(T* row, int 
   }
 }
 
-// acc[n] += W rows x token rows over k < K: the lane's weight row `w` (row tile_perm(lane % 32) or
+// acc[i][n] += W_i rows x token rows over k < K: the lane's weight row w[i] (row tile_perm(lane % 32) or
 // lane % 32 of a 32-feature chunk, already clamped to a row that exists) as one operand, rows
 // 32 n + trow of the LDS tile as the other.  A_IS_W puts the weights in the A operand (D rows are
 // features, columns tokens); otherwise the tokens.  Weights come straight from L2, PB k-steps ahead in
 // two register sets used in turn: each wave of a block needs other rows, so a pass through LDS would
 // only add barriers.  VEC as in stage_row, for the weight rows; a k-step that ends past K and the ones
 // left over from the batches are taken one at a time.
-template <typename T, int NT, bool A_IS_W, bool VEC, int PB = 4>
-__device__ __attribute__((always_inline)) inline void tile_gemm(f32x16 (&acc)[NT], const T* tile, int rs, int trow,
-                                                                const T* __restrict__ w, int K) {
+template <typename T, int NWT, int NT, bool A_IS_W, bool VEC, int PB>
+__device__ __attribute__((always_inline)) inline void tile_gemm_n(f32x16 (&acc)[NWT][NT], const T* tile, int rs,
+                                                                  int trow, const T* const (&w)[NWT], int K) {
   using M = TileMma<T>;
   using V = typename M::V;
   const int hk = (threadIdx.x >> 5 & 1) * M::VE, nk = (K + M::KS - 1) / M::KS;
   const int nb = VEC ? K / (M::KS * PB) : 0;
   const T* t0 = tile + trow * rs + hk;
-  auto load = [&](V(&r)[PB], int b) __attribute__((always_inline)) {
+  using Set = V[PB][NWT];
+  auto load = [&](Set& r, int b) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < PB; ++j) r[j] = ldg<V>(w + (b * PB + j) * M::KS + hk);
+    for (int j = 0; j < PB; ++j)
+#pragma unroll
+      for (int i = 0; i < NWT; ++i) r[j][i] = ldg<V>(w[i] + (b * PB + j) * M::KS + hk);
   };
-  auto mul = [&](V r, int s) __attribute__((always_inline)) {
+  auto mul = [&](const V(&r)[NWT], int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const V x = *reinterpret_cast<const V*>(t0 + 32 * n * rs + s * M::KS);
-      acc[n] = A_IS_W ? M::mma(r, x, acc[n]) : M::mma(x, r, acc[n]);
+#pragma unroll
+      for (int i = 0; i < NWT; ++i) acc[i][n] = A_IS_W ? M::mma(r[i], x, acc[i][n]) : M::mma(x, r[i], acc[i][n]);
     }
   };
-  auto step = [&](const V(&r)[PB], int b) __attribute__((always_inline)) {
+  auto step = [&](const Set& r, int b) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < PB; ++j) mul(r[j], b * PB + j);
   };
   if (nb > 0) {
-    V wa[PB], wb[PB];
+    Set wa, wb;
     load(wa, 0);
     int b = 0;
     for (; b + 2 < nb; b += 2) {
@@ -190,16 +194,25 @@ __device__ __attribute__((always_inline)) inline void tile_gemm(f32x16 (&acc)[NT
   }
   for (int s = nb * PB; s < nk; ++s) {
     const int k = s * M::KS + hk;
-    V r;
-    if constexpr (VEC) {
-      r = ldg<V>(w + (k < K ? k : 0));
-      if (k >= K) r = V{};
-    } else {
+    V r[NWT];
 #pragma unroll
-      for (int e = 0; e < M::VE; ++e) r[e] = k + e < K ? w[k + e] : (T)0.f;
+    for (int i = 0; i < NWT; ++i) {
+      if constexpr (VEC) {
+        r[i] = ldg<V>(w[i] + (k < K ? k : 0));
+        if (k >= K) r[i] = V{};
+      } else {
+#pragma unroll
+        for (int e = 0; e < M::VE; ++e) r[i][e] = k + e < K ? w[i][k + e] : (T)0.f;
+      }
     }
     mul(r, s);
   }
+}
+template <typename T, int NT, bool A_IS_W, bool VEC, int PB = 4>
+__device__ __attribute__((always_inline)) inline void tile_gemm(f32x16 (&acc)[1][NT], const T* tile, int rs, int trow,
+                                                                const T* w, int K) {
+  const T* const ws[1] = {w};
+  tile_gemm_n<T, 1, NT, A_IS_W, VEC, PB>(acc, tile, rs, trow, ws, K);
 }
 
 // Writes f(v), v = 0..15, to dst[0..15], leaving out elements >= n; VEC: in 16-byte chunks (n a
