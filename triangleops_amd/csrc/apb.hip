@@ -280,6 +280,204 @@ __global__ __launch_bounds__(256, 2) void apb_attn_kernel(const T* __restrict__ 
   }
 }
 
+// Few tokens: a block takes QB queries x 32 keys, as few queries as keep the blocks within the CUs.  A CU
+// reads some 23 GB/s of Z whatever the grid, so the general kernel's 32 x 32 pairs (256 KiB) take a
+// block 11 us alone (M = 128: 14.7 us on 16 CUs for 4 MB); smaller blocks put every CU to work.  The
+// 2 QB pair-bias steps (one query, 16 keys) are shared out over NW waves, SO to each and SH to the head
+// waves 0 .. 3, with all their Z loads issued first.  The head waves first bring their head's Q, K and V
+// into operand layout.  FROM_X: projected in place from the block's X rows (Q^T = Wq . X^T and K^T leave
+// the MFMA in operand layout, V = X . Wv^T likewise), the same products as apb_qkv_kernel's, which then
+// needs no launch; otherwise read and transposed through the matrix core as in the general kernel.
+// Same bits as apb_qkv_kernel + apb_attn_kernel.
+template <typename T, bool FROM_X, int QB, int NW, int SH, int SO>
+__global__ __launch_bounds__(64 * NW) void apb_attn_small_kernel(const T* __restrict__ X, const T* __restrict__ wqkv,
+                                                             const T* __restrict__ Qm, const T* __restrict__ Km,
+                                                             const T* __restrict__ Vm, const T* __restrict__ Z,
+                                                             int64_t sz0, int64_t sz1, const float* __restrict__ Wc,
+                                                             const float* __restrict__ sWc,
+                                                             const float* __restrict__ Bc,
+                                                             const int8_t* __restrict__ mask, T* __restrict__ Og,
+                                                             float* __restrict__ ws, int M, int nsplit, float scale,
+                                                             float eps) {
+  constexpr int C = 128, D = 32, H = 4;
+  static_assert(4 * SH + (NW - 4) * SO == 2 * QB && NW >= 8, "every (query, 16 keys) step of the block");
+  using V8 = vec<T, 8>;
+  using V4 = vec<T, 4>;
+  __shared__ __attribute__((aligned(16))) float bias_s[H][32 * kApbBRow];
+  __shared__ V8 wfrag[2][4][64];  // hi and lo term of the folded weights, MFMA operand order
+  const int qb = blockIdx.x / nsplit, sp = blockIdx.x % nsplit;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, col = lane & 31, l16 = lane & 15, g16 = lane >> 4;
+  const int q0 = qb * QB, k0 = sp * 32;
+  auto zload = [&](int u, V8* za) {
+    int q = q0 + (u >> 1), key = k0 + 16 * (u & 1) + l16;
+    q = q < M ? q : M - 1;
+    key = key < M ? key : M - 1;
+    const T* zr = Z + q * sz0 + key * sz1 + 8 * g16;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) za[s] = ldg<V8>(zr + 32 * s);
+  };
+  auto zbias = [&](int u, const V8* za) {  // as in apb_attn_kernel
+    const vec<T, 2> one = {(T)1.0f, (T)1.0f};
+    float sum = 0.f, sq = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const vec<T, 2> pr = {za[s][e], za[s][e + 1]};
+        sum = Mma<T>::dot2(pr, one, sum);
+        sq = Mma<T>::dot2(pr, pr, sq);
+      }
+    sum += __shfl_xor(sum, 16);
+    sq += __shfl_xor(sq, 16);
+    sum += __shfl_xor(sum, 32);
+    sq += __shfl_xor(sq, 32);
+    const float mean = sum * (1.0f / C);
+    const float var = fmaxf(sq * (1.0f / C) - mean * mean, 0.f);
+    const float rstd = rsqrtf(var + eps);
+    f32x4 acc = {};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = Mma<T>::m16(za[s], wfrag[t][s][lane], acc);
+    const float swc = l16 < H ? sWc[l16] : 0.f, bc = l16 < H ? Bc[l16] : 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float mu = __shfl(mean, 4 * g16 + v);
+      const float rs = __shfl(rstd, 4 * g16 + v);
+      if (l16 < H) bias_s[l16][(u >> 1) * kApbBRow + 16 * (u & 1) + 4 * g16 + v] = rs * (acc[v] - mu * swc) + bc;
+    }
+  };
+  const int mk = k0 + col;
+  const unsigned int kbits =
+      (unsigned int)__ballot(lane < 32 && mk < M && (mask ? (int)mask[mk < M ? mk : M - 1] : 1) != 0);
+  const int h = wave;  // of waves 0 .. 3
+  V8 qop[2], kop[2], vop[2];
+  if (wave >= 4) {
+    V8 z[SO][4];
+    const int u0 = 4 * SH + SO * (wave - 4);
+#pragma unroll
+    for (int i = 0; i < SO; ++i) zload(u0 + i, z[i]);
+    if (wave < 8) {  // [Wc_hi; Wc_lo], one 16-byte fragment of each per thread
+      const int s = wave - 4;
+      V8 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float w = l16 < H ? Wc[l16 * C + 32 * s + 8 * g16 + e] : 0.f;
+        hi[e] = (T)w;
+        lo[e] = (T)(w - (float)hi[e]);
+      }
+      wfrag[0][s][lane] = hi;
+      wfrag[1][s][lane] = lo;
+    }
+    __syncthreads();
+    if (kbits != 0) {
+#pragma unroll
+      for (int i = 0; i < SO; ++i) zbias(u0 + i, z[i]);
+    }
+    __syncthreads();
+    return;
+  }
+  V8 z[SH][4];
+#pragma unroll
+  for (int i = 0; i < SH; ++i) zload(SH * wave + i, z[i]);
+  {
+    const int tq = q0 + col < M ? q0 + col : M - 1, tk = k0 + col < M ? k0 + col : M - 1;
+    f32x16 qa = {}, ka = {}, va = {};
+    if constexpr (FROM_X) {
+      const T* wh = wqkv + (h * 3 * D + col) * C + 8 * hl;
+      const T *xq = X + (int64_t)tq * C + 8 * hl, *xk = X + (int64_t)tk * C + 8 * hl;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const V8 x = ldg<V8>(xk + 16 * s);
+        qa = Mma<T>::m32(ldg<V8>(wh + 16 * s), ldg<V8>(xq + 16 * s), qa);
+        ka = Mma<T>::m32(ldg<V8>(wh + D * C + 16 * s), x, ka);
+        va = Mma<T>::m32(x, ldg<V8>(wh + 2 * D * C + 16 * s), va);
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        V8 eye;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) eye[e] = (T)(16 * s + 8 * hl + e == col ? 1.0f : 0.0f);
+        const int c = 16 * (2 * h + s) + 8 * hl;
+        qa = Mma<T>::m32(eye, ldg<V8>(Qm + (int64_t)tq * C + c), qa);
+        ka = Mma<T>::m32(eye, ldg<V8>(Km + (int64_t)tk * C + c), ka);
+        va = Mma<T>::m32(ldg<V8>(Vm + (int64_t)tk * C + c), eye, va);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        qop[j][e] = (T)(qa[8 * j + e] * scale);
+        kop[j][e] = (T)ka[8 * j + e];
+        vop[j][e] = (T)va[8 * j + e];
+      }
+  }
+  __syncthreads();
+  if (kbits != 0) {
+#pragma unroll
+    for (int i = 0; i < SH; ++i) zbias(SH * wave + i, z[i]);
+  }
+  __syncthreads();
+  // ---- scores, softmax of the 32 keys, P.V for head h (waves 0 .. 3) ----
+  f32x16 o = {};
+  float m = -INFINITY, l = 0.f;
+  if (kbits != 0) {
+    f32x16 s;
+    const float* br = &bias_s[h][col * kApbBRow];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(br + 8 * g + 4 * hl);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * g + e] = b[e];
+    }
+    s = Mma<T>::m32(kop[0], qop[0], s);
+    s = Mma<T>::m32(kop[1], qop[1], s);
+    if (kbits != 0xffffffffu) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (!((kbits >> (8 * (v / 4) + 4 * hl + (v % 4))) & 1u)) s[v] = -INFINITY;
+    }
+    float mt = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) mt = fmaxf(mt, s[v]);
+    m = halves_max(mt);
+    const float nb = -(m == -INFINITY ? 0.f : m) * kLog2e;
+    V8 p[2];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float pv = fast_exp2(fmaf(s[v], kLog2e, nb));
+      l += pv;
+      p[v >> 3][v & 7] = (T)pv;
+    }
+    o = Mma<T>::m32(vop[0], p[0], o);
+    o = Mma<T>::m32(vop[1], p[1], o);
+  }
+  l = halves_sum(l);
+  const int q = q0 + col;
+  if (col >= QB || q >= M) return;
+  if (nsplit == 1) {
+    const float inv = 1.0f / l;
+    T* dst = Og + (int64_t)q * (H * D) + h * D + 4 * hl;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      V4 r = {(T)(o[4 * g] * inv), (T)(o[4 * g + 1] * inv), (T)(o[4 * g + 2] * inv), (T)(o[4 * g + 3] * inv)};
+      stg<V4>(dst + 8 * g, r);
+    }
+  } else {
+    float* wo = ws + ((int64_t)sp * M + q) * (H * D) + h * D + 4 * hl;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) stg<f32x4>(wo + 8 * g, f32x4{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]});
+    if (hl == 0) {
+      float* wml = ws + (int64_t)nsplit * M * (H * D) + (((int64_t)sp * M + q) * H + h) * 2;
+      wml[0] = m;
+      wml[1] = l;
+    }
+  }
+}
+
 // Merge split partials: one thread per (query, head, d).
 template <typename T>
 __global__ __launch_bounds__(256) void apb_combine_kernel(const float* __restrict__ ws, T* __restrict__ Og, int64_t M,
@@ -621,6 +819,37 @@ static int apb_qkv_t(const void* X, const void* wqkv, const void* bq, int qkn, c
   return launched("apb_qkv_kernel");
 }
 
+// Queries per block of apb_attn_small_kernel: the fewest that give every block a CU to itself, 0 where even
+// 32 do not or a block has more than one 32-key step.
+static int apb_small_queries(int64_t M, const ApbSplit& sp) {
+  if (sp.keys_per_split != 32) return 0;
+  for (int qb = 4; qb <= 32; qb *= 2)
+    if ((M + qb - 1) / qb * sp.nsplit <= num_cus()) return qb;
+  return 0;
+}
+
+template <typename T, bool FROM_X>
+static int apb_small_t(int qb, const void* X, const void* wqkv, const void* Q, const void* K, const void* V,
+                       const void* Z, int64_t sz0, int64_t sz1, const float* Wc, const float* sWc, const float* Bc,
+                       const void* mask, void* Og, void* part, int64_t M, int nsplit, float scale, float eps,
+                       hipStream_t st) {
+#define TOPS_APB_SMALL(QB, NW, SH, SO)                                                                                \
+  hipLaunchKernelGGL((apb_attn_small_kernel<T, FROM_X, QB, NW, SH, SO>), dim3((unsigned)((M + QB - 1) / QB * nsplit)), \
+                     dim3(64 * NW), 0, st, (const T*)X, (const T*)wqkv, (const T*)Q, (const T*)K, (const T*)V,         \
+                     (const T*)Z, sz0, sz1, Wc, sWc, Bc, (const int8_t*)mask, (T*)Og, (float*)part, (int)M, nsplit,    \
+                     scale, eps)
+  if (qb == 4)
+    TOPS_APB_SMALL(4, 8, 1, 1);
+  else if (qb == 8)
+    TOPS_APB_SMALL(8, 8, 2, 2);
+  else if (qb == 16)
+    TOPS_APB_SMALL(16, 12, 2, 3);
+  else
+    TOPS_APB_SMALL(32, 16, 1, 5);
+#undef TOPS_APB_SMALL
+  return launched("apb_attn_small_kernel");
+}
+
 // The attention kernel alone: Og when the keys are not split, else the split partials in `part`.
 template <typename T>
 static int apb_attention_core_t(const void* Q, const void* K, const void* V, const void* Z, int64_t sz0, int64_t sz1,
@@ -630,24 +859,47 @@ static int apb_attention_core_t(const void* Q, const void* K, const void* V, con
   const ApbSplit sp = apb_split(M);
   const int64_t qblocks = (M + 31) / 32;
   const int64_t grid = qblocks * sp.nsplit;
+  if (const int qb = apb_small_queries(M, sp))
+    return apb_small_t<T, false>(qb, nullptr, nullptr, Q, K, V, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, sp.nsplit,
+                                 scale, eps, st);
   hipLaunchKernelGGL((apb_attn_kernel<T>), dim3((unsigned)grid), dim3(256), 0, st, (const T*)Q, (const T*)K,
                      (const T*)V, (const T*)Z, sz0, sz1, Wc, sWc, Bc, (const int8_t*)mask, (T*)Og, (float*)part, M,
                      sp.nsplit, sp.keys_per_split, scale, eps);
   return launched("apb_attn_kernel");
 }
 
+// Q / K / V pre-pass and attention from X: Og when the keys are not split, else the partials in `part`
+// (q, k, v: scratch of M x 128 elements each).
 template <typename T>
-static int apb_attention_t(const void* Q, const void* K, const void* V, const void* Z, int64_t sz0, int64_t sz1,
-                           const float* Wc, const float* sWc, const float* Bc, const void* mask, void* Og, void* part,
-                           int64_t M, float scale, float eps, hipStream_t st) {
-  if (M == 0) return TOPS_OK;
+static int apb_from_x_t(const void* X, const void* wqkv, void* q, void* k, void* v, const void* Z, int64_t sz0,
+                        int64_t sz1, const float* Wc, const float* sWc, const float* Bc, const void* mask, void* Og,
+                        void* part, int64_t M, float scale, float eps, hipStream_t st) {
   const ApbSplit sp = apb_split(M);
-  int rc = apb_attention_core_t<T>(Q, K, V, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, scale, eps, st);
-  if (rc != TOPS_OK || sp.nsplit == 1) return rc;
+  if (const int qb = apb_small_queries(M, sp))
+    return apb_small_t<T, true>(qb, X, wqkv, nullptr, nullptr, nullptr, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M,
+                                sp.nsplit, scale, eps, st);
+  const int rc = apb_qkv_t<T>(X, wqkv, nullptr, 0, nullptr, nullptr, nullptr, nullptr, q, k, v, M, scale, eps, st);
+  if (rc != TOPS_OK) return rc;
+  return apb_attention_core_t<T>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, 1.0f, eps, st);
+}
+
+// Merge of the split partials into Og (nothing to do without a split).
+template <typename T>
+static int apb_combine_t(void* Og, const void* part, int64_t M, hipStream_t st) {
+  const ApbSplit sp = apb_split(M);
+  if (M == 0 || sp.nsplit == 1) return TOPS_OK;
   const int64_t n = M * 128;
   hipLaunchKernelGGL((apb_combine_kernel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                      (const float*)part, (T*)Og, M, sp.nsplit);
   return launched("apb_combine_kernel");
+}
+
+template <typename T>
+static int apb_attention_t(const void* Q, const void* K, const void* V, const void* Z, int64_t sz0, int64_t sz1,
+                           const float* Wc, const float* sWc, const float* Bc, const void* mask, void* Og, void* part,
+                           int64_t M, float scale, float eps, hipStream_t st) {
+  const int rc = apb_attention_core_t<T>(Q, K, V, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, scale, eps, st);
+  return rc != TOPS_OK ? rc : apb_combine_t<T>(Og, part, M, st);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -815,15 +1067,11 @@ extern "C" int tops_apb_forward_gated(const void* X, const void* wqkv, const voi
     return tops_gate_out(part, 128, 128, X, 128, 128, nullptr, nullptr, 1e-5f, 0, Wg, bg, Wo, bo, out, M, 1, 128,
                          dtype, stream);
   }
-  if (dtype == TOPS_DTYPE_BF16) {
-    rc = apb_qkv_t<__bf16>(X, wqkv, nullptr, 0, nullptr, nullptr, nullptr, nullptr, q, k, v, M, scale, eps, st);
-    if (rc == TOPS_OK)  // Og unused with a split: the partials go to `part`
-      rc = apb_attention_core_t<__bf16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, 1.0f, eps, st);
+  if (dtype == TOPS_DTYPE_BF16) {  // Og unused with a split: the partials go to `part`
+    rc = apb_from_x_t<__bf16>(X, wqkv, q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, scale, eps, st);
     return rc != TOPS_OK ? rc : apb_merge_gate_t<__bf16>((const float*)part, X, Wg, bg, Wo, bo, res, out, M, sp.nsplit, st);
   }
-  rc = apb_qkv_t<_Float16>(X, wqkv, nullptr, 0, nullptr, nullptr, nullptr, nullptr, q, k, v, M, scale, eps, st);
-  if (rc == TOPS_OK)
-    rc = apb_attention_core_t<_Float16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, 1.0f, eps, st);
+  rc = apb_from_x_t<_Float16>(X, wqkv, q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, scale, eps, st);
   return rc != TOPS_OK ? rc : apb_merge_gate_t<_Float16>((const float*)part, X, Wg, bg, Wo, bo, res, out, M, sp.nsplit, st);
 }
 
@@ -929,17 +1177,12 @@ static int apb_forward_impl(const char* who, const void* X, const void* wqkv, co
   int rc;
   // Og == NULL: the attention's split partials stay in `part` (tops_apb_merge_gate reads them)
   if (dtype == TOPS_DTYPE_BF16) {
-    rc = apb_qkv_t<__bf16>(X, wqkv, nullptr, 0, nullptr, nullptr, nullptr, nullptr, q, k, v, M, scale, eps, st);
-    if (rc != TOPS_OK) return rc;
-    return Og ? apb_attention_t<__bf16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, 1.0f, eps, st)
-              : apb_attention_core_t<__bf16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, 1.0f, eps, st);
+    rc = apb_from_x_t<__bf16>(X, wqkv, q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, scale, eps, st);
+    return rc != TOPS_OK || !Og ? rc : apb_combine_t<__bf16>(Og, part, M, st);
   }
   if (dtype == TOPS_DTYPE_F16) {
-    rc = apb_qkv_t<_Float16>(X, wqkv, nullptr, 0, nullptr, nullptr, nullptr, nullptr, q, k, v, M, scale, eps, st);
-    if (rc != TOPS_OK) return rc;
-    return Og ? apb_attention_t<_Float16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, 1.0f, eps, st)
-              : apb_attention_core_t<_Float16>(q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, nullptr, part, M, 1.0f, eps,
-                                               st);
+    rc = apb_from_x_t<_Float16>(X, wqkv, q, k, v, Z, sz0, sz1, Wc, sWc, Bc, mask, Og, part, M, scale, eps, st);
+    return rc != TOPS_OK || !Og ? rc : apb_combine_t<_Float16>(Og, part, M, st);
   }
   return fail(TOPS_EUNSUPPORTED, "%s: unsupported dtype code %d", who, dtype);
 }
