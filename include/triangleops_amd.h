@@ -188,6 +188,21 @@ int tops_gate_out_generic_residual(const void* o, int64_t so0, int64_t so1, cons
                                    int64_t M2, int64_t Cin, int64_t HD, int64_t Cout, int dtype, void* stream);
 
 /*
+ * tops_gate_out_generic[_residual] (res may be NULL, then sr0 / sr1 are not read; out strided either
+ * way) with a workspace: where tops_gate_generic_workspace_bytes is not 0 (few tokens in one column,
+ * M2 == 1, wide rows, no LayerNorm) and `work` (16-byte aligned, that many bytes) is given, the gate
+ * and the output projection run as two launches whose blocks each read a part of the weights, the
+ * gated activations going through `work`; otherwise as one launch.
+ */
+int64_t tops_gate_generic_workspace_bytes(int64_t M1, int64_t M2, int64_t Cin, int64_t HD, int64_t Cout,
+                                          int apply_ln, int dtype);
+int tops_gate_out_generic_work(const void* o, int64_t so0, int64_t so1, const void* gin, int64_t sg0, int64_t sg1,
+                               const void* w_ln, const void* b_ln, float ln_eps, int apply_ln, const void* Wg,
+                               const void* bg, const void* Wo, const void* bo, const void* res, int64_t sr0,
+                               int64_t sr1, void* out, int64_t sd0, int64_t sd1, void* work, int64_t M1, int64_t M2,
+                               int64_t Cin, int64_t HD, int64_t Cout, int dtype, void* stream);
+
+/*
  * attention_pair_bias core.  Replaces `apb_forward` + `_apb_kernel`
  * (attn_pair_bias/kernel.py:205-257, :24-202).
  *   X      io   (M, C) contiguous, C == 128

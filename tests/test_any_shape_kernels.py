@@ -31,24 +31,25 @@ def _within(out, ref, bound, name):
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("M,Cin,HD,Cout", [(1, 64, 64, 64), (31, 384, 384, 384), (65, 33, 40, 7), (8225, 96, 72, 100),
                                            (8225, 24, 24, 24), (131137, 32, 32, 32), (33, 512, 512, 130)])
-@pytest.mark.parametrize("extras", [False, True])
+@pytest.mark.parametrize("extras", ["", "bias", "ln"])
 def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
-    """extras: LayerNorm of the gate input, both biases, a residual, and rows of o and of the gate input
-    that are column slices of wider tensors (odd strides: element-wise loads)."""
+    """bias: both biases and a residual; ln: also LayerNorm of the gate input, and rows of o and of the
+    gate input that are column slices of wider tensors (odd strides: element-wise loads).  Few tokens with
+    wide rows and no LayerNorm run as two launches."""
     from triangleops_amd.triangle_attn.kernel import _gate_out_generic
 
     g = torch.Generator().manual_seed(M + Cin)
-    pad = 3 if extras else 0
+    pad = 3 if extras == "ln" else 0
     o, gin = _rnd(g, dtype, M, 1, HD + pad), _rnd(g, dtype, M, 1, Cin + pad)
     wg, wo = _rnd(g, dtype, HD, Cin, scale=Cin**-0.5), _rnd(g, dtype, Cout, HD, scale=HD**-0.5)
     bg, bo, res, w_ln, b_ln = (_rnd(g, dtype, *s) if extras else None for s in
                                ((HD,), (Cout,), (M, 1, Cout), (Cin,), (Cin,)))
     dev = [t if t is None else t.to(device) for t in (o, gin, wg, bg, wo, bo, res, w_ln, b_ln)]
     out = _gate_out_generic(dev[0][..., :HD], dev[1][..., :Cin], dev[2], dev[3], dev[4], dev[5],
-                            ln=(dev[7], dev[8], 1e-5) if extras else None, residual=dev[6])
+                            ln=(dev[7], dev[8], 1e-5) if extras == "ln" else None, residual=dev[6])
     od, gd = o[..., :HD].double(), gin[..., :Cin].double()
     slack = 0.0
-    if extras:
+    if extras == "ln":
         gd = torch.nn.functional.layer_norm(gd, (Cin,), w_ln.double(), b_ln.double(), 1e-5).to(dtype).double()
         slack = (gd.abs() + 1e-2) @ wg.double().T.abs() / 4  # the sigmoid's slope; see size below for small values
     z = gd @ wg.double().T + (bg.double() if extras else 0.0)
@@ -99,9 +100,10 @@ def test_tri_prep_any_shape(device, dtype, N, C, H, D, ln):
 
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("M,C,H,D", [(1, 8, 1, 8), (31, 384, 16, 24), (33, 30, 3, 10), (65, 512, 2, 64), (64, 520, 3, 20),
-                                     (40, 1100, 5, 16)])
+                                     (40, 1100, 5, 16), (1000, 40, 16, 24), (1000, 1100, 16, 24)])
 def test_apb_qkv_any_shape(device, dtype, M, C, H, D):
-    """Q / K / V at one, exactly one and several 512-channel stages, odd channel counts and head widths."""
+    """Q / K / V for few tokens (the k range split over a block's waves) and for more (rows staged 512
+    channels at a time), odd channel counts and head widths."""
     from triangleops_amd import _native
     from triangleops_amd._common.dtype import any_shape_dtype_code
 

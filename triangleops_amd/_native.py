@@ -72,6 +72,10 @@ _SIGNATURES = {
         _p, _p, _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _i32, _p,
     ],
     "tops_apb_generic_attention": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _f32, _i32, _p],
+    "tops_gate_out_generic_work": [
+        _p, _i64, _i64, _p, _i64, _i64, _p, _p, _f32, _i32, _p, _p, _p, _p, _p, _i64, _i64, _p, _i64, _i64, _p, _i64,
+        _i64, _i64, _i64, _i64, _i32, _p,
+    ],
     "tops_gate_out_generic": [
         _p, _i64, _i64, _p, _i64, _i64, _p, _p, _f32, _i32, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i32,
         _p,
@@ -82,6 +86,7 @@ _OTHER = {
     "tops_abi_version": ([], ctypes.c_int),
     "tops_apb_workspace_bytes": ([_i64, _i64, _i64], ctypes.c_int64),
     "tops_apb_gated_workspace_bytes": ([_i64, _i64, _i64], ctypes.c_int64),
+    "tops_gate_generic_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64, _i32, _i32], ctypes.c_int64),
 }
 
 EXPORTED = tuple(_SIGNATURES) + tuple(_OTHER)
@@ -142,6 +147,12 @@ def apb_workspace_bytes(M: int, H: int, D: int) -> int:
 def apb_gated_workspace_bytes(M: int, H: int, D: int) -> int:
     lib = _lib if _lib is not None else load()
     return int(lib.tops_apb_gated_workspace_bytes(M, H, D))
+
+
+@functools.lru_cache(maxsize=256)
+def gate_generic_workspace_bytes(M1: int, M2: int, Cin: int, HD: int, Cout: int, apply_ln: int, code: int) -> int:
+    lib = _lib if _lib is not None else load()
+    return int(lib.tops_gate_generic_workspace_bytes(M1, M2, Cin, HD, Cout, apply_ln, code))
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

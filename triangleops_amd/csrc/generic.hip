@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // exponentials and the split of the weights in 16 bits (the same in bf16: 245 -> 44 us).
 // ---------------------------------------------------------------------------------------------
 template <typename T, int DP, int KSPL, bool MASK_INF, bool VEC>
-__global__ __launch_bounds__(256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel(
+__global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel(
     const T* __restrict__ qi_, const T* __restrict__ ki_, const T* __restrict__ vi_, const float* __restrict__ bias,
     const int8_t* __restrict__ mask, int64_t sm0, int64_t sm1, T* __restrict__ out, int64_t so0, int64_t so1, int N,
     int H, int D, float scale) {
@@ -227,14 +227,19 @@ __global__ __launch_bounds__(256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel
   using V = typename M::V;
   constexpr int ND = (DP + 31) / 32;               // 32-channel tiles of O
   constexpr int NQ = DP / M::KS, NV = 16 / M::VE;  // k-steps of q . k, 16-byte pieces of 16 keys
-  constexpr int QB = 128 / KSPL;                          // queries per block
   constexpr float kShift = std::is_same<T, _Float16>::value ? 10.f : 0.f;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hl = lane >> 5, col = lane & 31;
-  const uint32_t nqb = (N + QB - 1) / QB, ih = blockIdx.x / nqb, qb = blockIdx.x - ih * nqb;
+  // consecutive blocks go to the 8 XCDs in turn: XCD x takes the x-th eighth of the work, so the query
+  // tiles of one (row, head) read its keys through one L2
+  uint32_t w = blockIdx.x;
+  if constexpr (KSPL == 1) {
+    const uint32_t per = gridDim.x / 8, x = w % 8, rem = gridDim.x % 8;
+    w = x * per + (x < rem ? x : rem) + w / 8;
+  }
+  const uint32_t nqb = (N + 31) / 32, ih = w / nqb, qb = w - ih * nqb;
   const int i = ih / (uint32_t)H, h = ih - i * H;
-  const int q0 = qb * QB + (KSPL == 1 ? 32 * wave : 0);
-  if (KSPL == 1 && q0 >= N) return;
+  const int q0 = qb * 32;
   // all reads go through buffers of the row's keys and of the tile's bias rows: a lane keeps 32-bit byte
   // offsets (64-bit addresses of every element would take the registers of two more waves per SIMD),
   // and keys past N read 0.  kOut is past any buffer's end.
@@ -394,6 +399,121 @@ __global__ __launch_bounds__(256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel
 }
 
 // ---------------------------------------------------------------------------------------------
+// x . W^T for few tokens: 32 tokens x 32 features per block, the k range split over its 4 waves, both
+// operands straight from memory in operand order with PB k-steps in flight, partial sums added through
+// LDS.  With few tokens a kernel whose blocks read whole weight matrices is bound by what one CU can
+// read (600 tokens, C = HD = C_out = 384: gate and output projection in one launch bf16 20 us, fp32 45; as
+// two launches of this 9 and 14): here a block reads 32 rows.
+// A thread ends up with 4 consecutive features fl .. fl + 3 of token tok: epi(tok, fl, values, count).
+// ---------------------------------------------------------------------------------------------
+template <typename T, bool VEC, typename Epi>
+__device__ __attribute__((always_inline)) inline void few_token_linear(const T* __restrict__ x, int64_t sx,
+                                                                       const T* __restrict__ W, int M, int K, int F,
+                                                                       Epi epi) {
+  using TM = TileMma<T>;
+  using V = typename TM::V;
+  constexpr int PB = 4;
+  __shared__ f32x4 part[4][4][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const int tok0 = blockIdx.x * 32, f0 = blockIdx.y * 32;
+  const int tok = tok0 + col < M ? tok0 + col : M - 1, row = f0 + tile_perm(col);
+  const T* xr = x + tok * sx + hl * TM::VE;
+  const T* wr = W + (int64_t)(row < F ? row : F - 1) * K + hl * TM::VE;
+  const int nk = (K + TM::KS - 1) / TM::KS, per = (nk + 3) / 4, s1 = per * (wave + 1) < nk ? per * (wave + 1) : nk;
+  const int kl = K - hl * TM::VE;  // this lane's k-range
+  auto load = [&](V& r, const T* p, int s) __attribute__((always_inline)) {
+    const int k = s * TM::KS;
+    if constexpr (VEC) {
+      r = ldg<V>(p + (k < kl ? k : -hl * TM::VE));
+      if (k >= kl) r = V{};
+    } else {
+#pragma unroll
+      for (int e = 0; e < TM::VE; ++e) r[e] = k + e < kl ? p[k + e] : (T)0.f;
+    }
+  };
+  f32x16 acc = {};
+  for (int s0 = per * wave; s0 < s1; s0 += PB) {
+    V a[PB], b[PB];
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {  // (past the wave's part: the last k-step again, not used)
+      const int s = s0 + j < s1 ? s0 + j : s1 - 1;
+      load(a[j], wr, s);
+      load(b[j], xr, s);
+    }
+#pragma unroll
+    for (int j = 0; j < PB; ++j)
+      if (s0 + j < s1) acc = TM::mma(a[j], b[j], acc);
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) part[wave][g][lane] = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  __syncthreads();
+  const f32x4 v = (part[0][wave][lane] + part[1][wave][lane]) + (part[2][wave][lane] + part[3][wave][lane]);
+  const int fl = f0 + 16 * hl + 4 * wave;
+  if (tok0 + col < M && fl < F) epi(tok, fl, v, F - fl < 4 ? F - fl : 4);
+}
+
+// Elements p[0 .. 3] as floats (p may be null: zeros; n: those that exist; VEC: n = 4, aligned).
+template <typename T, bool VEC>
+__device__ inline f32x4 load4(const T* p, int n) {
+  f32x4 r = {};
+  if (p) {
+    if constexpr (VEC) {
+      const vec<T, 4> v = ldg<vec<T, 4>>(p);
+      r = f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = e < n ? (float)p[e] : 0.f;
+    }
+  }
+  return r;
+}
+template <typename T, bool VEC>
+__device__ inline void store4(T* p, int n, vec<T, 4> v) {
+  if constexpr (VEC) {
+    *reinterpret_cast<vec<T, 4>*>(p) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < n) p[e] = v[e];
+  }
+}
+
+// y = io(o * sigmoid(gin . Wg^T + bg)), y (M, HD) contiguous.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void gate_act_few_kernel(const T* __restrict__ o, int64_t so, const T* __restrict__ gin,
+                                                          int64_t sg, const T* __restrict__ Wg, const T* __restrict__ bg,
+                                                          T* __restrict__ y, int M, int Cin, int HD) {
+  few_token_linear<T, VEC>(gin, sg, Wg, M, Cin, HD, [&](int tok, int f, f32x4 v, int n) __attribute__((always_inline)) {
+    const f32x4 b = load4<T, VEC>(bg ? bg + f : nullptr, n), ov = load4<T, VEC>(o + tok * so + f, n);
+    vec<T, 4> r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (T)(ov[e] * sigmoid(v[e] + b[e]));
+    store4<T, VEC>(y + (int64_t)tok * HD + f, n, r);
+  });
+}
+
+// out = y . Wo^T + bo, with a residual rounded first as a separate add would see it.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void gate_proj_few_kernel(const T* __restrict__ y, const T* __restrict__ Wo,
+                                                           const T* __restrict__ bo, const T* __restrict__ res,
+                                                           int64_t sr, T* __restrict__ out, int64_t sd, int M, int HD,
+                                                           int Cout) {
+  few_token_linear<T, VEC>(y, HD, Wo, M, HD, Cout, [&](int tok, int f, f32x4 v, int n) __attribute__((always_inline)) {
+    const f32x4 b = load4<T, VEC>(bo ? bo + f : nullptr, n);
+    vec<T, 4> r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (T)(v[e] + b[e]);
+    if (res) {
+      const f32x4 rv = load4<T, VEC>(res + tok * sr + f, n);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = (T)(rv[e] + (float)r[e]);
+    }
+    store4<T, VEC>(out + tok * sd + f, n, r);
+  });
+}
+
+// ---------------------------------------------------------------------------------------------
 // Gate + output projection, any (C_in, HD, C_out): 32 tokens per block of NW waves.  Both input
 // tiles are staged in LDS; each wave takes 32-feature chunks of the two products in turn (weights
 // from L2 as the A operand, tokens as B), so a lane ends up with 16 consecutive features of one
@@ -414,6 +534,7 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
                                                               int64_t sd0, int64_t sd1, int64_t M1, int64_t M2,
                                                               int Cin, int HD, int Cout) {
   constexpr int TT = 32, TPT = 64 * NW / TT;
+  constexpr int PB = sizeof(T) == 4 && NW == 16 ? 2 : 4;  // (fp32, 4 waves: 2 k-steps ahead 7 % slower)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int rg = tile_row<T>(Cin), ry = tile_row<T>(HD);
   T* gs = reinterpret_cast<T*>(smem);  // [TT][rg] gate input (normalised)
@@ -438,7 +559,7 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
   for (int f0 = 32 * wave; f0 < HD; f0 += 32 * NW) {
     const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
     f32x16 acc[1][1] = {};
-    tile_gemm<T, 1, true, VEC>(acc, gs, rg, col, Wg + (int64_t)(row < HD ? row : HD - 1) * Cin, Cin);
+    tile_gemm<T, 1, true, VEC, PB>(acc, gs, rg, col, Wg + (int64_t)(row < HD ? row : HD - 1) * Cin, Cin);
     const f32x16 b = load16<T, VEC>(bg && fl < HD ? bg + fl : nullptr, HD - fl);
     T* y = ys + col * ry + fl;
     store16<T, true>(y, 16, [&](int v) __attribute__((always_inline)) {
@@ -451,7 +572,7 @@ __global__ __launch_bounds__(64 * NW) void gate_generic_kernel(const T* __restri
   for (int f0 = 32 * wave; f0 < Cout; f0 += 32 * NW) {
     const int row = f0 + tile_perm(col), fl = f0 + 16 * hl;
     f32x16 acc[1][1] = {};
-    tile_gemm<T, 1, true, VEC>(acc, ys, ry, col, Wo + (int64_t)(row < Cout ? row : Cout - 1) * HD, HD);
+    tile_gemm<T, 1, true, VEC, PB>(acc, ys, ry, col, Wo + (int64_t)(row < Cout ? row : Cout - 1) * HD, HD);
     if (tok0 + col >= M || fl >= Cout) continue;
     const f32x16 b = load16<T, VEC>(bo ? bo + fl : nullptr, Cout - fl);
     T* dst = out + m1 * sd0 + m2 * sd1 + fl;
@@ -499,13 +620,14 @@ static int generic_attention_t(const char* name, const void* q, const void* k, c
   const int64_t rh = R * H;
   // keys split over the waves while 128-query blocks are fewer than the CUs (80 blocks, 600 tokens x 16
   // heads of 24, bf16: 14 us against 31; 192 blocks, 1500 tokens: 41 against 75; 400 blocks, N = 100 x 4
-  // heads: 13 against 10)
+  // heads: 13 against 10; measured with 4 query tiles per block without the split)
   const bool split = rh * ((N + 127) / 128) < num_cus();
-  const int64_t blocks = rh * (split ? (N + 31) / 32 : (N + 127) / 128);
+  const int64_t blocks = rh * ((N + 31) / 32);
   TOPS_REQUIRE(blocks < (1LL << 31), "%s: too many query blocks", name);
   const bool vec = aligned16({q, k, v, out}) && multiples_of(TileMma<T>::VE, {D, so0, so1});
 #define TOPS_GEN_ATTN(DP, KS, VEC)                                                                                  \
-  hipLaunchKernelGGL((tri_generic_attn_kernel<T, DP, KS, MASK_INF, VEC>), dim3((unsigned)blocks), dim3(256), 0, st, \
+  hipLaunchKernelGGL((tri_generic_attn_kernel<T, DP, KS, MASK_INF, VEC>), dim3((unsigned)blocks),                   \
+                     dim3(KS == 1 ? 64 : 256)        , 0, st,                                                       \
                      (const T*)q, (const T*)k, (const T*)v, bias, (const int8_t*)mask, sm0, sm1, (T*)out, so0, so1,  \
                      (int)N, H, D, scale)
 #define TOPS_GEN_ATTN_V(DP, KS) \
@@ -570,6 +692,36 @@ static int gate_generic_t(const void* o, int64_t so0, int64_t so1, const void* g
   return launched(res ? "tops_gate_out_generic_residual" : "tops_gate_out_generic");
 }
 
+// True where gate and output projection run as two launches of few_token_linear: tokens in one column, no
+// LayerNorm, and weights that one CU would read for longer than a launch takes (bf16 / fp32, 384 / 384 /
+// 384, 600 tokens: 20 / 45 us in one launch, 9 / 14 in two; 2048: 20 / 45 and 16 / 24; 6000: 21 / 47 and
+// 42 / 62; 128 / 128 / 128, 2000 tokens in bf16: 6.2 and 6.8).
+static bool gate_few(int64_t M1, int64_t M2, int64_t Cin, int64_t HD, int64_t Cout, int apply_ln, size_t es) {
+  return M2 == 1 && !apply_ln && (M1 + 31) / 32 <= num_cus() / 4 && (int64_t)es * HD * (Cin + Cout) >= 128 * 1024;
+}
+
+template <typename T>
+static int gate_few_t(const void* o, int64_t so, const void* gin, int64_t sg, const void* Wg, const void* bg,
+                      const void* Wo, const void* bo, const void* res, int64_t sr, void* out, int64_t sd, void* y,
+                      int M, int Cin, int HD, int Cout, hipStream_t st) {
+  constexpr int VE = TileMma<T>::VE;
+  const unsigned mt = (unsigned)((M + 31) / 32);
+  const dim3 g1(mt, (unsigned)((HD + 31) / 32)), g2(mt, (unsigned)((Cout + 31) / 32));
+  if (aligned16({o, gin, Wg, bg, y}) && multiples_of(VE, {so, sg, Cin, HD}))
+    hipLaunchKernelGGL((gate_act_few_kernel<T, true>), g1, dim3(256), 0, st, (const T*)o, so, (const T*)gin, sg,
+                       (const T*)Wg, (const T*)bg, (T*)y, M, Cin, HD);
+  else
+    hipLaunchKernelGGL((gate_act_few_kernel<T, false>), g1, dim3(256), 0, st, (const T*)o, so, (const T*)gin, sg,
+                       (const T*)Wg, (const T*)bg, (T*)y, M, Cin, HD);
+  if (aligned16({y, Wo, bo, res, out}) && multiples_of(VE, {HD, Cout, sr, sd}))
+    hipLaunchKernelGGL((gate_proj_few_kernel<T, true>), g2, dim3(256), 0, st, (const T*)y, (const T*)Wo, (const T*)bo,
+                       (const T*)res, sr, (T*)out, sd, M, HD, Cout);
+  else
+    hipLaunchKernelGGL((gate_proj_few_kernel<T, false>), g2, dim3(256), 0, st, (const T*)y, (const T*)Wo, (const T*)bo,
+                       (const T*)res, sr, (T*)out, sd, M, HD, Cout);
+  return launched("tops_gate_out_generic_work");
+}
+
 // ---------------------------------------------------------------------------------------------
 // attention_pair_bias, any (C_s, C_z, H, D) (attn_pair_bias/kernel.py:205-257):
 //   apb_generic_qkv_kernel   per token m: q / k / v [m][h][d] = X[m] . W (rounded to the I/O type)
@@ -609,6 +761,28 @@ __global__ __launch_bounds__(256) void apb_generic_qkv_kernel(const T* __restric
                    [&](int v) __attribute__((always_inline)) { return acc[0][0][v]; });
 }
 
+// The same for few tokens (pw < 4: element-wise stores).
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void apb_qkv_few_kernel(const T* __restrict__ X, const T* __restrict__ wqkv,
+                                                         T* __restrict__ qo, T* __restrict__ ko, T* __restrict__ vo,
+                                                         int M, int C, int H, int D, int pw) {
+  few_token_linear<T, VEC>(X, C, wqkv, M, C, 3 * H * D, [&](int tok, int f, f32x4 v, int n) __attribute__((always_inline)) {
+    const int64_t row = (int64_t)tok * H * D;
+    auto dst = [&](int fr) __attribute__((always_inline)) {
+      const int h = fr / (3 * D), r = fr - h * 3 * D, which = r / D;
+      const uint64_t aq = (uint64_t)qo, dk = (uint64_t)ko - aq, dv = (uint64_t)vo - aq;
+      return reinterpret_cast<T*>(aq + (which == 1 ? dk : 0) + (which == 2 ? dv : 0)) + row + h * D + (r - which * D);
+    };
+    if (pw >= 4) {
+      store4<T, true>(dst(f), 4, vec<T, 4>{(T)v[0], (T)v[1], (T)v[2], (T)v[3]});
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < n) *dst(f + e) = (T)v[e];
+    }
+  });
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void apb_generic_bias_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
                                                               const float* __restrict__ Wc,
@@ -640,10 +814,10 @@ __global__ __launch_bounds__(256) void apb_generic_bias_kernel(const T* __restri
 // 16-byte chunks 4 j + qd of pair lane % 16, takes the two-pass LayerNorm in registers and feeds the
 // normalised fp32 values to v_mfma_f32_16x16x4_f32 against the fp32 folded weights, which stay in
 // registers over all steps.  The next step's loads are issued before this step's arithmetic.  Bound by
-// the read of Z and the matrix cores together (600 tokens, 16 heads, C_z = 128, bf16: 148 -> 39 us
-// against LDS tiles and FMAs, 2.9 TB/s).
+// the read of Z and the matrix cores together (600 tokens, 16 heads, C_z = 128, bf16: 148 -> 38 us
+// against LDS tiles and FMAs, 3 TB/s).
 template <typename T, int NKC, bool VEC>
-__global__ __launch_bounds__(256) void apb_gen_bias_mma_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
+__global__ __launch_bounds__(256, NKC <= 4 ? 4 : 1) void apb_gen_bias_mma_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
                                                               const float* __restrict__ Wc,
                                                               const float* __restrict__ Bc, float* __restrict__ bias,
                                                               uint32_t M, int Cz, int H, float eps) {
@@ -731,7 +905,18 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
                               int C, int Cz, int H, int D, float eps, hipStream_t st) {
   if (M == 0) return TOPS_OK;
   const int pw = qkv_piece<T>(D, q, k, v);
-  {
+  // few tokens: the other kernel's blocks (128 weight rows each) would reach less than half of the CUs (with
+  // the bias, 128 tokens, C = 384, 16 heads of 24: bf16 19.3 us, fp32 18.2; 18.8 and 13.1 so; at 600 tokens,
+  // 171 blocks, bf16 46.0 and 48.2)
+  if ((M + 31) / 32 * ((3 * H * D + 127) / 128) < num_cus() / 2) {
+    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)((3 * H * D + 31) / 32));
+    if (aligned16({X, wqkv}) && C % TileMma<T>::VE == 0)
+      hipLaunchKernelGGL((apb_qkv_few_kernel<T, true>), grid, dim3(256), 0, st, (const T*)X, (const T*)wqkv, (T*)q,
+                         (T*)k, (T*)v, (int)M, C, H, D, pw);
+    else
+      hipLaunchKernelGGL((apb_qkv_few_kernel<T, false>), grid, dim3(256), 0, st, (const T*)X, (const T*)wqkv, (T*)q,
+                         (T*)k, (T*)v, (int)M, C, H, D, pw);
+  } else {
     const bool vec = aligned16({X, wqkv}) && C % TileMma<T>::VE == 0;
     const size_t lds = (size_t)32 * tile_row<T>(C < kQkvC ? C : kQkvC) * sizeof(T);
     const dim3 grid((unsigned)((M + 31) / 32), (unsigned)((3 * H * D + 127) / 128));
@@ -750,9 +935,11 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
   if (Cz <= 256 && M < 65536) {
     const bool vec = aligned16({Z}) && multiples_of(TileMma<T>::VE, {sz0, sz1, Cz});
     const int64_t steps = (M * M + 63) / 64;  // of 4 waves
-    // 2 blocks per CU: 600 tokens x 16 heads, C_z = 128 in bf16 39 us against 42 with 4 and 52 with 8 (whose
-    // waves take 3 and 1.5 steps each, unevenly), 500 tokens x 2 heads, C_z = 32 equal within 1 us
-    const dim3 grid((unsigned)(steps < 2 * num_cus() ? steps : 2 * num_cus()), (unsigned)((H + 15) / 16));
+    // blocks that a CU holds at once: 4 in 128 registers (up to 4 chunks), 2 with more chunks (fp32, 600 tokens x
+    // 16 heads, C_z = 128: 50 us, 55 with 4 blocks and 65 with 8, whose waves take uneven step counts)
+    constexpr int W = 4 * TileMma<T>::VE;  // channels per chunk of the four lanes
+    const int64_t cap = (Cz <= 4 * W ? 4 : 2) * num_cus();
+    const dim3 grid((unsigned)(steps < cap ? steps : cap), (unsigned)((H + 15) / 16));
 #define TOPS_GEN_BIAS(NKC, VEC)                                                                                     \
   hipLaunchKernelGGL((apb_gen_bias_mma_kernel<T, NKC, VEC>), grid, dim3(256), 0, st, (const T*)Z, sz0, sz1, Wc, Bc, \
                      bias, (uint32_t)M, Cz, H, eps)
@@ -763,7 +950,6 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
     else                        \
       TOPS_GEN_BIAS(NKC, false);\
   } while (0)
-    constexpr int W = 4 * TileMma<T>::VE;  // channels per chunk of the four lanes
     if (Cz <= W)
       TOPS_GEN_BIAS_V(1);
     else if (Cz <= 2 * W)
@@ -1203,4 +1389,40 @@ extern "C" int tops_gate_out_generic_residual(const void* o, int64_t so0, int64_
                (long long)Cin, (long long)HD, (long long)Cout);
   return gate_generic_dispatch(o, so0, so1, gin, sg0, sg1, w_ln, b_ln, ln_eps, apply_ln, Wg, bg, Wo, bo, res, sr0, sr1,
                                out, sd0, sd1, M1, M2, Cin, HD, Cout, dtype, (hipStream_t)stream);
+}
+
+static size_t io_size(int dtype) { return dtype == TOPS_DTYPE_F32 ? 4 : 2; }
+
+extern "C" int64_t tops_gate_generic_workspace_bytes(int64_t M1, int64_t M2, int64_t Cin, int64_t HD, int64_t Cout,
+                                                     int apply_ln, int dtype) {
+  if (M1 <= 0 || M2 <= 0 || !gate_few(M1, M2, Cin, HD, Cout, apply_ln, io_size(dtype))) return 0;
+  return M1 * HD * (int64_t)io_size(dtype);
+}
+
+extern "C" int tops_gate_out_generic_work(const void* o, int64_t so0, int64_t so1, const void* gin, int64_t sg0,
+                                          int64_t sg1, const void* w_ln, const void* b_ln, float ln_eps, int apply_ln,
+                                          const void* Wg, const void* bg, const void* Wo, const void* bo,
+                                          const void* res, int64_t sr0, int64_t sr1, void* out, int64_t sd0,
+                                          int64_t sd1, void* work, int64_t M1, int64_t M2, int64_t Cin, int64_t HD,
+                                          int64_t Cout, int dtype, void* stream) {
+  TOPS_REQUIRE(o && gin && Wg && Wo && out, "tops_gate_out_generic_work: null pointer argument");
+  TOPS_REQUIRE(!apply_ln || w_ln, "tops_gate_out_generic_work: w_ln is required when apply_ln != 0");
+  TOPS_REQUIRE(M1 >= 0 && M2 >= 0, "tops_gate_out_generic_work: bad sizes");
+  TOPS_REQUIRE(Cin >= 1 && HD >= 1 && Cout >= 1 && Cin + HD <= 1024 && Cout <= 4096,
+               "tops_gate_out_generic_work: supports C_in + H*D <= 1024, C_out <= 4096 (got %lld, %lld, %lld)",
+               (long long)Cin, (long long)HD, (long long)Cout);
+  hipStream_t st = (hipStream_t)stream;
+  if (!work || M1 == 0 || !gate_few(M1, M2, Cin, HD, Cout, apply_ln, io_size(dtype)))
+    return gate_generic_dispatch(o, so0, so1, gin, sg0, sg1, w_ln, b_ln, ln_eps, apply_ln, Wg, bg, Wo, bo, res, sr0,
+                                 sr1, out, sd0, sd1, M1, M2, Cin, HD, Cout, dtype, st);
+  if (dtype == TOPS_DTYPE_BF16)
+    return gate_few_t<__bf16>(o, so0, gin, sg0, Wg, bg, Wo, bo, res, sr0, out, sd0, work, (int)M1, (int)Cin, (int)HD,
+                              (int)Cout, st);
+  if (dtype == TOPS_DTYPE_F16)
+    return gate_few_t<_Float16>(o, so0, gin, sg0, Wg, bg, Wo, bo, res, sr0, out, sd0, work, (int)M1, (int)Cin, (int)HD,
+                                (int)Cout, st);
+  if (dtype == TOPS_DTYPE_F32)
+    return gate_few_t<float>(o, so0, gin, sg0, Wg, bg, Wo, bo, res, sr0, out, sd0, work, (int)M1, (int)Cin, (int)HD,
+                             (int)Cout, st);
+  return fail(TOPS_EUNSUPPORTED, "tops_gate_out_generic_work: unsupported dtype code %d", dtype);
 }

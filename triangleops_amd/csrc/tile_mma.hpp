@@ -145,7 +145,8 @@ __device__ __attribute__((always_inline)) inline void normalise_row(T* row, int 
 // 32 n + trow of the LDS tile as the other.  A_IS_W puts the weights in the A operand (D rows are
 // features, columns tokens); otherwise the tokens.  Weights come straight from L2, PB k-steps ahead in
 // two register sets used in turn: each wave of a block needs other rows, so a pass through LDS would
-// only add barriers.  VEC as in stage_row, for the weight rows; a k-step that ends past K and the ones
+// only add barriers.  (fp32: 2 k-steps of 4 MFMAs each cover the latency; 4 cost registers, 2-6 % slower.)  VEC as
+// in stage_row, for the weight rows; a k-step that ends past K and the ones
 // left over from the batches are taken one at a time.
 template <typename T, int NWT, int NT, bool A_IS_W, bool VEC, int PB>
 __device__ __attribute__((always_inline)) inline void tile_gemm_n(f32x16 (&acc)[NWT][NT], const T* tile, int rs,
@@ -208,7 +209,7 @@ __device__ __attribute__((always_inline)) inline void tile_gemm_n(f32x16 (&acc)[
     mul(r, s);
   }
 }
-template <typename T, int NT, bool A_IS_W, bool VEC, int PB = 4>
+template <typename T, int NT, bool A_IS_W, bool VEC, int PB = sizeof(T) == 4 ? 2 : 4>
 __device__ __attribute__((always_inline)) inline void tile_gemm(f32x16 (&acc)[1][NT], const T* tile, int rs, int trow,
                                                                 const T* w, int K) {
   const T* const ws[1] = {w};

@@ -358,11 +358,20 @@ def _gate_out_generic(o, gin, W_g, b_g, W_o, b_o, *, ln=None, residual=None, out
     code = any_shape_dtype_code(o.dtype)
     if residual is None:
         out = torch.empty(N1, N2, Cout, device=o.device, dtype=o.dtype)
+    else:
+        residual, out = _residual_views(o, residual, out, Cout, lambda t: t.stride(2) == 1)
+    nbytes = _native.gate_generic_workspace_bytes(N1, N2, Cin, HD, Cout, 1 if ln is not None else 0, code)
+    if nbytes:  # few tokens, wide rows: two launches with the gated activations in between
+        work = torch.empty(nbytes, device=o.device, dtype=torch.uint8)
+        rs = (0, 0) if residual is None else (residual.stride(0), residual.stride(1))
+        _native.call("tops_gate_out_generic_work", *args, _native.ptr(residual), *rs, out.data_ptr(), out.stride(0),
+                     out.stride(1), work.data_ptr(), N1, N2, Cin, HD, Cout, code, _native.stream_of(o))
+    elif residual is None:
         _native.call("tops_gate_out_generic", *args, out.data_ptr(), N1, N2, Cin, HD, Cout, code, _native.stream_of(o))
-        return out
-    residual, out = _residual_views(o, residual, out, Cout, lambda t: t.stride(2) == 1)
-    _native.call("tops_gate_out_generic_residual", *args, residual.data_ptr(), residual.stride(0), residual.stride(1),
-                 out.data_ptr(), out.stride(0), out.stride(1), N1, N2, Cin, HD, Cout, code, _native.stream_of(o))
+    else:
+        _native.call("tops_gate_out_generic_residual", *args, residual.data_ptr(), residual.stride(0),
+                     residual.stride(1), out.data_ptr(), out.stride(0), out.stride(1), N1, N2, Cin, HD, Cout, code,
+                     _native.stream_of(o))
     return out
 
 
