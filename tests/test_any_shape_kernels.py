@@ -63,6 +63,23 @@ def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
     _within(out, ref, bound, f"gate {dtype} {M} {Cin} {HD} {Cout}")
 
 
+# one launch and two; weights of another dtype, or transposed: the launcher makes copies
+@pytest.mark.parametrize("C", [96, 128, 384])
+@pytest.mark.parametrize("form", ["fp32", "transposed"])
+def test_gate_converted_weights_bitwise(device, C, form):
+    """Weights that the launcher has to convert give the bits of the same weights converted beforehand."""
+    from triangleops_amd.triangle_attn.kernel import gate_out_forward
+
+    dtype = torch.bfloat16
+    g = torch.Generator().manual_seed(C)
+    o, gin, res = (_rnd(g, dtype, 33, 1, C).to(device) for _ in range(3))
+    w = [_rnd(g, dtype, *s).to(device) for s in ((C, C), (C,), (C, C), (C,))]
+    other = [t.float() for t in w] if form == "fp32" else [t.t().contiguous().t() if t.dim() == 2 else t for t in w]
+    assert torch.equal(gate_out_forward(o, gin, *other), gate_out_forward(o, gin, *w))
+    assert torch.equal(gate_out_forward(o, gin, *other, residual=res.float()),
+                       gate_out_forward(o, gin, *w, residual=res))
+
+
 # grids of one token, one short of and past a 32-token tile, a few thousand blocks;
 # head widths of every store width, C of one and several k batches and with a tail
 @pytest.mark.parametrize("dtype", TYPES)

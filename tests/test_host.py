@@ -7,6 +7,7 @@ import os
 import re
 import subprocess
 import sys
+import weakref
 
 import pytest
 import torch
@@ -319,3 +320,91 @@ def test_apb_noalloc_rejects_oversized_call_cpu():
     rc = lib.tops_apb_forward_noalloc(fake, fake, fake, 128 * 65536, 128, fake, fake, fake, None, fake, 65536, 128, 128,
                                       4, 32, 1.0, 1e-5, 2, None)
     assert rc == 1 and b"static workspace" in lib.tops_last_error()
+
+
+def _wrapper_calls():
+    """(name, call) for every launcher that converts operands, each with fp32 or transposed weights next to
+    bf16 activations, so that each converted operand is a copy the launcher alone holds."""
+    from triangleops_amd.attn_pair_bias import kernel as apb
+    from triangleops_amd.triangle_attn import kernel as tri
+    from triangleops_amd.triangle_mul import kernel as tmu
+
+    def io(*s):
+        return torch.zeros(*s, dtype=torch.bfloat16)
+
+    def f32(*s):
+        return torch.zeros(*s)
+
+    def f64(*s):
+        return torch.zeros(*s, dtype=torch.float64)
+
+    def gate(M, N2, c, ln, residual, w):
+        return tri.gate_out_forward(io(M, N2, c), io(M, N2, c), w(c, c), f32(c), w(c, c), f32(c),
+                                    ln=(f32(c), f32(c), 1e-5) if ln else None,
+                                    residual=f32(M, N2, c) if residual else None)
+
+    def flipped(a, b):
+        return io(b, a).t()
+
+    for c, name in ((128, "tuned"), (96, "any shape"), (384, "two launches")):
+        for residual in (False, True):
+            for w in (f32, flipped):
+                yield f"gate {name} {residual} {w.__name__}", (
+                    lambda c=c, r=residual, w=w: gate(33, 1, c, c != 384, r, w))
+    for c in (128, 96):
+        prep = tri.prep_forward if c == 128 else tri.generic_prep_forward
+        yield f"pre-pass {c}", lambda c=c, f=prep: f(io(8, 8, c), f32(c), f32(c), f32(4, 3, 32, c), f32(4, c), f64(4))
+    yield "attention of LN(x)", lambda: tri.triangle_attn_forward(
+        io(8, 8, 96), f32(96, 96), f32(96, 192), f32(3, 96), f64(3), io(8, 8, 96))
+    consts = lambda n: [f64(n) for _ in range(4)]  # noqa: E731
+    for c in (128, 96):
+        yield f"tmu in {c}", lambda c=c: tmu.input_phase(io(1, 8, 8, c), f32(1, 8, 8), f32(2 * c, c), f32(2 * c, c),
+                                                         *consts(2 * c), 1e-5)
+        yield f"tmu out {c}", lambda c=c: tmu.output_phase(io(c, 1, 8, 8), io(1, 8, 8, c), f32(c, c), f32(c, c),
+                                                           *consts(c), 1e-5, residual=f32(1, 8, 8, c))
+    for M in (40, 600):
+        yield f"apb gated {M}", lambda M=M: apb.apb_forward_gated(
+            io(M, 256)[:, :128], io(M, M, 129)[..., :128], f64(4, 128), f64(4), f64(4), f32(4, 3, 32, 128),
+            f32(128, 128), f32(128), f32(128, 128), f32(128), mask=f32(M), residual=f32(M, 128))
+    for c in (128, 96):
+        h = c // 32
+        yield f"apb {c}", lambda c=c, h=h: apb.apb_forward(
+            io(40, 2 * c)[:, :c], f32(c, 3 * c), io(40, 40, c), f64(h, c), f64(h), f64(h), io(40, c), mask=f32(40),
+            wqkv_hm=f32(h, 3, 32, c))
+        yield f"apb qk-norm pre-pass {c}", lambda c=c, h=h: apb.apb_qkn_prep(
+            io(40, 2 * c)[:, :c], f32(h, 3, 32, c), f32(c), tuple(f32(c) for _ in range(4)))
+        yield f"apb given q, k, v {c}", lambda c=c, h=h: apb.apb_forward_qkv(
+            *(io(40, 2 * c)[:, :c] for _ in range(3)), io(40, 40, c), f64(h, c), f64(h), f64(h), io(40, c),
+            mask=f32(40))
+
+
+_WRAPPER_CALLS = dict(_wrapper_calls())
+
+
+@pytest.mark.skipif(not os.path.exists(_native.LIB_PATH), reason="HIP library not built")
+@pytest.mark.parametrize("name", sorted(_WRAPPER_CALLS))
+def test_converted_operands_live_until_the_launch(monkeypatch, name):
+    """A copy that a launcher makes of an operand (another dtype, strides or alignment) is still held, and its
+    memory not handed out again, when the entry point is called with its address."""
+    copies, made, launches = [], [], []
+    dense = _native.dense
+
+    def traced(t, dtype=None):
+        d = dense(t, dtype)
+        if d is not t:
+            copies.append(weakref.ref(d))
+            made.append(d.shape)
+        return d
+
+    def call(entry, *args):
+        launches.append(entry)
+        gone = sum(r() is None for r in copies)
+        assert gone == 0, f"{entry}: {gone} of {len(copies)} converted operands are freed before it is called"
+        copies.clear()
+
+    monkeypatch.setattr(_native, "dense", traced)
+    monkeypatch.setattr(_native, "call", call)
+    monkeypatch.setattr(_native, "check_device", lambda *t: None)
+    monkeypatch.setattr(_native, "stream_of", lambda t: 0)
+    _WRAPPER_CALLS[name]()
+    assert made and launches

@@ -14,9 +14,11 @@ from .. import _native
 from .._common.dtype import any_shape_dtype_code, io_dtype_code
 
 
-def _as(x, t):
-    """A weight or parameter vector as a dense, 16-byte aligned tensor of x's dtype."""
-    return _native.dense(t, x.dtype)
+def _as(x, *ts):
+    """Weights or parameter vectors as dense, 16-byte aligned tensors of x's dtype.  Where one is a copy, the
+    caller's name for it is what keeps its memory: it has to last until the launch that reads it is issued
+    (an allocation in between would be given the same block)."""
+    return tuple(_native.dense(t, x.dtype) for t in ts)
 
 
 def row_stride(N):
@@ -53,17 +55,19 @@ def prep_forward(X, W_ln, B_ln, wqkv, WZ_c, BZ, *, scale=1.0, eps=1e-5, apply_ln
     Qp = torch.empty(N, H, ldn, 32, device=X.device, dtype=X.dtype)
     KV = torch.empty(N, H, ldn // 64, 4096, device=X.device, dtype=X.dtype)
     bias = torch.empty(H, (N + 31) // 32, ldn // 32, 1024, device=X.device, dtype=X.dtype)
+    W_ln, B_ln = _as(X, W_ln, B_ln) if apply_ln else (None, None)
+    wqkv, WZ_c = _as(X, wqkv, WZ_c)
     BZf = None if BZ is None else _native.dense(BZ, torch.float32)
     _native.call(
         "tops_tri_prep",
         X.data_ptr(),
         X.stride(0),
         X.stride(1),
-        _native.ptr(_as(X, W_ln)) if apply_ln else None,
-        _native.ptr(_as(X, B_ln)) if apply_ln else None,
+        _native.ptr(W_ln),
+        _native.ptr(B_ln),
         1 if apply_ln else 0,
-        _as(X, wqkv).data_ptr(),
-        _as(X, WZ_c).data_ptr(),
+        wqkv.data_ptr(),
+        WZ_c.data_ptr(),
         _native.ptr(BZf),
         Qp.data_ptr(),
         KV.data_ptr(),
@@ -112,17 +116,19 @@ def generic_prep_forward(X, W_ln, B_ln, wqkv, WZ_c, BZ, *, eps=1e-5, apply_ln=Tr
     xln = torch.empty(N, N, C, device=X.device, dtype=dt)
     q, k, v = (torch.empty(N, N, H, D, device=X.device, dtype=dt) for _ in range(3))
     bias = torch.empty(H, N, N, device=X.device, dtype=torch.float32)
+    W_ln, B_ln = _as(X, W_ln, B_ln) if apply_ln else (None, None)
+    wqkv, WZ_c = _as(X, wqkv, WZ_c)
     BZf = None if BZ is None else _native.dense(BZ, torch.float32)
     _native.call(
         "tops_tri_generic_prep",
         X.data_ptr(),
         X.stride(0),
         X.stride(1),
-        _native.ptr(_as(X, W_ln)) if apply_ln else None,
-        _native.ptr(_as(X, B_ln)) if apply_ln else None,
+        _native.ptr(W_ln),
+        _native.ptr(B_ln),
         1 if apply_ln else 0,
-        _as(X, wqkv).data_ptr(),
-        _as(X, WZ_c).data_ptr(),
+        wqkv.data_ptr(),
+        WZ_c.data_ptr(),
         _native.ptr(BZf),
         xln.data_ptr(),
         q.data_ptr(),
@@ -274,7 +280,8 @@ def triangle_attn_forward(
     D = WQ_c.shape[1] // H
     assert WKV_c.shape == (C, 2 * H * D)
     assert out.shape == (N, N, H * D)
-    wqkv = wqkv_from_layouts(_as(X_ln, WQ_c), _as(X_ln, WKV_c), H, D, _as(X_ln, WK_c), _as(X_ln, WV_c))
+    WQ_c, WKV_c, WK_c, WV_c = _as(X_ln, WQ_c, WKV_c, WK_c, WV_c)
+    wqkv = wqkv_from_layouts(WQ_c, WKV_c, H, D, WK_c, WV_c)
     if not fast_shape(C, H, D, N=N) or X_ln.dtype == torch.float32:
         xln, q, k, v, bias = generic_prep_forward(X_ln, None, None, wqkv, WZ_c, BZ, apply_ln=False)
         if Bias_buf is not None:
@@ -324,9 +331,10 @@ def gate_out_forward(o, gin, W_g, b_g, W_o, b_o, *, ln=None, residual=None, out=
     eps = 1e-5
     if ln is not None:
         w_ln, b_ln, eps = ln
-    args = [o.data_ptr(), o.stride(0), o.stride(1), gin.data_ptr(), gin.stride(0), gin.stride(1),
-            _native.ptr(_as(o, w_ln)), _native.ptr(_as(o, b_ln)), float(eps), 1 if ln is not None else 0,
-            _as(o, W_g).data_ptr(), _native.ptr(_as(o, b_g)), _as(o, W_o).data_ptr(), _native.ptr(_as(o, b_o))]
+    w_ln, b_ln, W_g, b_g, W_o, b_o = _as(o, w_ln, b_ln, W_g, b_g, W_o, b_o)
+    args = [o.data_ptr(), o.stride(0), o.stride(1), gin.data_ptr(), gin.stride(0), gin.stride(1), _native.ptr(w_ln),
+            _native.ptr(b_ln), float(eps), 1 if ln is not None else 0, W_g.data_ptr(), _native.ptr(b_g),
+            W_o.data_ptr(), _native.ptr(b_o)]
     if residual is None:
         out = torch.empty(N1, N2, C, device=o.device, dtype=o.dtype)
         _native.call("tops_gate_out", *args, out.data_ptr(), N1, N2, C, io_dtype_code(o.dtype), _native.stream_of(o))
@@ -352,9 +360,10 @@ def _gate_out_generic(o, gin, W_g, b_g, W_o, b_o, *, ln=None, residual=None, out
     eps = 1e-5
     if ln is not None:
         w_ln, b_ln, eps = ln
-    args = [o.data_ptr(), o.stride(0), o.stride(1), gin.data_ptr(), gin.stride(0), gin.stride(1),
-            _native.ptr(_as(o, w_ln)), _native.ptr(_as(o, b_ln)), float(eps), 1 if ln is not None else 0,
-            _as(o, W_g).data_ptr(), _native.ptr(_as(o, b_g)), _as(o, W_o).data_ptr(), _native.ptr(_as(o, b_o))]
+    w_ln, b_ln, W_g, b_g, W_o, b_o = _as(o, w_ln, b_ln, W_g, b_g, W_o, b_o)
+    args = [o.data_ptr(), o.stride(0), o.stride(1), gin.data_ptr(), gin.stride(0), gin.stride(1), _native.ptr(w_ln),
+            _native.ptr(b_ln), float(eps), 1 if ln is not None else 0, W_g.data_ptr(), _native.ptr(b_g),
+            W_o.data_ptr(), _native.ptr(b_o)]
     code = any_shape_dtype_code(o.dtype)
     if residual is None:
         out = torch.empty(N1, N2, Cout, device=o.device, dtype=o.dtype)
