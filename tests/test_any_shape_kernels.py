@@ -183,6 +183,46 @@ def test_attention_any_shape(device, dtype, N, H, D, mask):
     _within(out, ref, 0.5 * EPS[dtype] * ref.abs() + EPS[torch.float32] * size + 1e-7, f"{dtype} {N} {H} {D} {mask}")
 
 
+# keys split over the waves (H = 2) and not (H = 8); one and two 32-channel tiles
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("N,H,D", [(40, 2, 24), (40, 8, 24), (40, 2, 64), (40, 8, 64)])
+def test_attention_weights_keep_fp32(device, dtype, N, H, D):
+    """The weights count with fp32's 24 bits, large and small ones alike.  Scores come from the bias alone.
+
+    Rows of even i: V of the first keys is chosen so that the weighted sum cancels to a few units of fp32, each
+    key taking off what the I/O type's rounding left of the ones before.  A weight exp(s - max) with |s| <= 1.4 is
+    off by one unit of exp2 and less than one of its argument's, 2 * 2^-23, and the sums of 4 terms round to less
+    than that again: 2^-21 of the absolute sum, plus the rounding of the result.
+    Rows of odd i: all of an output is one large V under a weight of about e^-18 (a unit of the argument is
+    2^-20 there, and there are two of them)."""
+    from triangleops_amd.triangle_attn.kernel import generic_attention
+
+    g = torch.Generator().manual_seed(N + D)
+    b = torch.rand(H, N, generator=g) * 1.4 - 1.4
+    b[:, 0] = 0.0
+    b[:, 6:] = -18.0 - torch.rand(H, N - 6, generator=g)
+    w = torch.exp(b.double())
+    v = torch.zeros(N, N, H, D, dtype=dtype)
+    acc = torch.zeros(N, H, D, dtype=torch.float64)
+    steps = {torch.bfloat16: 4, torch.float16: 3, torch.float32: 2}[dtype]
+    for k in range(steps):
+        vk = torch.rand(N, H, D, generator=g, dtype=torch.float64) + 1.0 if k == 0 else -acc / w[None, :, k, None]
+        v[:, k] = vk.to(dtype)
+        acc += w[None, :, k, None] * v[:, k].double()
+    v[1::2] = 0.0
+    for d in range(D):
+        v[1::2, 6 + d % (N - 6), :, d] = 6e4
+    q, k = torch.zeros(N, N, H, D, dtype=dtype), _rnd(g, dtype, N, N, H, D)
+    bias = b[:, None, :].expand(H, N, N).contiguous()
+    out = torch.empty(N, N, H * D, device=device, dtype=dtype)
+    generic_attention(*(t.to(device) for t in (q, k, v, bias)), out)
+    p = w / w.sum(-1, keepdim=True)
+    ref = torch.einsum("hk,ikhd->ihd", p, v.double()).reshape(N, 1, H * D)
+    size = torch.einsum("hk,ikhd->ihd", p, v.double().abs()).reshape(N, 1, H * D)
+    ulp = torch.tensor([2.0**-21, 2.0**-18], dtype=torch.float64).repeat(N // 2)[:, None, None]
+    _within(out, ref.expand(out.shape), (0.5 * EPS[dtype] * ref.abs() + ulp * size).expand(out.shape), f"{dtype} {H} {D}")
+
+
 # pairs: one, below and past a 16-pair step, several steps per wave; C_z of every chunk count with tails;
 # one, exactly 16 and more heads
 @pytest.mark.parametrize("dtype", TYPES)

@@ -209,8 +209,10 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // "+ (-1e9)" in fp32 (triangle attention) or -inf (MASK_INF, attention_pair_bias: a row without valid
 // keys gives NaN, as torch's softmax does) and keys >= N left out, online softmax in fp32, and
 // O^T += V^T . P^T with the score registers as the operand.  fp32 I/O runs the fp32 MFMA throughout;
-// with 16-bit I/O the fp32 weights enter as two 16-bit terms (hi + lo, two MFMAs: 16 bits of each
-// weight or more, as fp16 weights are scaled by 2^10 to stay clear of its denormals).
+// with 16-bit I/O each fp32 weight enters as three 16-bit terms that hold all its 24 bits (weight_terms).  Three
+// MFMAs: two terms, 16 to 22 bits, are 1-7 % faster in bf16 and 1-20 % in fp16 and lose weight bits (bf16 / fp16,
+// N = 500, 2 heads of 64: 246 / 244 -> 252 / 274 us; 600 tokens x 16 heads of 24: 11.6 / 12.2 -> 12.0 / 12.7);
+// V and weights converted to the fp32 MFMA, as in fp32 I/O: 392 / 393 and 13.1 / 13.0.
 // K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
 // per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block's
 // 4 waves take 4 query tiles and share the key reads through L1; with KSPL = 4 they take every 4th chunk
@@ -218,6 +220,31 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // of 32: 247 -> 75 us against a query per lane on the VALU, half of the fp32 matrix rate), by the
 // exponentials and the split of the weights in 16 bits (the same in bf16: 245 -> 44 us).
 // ---------------------------------------------------------------------------------------------
+// w[0 .. 15] as three terms of the I/O type that add up to all 24 bits: w = t[0] + (t[1] + t[2] / S) / S.  bf16 has
+// fp32's range: S = 1 and the terms are the first, second and last 8 bits.  fp16 has not: S = 2^11, a term's
+// width, keeps the rests clear of its denormals.
+template <typename T>
+constexpr int kTermScale = std::is_same<T, _Float16>::value ? 1 << 11 : 1;
+template <typename T, typename V, int NV>
+__device__ __attribute__((always_inline)) inline void weight_terms(const f32x16& w, V (&t)[3][NV]) {
+  constexpr int VE = 16 / NV;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    float r = w[v];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if constexpr (std::is_same<T, __bf16>::value) {
+        const uint32_t top = __float_as_uint(r) & 0xffff0000u;
+        t[k][v / VE][v % VE] = __builtin_bit_cast(T, (uint16_t)(top >> 16));
+        r -= __uint_as_float(top);
+      } else {
+        t[k][v / VE][v % VE] = (T)r;
+        r = (r - (float)t[k][v / VE][v % VE]) * kTermScale<T>;
+      }
+    }
+  }
+}
+
 template <typename T, int DP, int KSPL, bool MASK_INF, bool VEC>
 __global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_generic_attn_kernel(
     const T* __restrict__ qi_, const T* __restrict__ ki_, const T* __restrict__ vi_, const float* __restrict__ bias,
@@ -227,7 +254,7 @@ __global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_ge
   using V = typename M::V;
   constexpr int ND = (DP + 31) / 32;               // 32-channel tiles of O
   constexpr int NQ = DP / M::KS, NV = 16 / M::VE;  // k-steps of q . k, 16-byte pieces of 16 keys
-  constexpr float kShift = std::is_same<T, _Float16>::value ? 10.f : 0.f;
+  constexpr float kShift = kTermScale<T> == 1 ? 0.f : 15.f;  // weights up to 2^15: fp16's range, used from the top
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hl = lane >> 5, col = lane & 31;
   // consecutive blocks go to the 8 XCDs in turn: XCD x takes the x-th eighth of the work, so the query
@@ -273,82 +300,101 @@ __global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_ge
     vd[n] = 16 * hl * HDB + (d < D ? d : D - 1) * ES;  // channels past D are computed and not stored
   }
   const uint32_t bd = (uint32_t)(q - q0) * N * 4 + 64 * hl, kd = tile_perm(col) * HDB;
-  f32x16 o[ND] = {};
-  float m = -INFINITY, l = 0.f;
-  const int nch = (N + 31) / 32;
-  int c = KSPL == 1 ? 0 : wave;
-  if (c < nch) load_row(kf, kr, kd + 32 * c * HDB);
-  for (; c < nch; c += KSPL) {
-    const int k0 = 32 * c;
-    // this chunk's V, bias and mask, used after the scores
-    V vf[ND][NV];
-    f32x16 b;
+  f32x16 o[ND];
+  float m, l;
+  const int nch = (N + 31) / 32, c0 = KSPL == 1 ? 0 : wave;
+  auto walk = [&](auto full) __attribute__((always_inline)) {  // full: weights and V enter the products as fp32
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
+    for (int n = 0; n < ND; ++n) o[n] = f32x16{};
+    m = -INFINITY;
+    l = 0.f;
+    if (c0 < nch) load_row(kf, kr, kd + 32 * c0 * HDB);
+    for (int c = c0; c < nch; c += KSPL) {
+      const int k0 = 32 * c;
+      // this chunk's V, bias and mask, used after the scores
+      V vf[ND][NV];
+      f32x16 b;
 #pragma unroll
-      for (int n = 0; n < ND; ++n) vf[n][v / M::VE][v % M::VE] = buffer_load<T>(vr, vd[n] + (k0 + v) * HDB);
-    if (k0 + 32 <= N) {
+      for (int v = 0; v < 16; ++v)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 t = buffer_load<f32x4>(br, bd + k0 * 4 + 16 * g);
+        for (int n = 0; n < ND; ++n) vf[n][v / M::VE][v % M::VE] = buffer_load<T>(vr, vd[n] + (k0 + v) * HDB);
+      if (k0 + 32 <= N) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) b[4 * g + e] = t[e];
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 t = buffer_load<f32x4>(br, bd + k0 * 4 + 16 * g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) b[4 * g + e] = t[e];
+        }
+      } else {  // (past the end of a row: the next row or 0, replaced by -inf below)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) b[v] = buffer_load<float>(br, bd + k0 * 4 + 4 * v);
       }
-    } else {  // (past the end of a row: the next row or 0, replaced by -inf below)
+      const bool in = k0 + col < N;
+      const bool on = in && (!mrow || mrow[(int64_t)(k0 + col) * sm1] != 0);
+      const uint32_t inb = (uint32_t)__builtin_amdgcn_ballot_w64(in), onb = (uint32_t)__builtin_amdgcn_ballot_w64(on);
+      f32x16 s = {};
 #pragma unroll
-      for (int v = 0; v < 16; ++v) b[v] = buffer_load<float>(br, bd + k0 * 4 + 4 * v);
-    }
-    const bool in = k0 + col < N;
-    const bool on = in && (!mrow || mrow[(int64_t)(k0 + col) * sm1] != 0);
-    const uint32_t inb = (uint32_t)__builtin_amdgcn_ballot_w64(in), onb = (uint32_t)__builtin_amdgcn_ballot_w64(on);
-    f32x16 s = {};
+      for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
+      if (c + KSPL < nch) load_row(kf, kr, kd + 32 * (c + KSPL) * HDB);
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
-    if (c + KSPL < nch) load_row(kf, kr, kd + 32 * (c + KSPL) * HDB);
+      for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], scale, b[v]);
+      if (onb != 0xffffffffu) {  // some key is masked or past the end
+        const uint32_t ib = inb >> (16 * hl), ob = onb >> (16 * hl);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], scale, b[v]);
-    if (onb != 0xffffffffu) {  // some key is masked or past the end
-      const uint32_t ib = inb >> (16 * hl), ob = onb >> (16 * hl);
+        for (int v = 0; v < 16; ++v) {
+          s[v] = (ob >> v) & 1 ? s[v] : (MASK_INF ? -INFINITY : s[v] - 1e9f);
+          s[v] = (ib >> v) & 1 ? s[v] : -INFINITY;
+        }
+      }
+      float cm = s[0];
+#pragma unroll
+      for (int v = 1; v < 16; ++v) cm = fmaxf(cm, s[v]);
+      const float mn = fmaxf(m, halves_max(cm));
+      // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
+      // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
+      const float sh = mn == -INFINITY ? 0.f : mn;
+      const float corr = fast_exp2((m - sh) * kLog2e);
+      m = mn;
+      float lc = 0.f;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        s[v] = (ob >> v) & 1 ? s[v] : (MASK_INF ? -INFINITY : s[v] - 1e9f);
-        s[v] = (ib >> v) & 1 ? s[v] : -INFINITY;
+        s[v] = fast_exp2(fmaf(s[v] - sh, kLog2e, kShift));
+        lc += s[v];
+      }
+      // the chunk's sums start at zero and are added to the running ones: a chain over all keys rounds
+      // against the whole sum at every key (fp32, N = 291: 18 % more error than sums over a quarter each)
+      l = fmaf(l, corr, lc);
+      auto add = [&](int n, const f32x16& t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[n][v] = fmaf(o[n][v], corr, t[v]);
+      };
+      if constexpr (!full) {
+        V p[3][NV];
+        weight_terms<T>(s, p);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+          f32x16 t = {};
+#pragma unroll
+          for (int k = 2; k >= 0; --k) {  // the smallest terms first
+#pragma unroll
+            for (int j = 0; j < NV; ++j) t = M::mma(vf[n][j], p[k][j], t);
+            if (k > 0 && kTermScale<T> != 1) t *= 1.f / kTermScale<T>;
+          }
+          add(n, t);
+        }
+      } else {
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+          f32x16 t = {};
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32((float)vf[n][v / M::VE][v % M::VE], s[v], t, 0, 0, 0);
+          add(n, t);
+        }
       }
     }
-    float cm = s[0];
-#pragma unroll
-    for (int v = 1; v < 16; ++v) cm = fmaxf(cm, s[v]);
-    const float mn = fmaxf(m, halves_max(cm));
-    // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
-    // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
-    const float sh = mn == -INFINITY ? 0.f : mn;
-    const float corr = fast_exp2((m - sh) * kLog2e);
-    m = mn;
-    V p[NV], pl[NV];
-    float lc = 0.f;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float w = fast_exp2(fmaf(s[v] - sh, kLog2e, kShift));
-      lc += w;
-      const T hi = (T)w;
-      p[v / M::VE][v % M::VE] = hi;
-      pl[v / M::VE][v % M::VE] = (T)(w - (float)hi);
-    }
-    // the chunk's sums start at zero and are added to the running ones: a chain over all keys rounds
-    // against the whole sum at every key (fp32, N = 291: 18 % more error than sums over a quarter each)
-    l = fmaf(l, corr, lc);
-#pragma unroll
-    for (int n = 0; n < ND; ++n) {
-      f32x16 t = {};
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        t = M::mma(vf[n][j], p[j], t);
-        if constexpr (sizeof(T) == 2) t = M::mma(vf[n][j], pl[j], t);
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) o[n][v] = fmaf(o[n][v], corr, t[v]);
-    }
-  }
+  };
+  walk(std::bool_constant<sizeof(T) == 4>{});
   l = halves_sum(l);
   if constexpr (KSPL == 1) {
     const float inv = 1.f / l;
