@@ -223,6 +223,31 @@ def test_attention_weights_keep_fp32(device, dtype, N, H, D):
     _within(out, ref.expand(out.shape), (0.5 * EPS[dtype] * ref.abs() + ulp * size).expand(out.shape), f"{dtype} {H} {D}")
 
 
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("H,D", [(2, 32), (8, 32), (2, 64), (8, 64)])
+def test_attention_infinities_in_v(device, dtype, H, D):
+    """An infinity or a NaN of V reaches its own channel and no other, as in a plain sum of products."""
+    from triangleops_amd.triangle_attn.kernel import generic_attention
+
+    N, inf = 70, float("inf")
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (_rnd(g, dtype, N, N, H, D) for _ in range(3))
+    bias = _rnd(g, torch.float32, H, N, N)
+    v[3, 0, :, 1], v[3, 69, :, 5], v[3, 40, :, 9] = inf, -inf, float("nan")
+    v[5, 31, :, 0], v[5, 32, :, 0], v[5, 33, 1, 17] = inf, -inf, inf
+    out = torch.empty(N, N, H * D, device=device, dtype=dtype)
+    generic_attention(*(t.to(device) for t in (q, k, v, bias)), out, scale=D**-0.5)
+    s = torch.einsum("iqhd,ikhd->ihqk", q.double(), k.double()) * D**-0.5 + bias.double()
+    vf = v.double().nan_to_num(0.0, 0.0, 0.0)
+    p = torch.softmax(s, -1)
+    ref = torch.einsum("ihqk,ikhd->iqhd", p, vf) + (v.double() - vf).sum(1)[:, None]
+    size = torch.einsum("ihqk,ikhd->iqhd", p, vf.abs())
+    ref, size = ref.reshape(out.shape), size.reshape(out.shape)
+    got, ok = out.double().cpu(), ref.isfinite()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+    _within(got[ok], ref[ok], 0.5 * EPS[dtype] * ref[ok].abs() + EPS[torch.float32] * size[ok] + 1e-7, f"{dtype} {H} {D}")
+
+
 # pairs: one, below and past a 16-pair step, several steps per wave; C_z of every chunk count with tails;
 # one, exactly 16 and more heads
 @pytest.mark.parametrize("dtype", TYPES)

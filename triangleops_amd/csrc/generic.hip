@@ -395,6 +395,16 @@ __global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_ge
     }
   };
   walk(std::bool_constant<sizeof(T) == 4>{});
+  if constexpr (sizeof(T) == 2) {
+    // an infinity of V times a weight's zero term is NaN where the weight itself gives an infinity: a tile with an
+    // element that is not finite is done again in fp32 (twice the time for such a tile; 16 FMAs for the others)
+    float z = 0.f;
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) z = fmaf(o[n][v], 0.f, z);
+    if (__builtin_amdgcn_ballot_w64(z != z) != 0) walk(std::true_type{});
+  }
   l = halves_sum(l);
   if constexpr (KSPL == 1) {
     const float inv = 1.f / l;
