@@ -323,3 +323,22 @@ def test_tmu_phases_any_shape(device, dtype, B, L, C, transpose):
         ref = res.double() + ref
         bound = bound + EPS[dtype] * ref.abs()
     _within(out, ref, bound, f"output phase {dtype} {L} {C}")
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("L,C", [(33, 64), (70, 100), (5, 500)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_tmu_padding_zero_beside_nan(device, dtype, L, C, transpose):
+    """Columns [L, ld) are zero where the last token of a row is NaN, and only its own row's values are NaN."""
+    from triangleops_amd.triangle_mul.kernel import input_phase
+
+    g = torch.Generator().manual_seed(L)
+    x = _rnd(g, dtype, 1, L, L, C)
+    x[0, 2, L - 1], x[0, L - 1, 3, 0] = float("nan"), float("inf")
+    (wp, wg), c = _rnd(g, dtype, 2, C, C), torch.zeros(C, device=device)
+    ab = input_phase(x.to(device), None, wp.to(device), wg.to(device), c, c, c, c, 1e-5, transpose=transpose,
+                     ld=(L + 63) // 64 * 64)
+    assert not ab[..., L:].any()
+    bad = torch.zeros(1, L, L, dtype=torch.bool, device=device)
+    bad[0, 2, L - 1] = bad[0, L - 1, 3] = True
+    assert torch.equal(ab[..., :L].isnan(), (bad.transpose(1, 2) if transpose else bad).expand(C, 1, L, L))

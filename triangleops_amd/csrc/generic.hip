@@ -1066,9 +1066,11 @@ __global__ __launch_bounds__(256, 3) void tmu_generic_in_kernel(const T* __restr
     const uint32_t c = c0 + t < L ? c0 + t : L - 1;
     const int64_t tok = transpose ? ((int64_t)bb * L + c) * L + r : ((int64_t)bb * L + r) * L + c;
     T* row = xs + t * rx;
-    stage_row<T, TPT, VEC>(row, x + tok * C, true, part, C, tile_kp(C));
+    // past L: a row of zeros, normalised by 0 (the values of token L - 1 may not be finite)
+    stage_row<T, TPT, VEC>(row, x + tok * C, c0 + t < L, part, C, tile_kp(C));
     float mean, rstd;
     row_stats<T, TPT>(row, part, C, eps, mean, rstd);
+    if (c0 + t >= L) rstd = 0.f;
     normalise_row<T, TPT>(row, part, C, mean, rstd, nullptr, nullptr);
     if (part == 0) msk[t] = c0 + t < L && (!mask || mask[tok] != 0) ? 1.f : 0.f;
   }
