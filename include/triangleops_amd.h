@@ -216,8 +216,12 @@ int tops_gate_out_generic_work(const void* o, int64_t so0, int64_t so1, const vo
  * Og may be NULL when the keys are split (tops_apb_workspace_bytes exceeds the Q / K / V region):
  * the attention's fp32 split partials then stay in `work` right after Q / K / V, the input of
  * tops_apb_merge_gate.
+ * tops_apb_single_launch: 1 where the Q / K / V pre-pass and the attention of tops_apb_forward[_gated] are
+ * one launch on the current device (few tokens: up to 512 on 256 CUs), else 0.  Then the Q / K / V region
+ * of `work` is not written.
  */
 int64_t tops_apb_workspace_bytes(int64_t M, int64_t H, int64_t D);
+int tops_apb_single_launch(int64_t M, int64_t H, int64_t D);
 int tops_apb_forward(const void* X, const void* wqkv, const void* Z, int64_t sz0, int64_t sz1, const float* Wc,
                      const float* sWc, const float* Bc, const void* mask, void* Og, void* work, int64_t M, int64_t C,
                      int64_t Cz, int64_t H, int64_t D, float scale, float eps, int dtype, void* stream);
@@ -273,8 +277,9 @@ int tops_apb_forward_noalloc(const void* X, const void* wqkv, const void* Z, int
                              void* stream);
 
 /*
- * Q / K / V pre-pass and the attention with given Q / K / V.  tops_apb_forward is the two run
- * back to back (Q scaled by `scale` in the pre-pass, Q / K / V at the head of `work`).  They also
+ * Q / K / V pre-pass and the attention with given Q / K / V.  tops_apb_forward leaves the bits of the two
+ * run back to back (Q scaled by `scale` in the pre-pass, Q / K / V at the head of `work`) and is just that
+ * where tops_apb_single_launch is 0; where it is 1 the attention's blocks project from X.  They also
  * serve the qk-norm variant of attention_pair_bias (the K-Fold formulation the reference states
  * in benchmarks/references.py:230-277 as `torch_attn_pair_bias_qknorm`; the reference has no
  * kernel for it, so these entry points replace that torch function).

@@ -408,3 +408,27 @@ def test_converted_operands_live_until_the_launch(monkeypatch, name):
     monkeypatch.setattr(_native, "stream_of", lambda t: 0)
     _WRAPPER_CALLS[name]()
     assert made and launches
+
+
+@pytest.mark.skipif(not os.path.exists(_native.LIB_PATH), reason="HIP library not built")
+@pytest.mark.parametrize("M", [1, 512, 513, 724, 8200])
+def test_apb_single_launch_decides_the_calls(monkeypatch, M):
+    """The library says up to which M one launch covers the Q / K / V pre-pass and the attention (16 query
+    blocks x 16 key steps on the 256 CUs that it assumes without a GPU); there one call issues everything."""
+    from triangleops_amd.attn_pair_bias import kernel as apb
+
+    lib = _native.load()
+    single = lib.tops_apb_single_launch(M, 4, 32)
+    assert single == (1 if M <= 512 else 0)
+    assert lib.tops_apb_single_launch(0, 4, 32) == 0 and lib.tops_apb_single_launch(M, 8, 32) == 0
+    launches = []
+    monkeypatch.setattr(_native, "call", lambda entry, *args: launches.append(entry))
+    monkeypatch.setattr(_native, "check_device", lambda *t: None)
+    monkeypatch.setattr(_native, "stream_of", lambda t: 0)
+    z = torch.zeros(1, dtype=torch.bfloat16).expand(M, M, 128)
+    monkeypatch.setattr(_native, "vec16", lambda t: t)
+    w, c = torch.zeros(128, 128, dtype=torch.bfloat16), torch.zeros(4)
+    apb.apb_forward_gated(torch.zeros(M, 128, dtype=torch.bfloat16), z, torch.zeros(4, 128), c, c,
+                          torch.zeros(4, 3, 32, 128, dtype=torch.bfloat16), w, None, w, None)
+    assert launches == (["tops_apb_forward_gated"] if single else
+                        ["tops_apb_qkn_prep", "tops_apb_forward_qkv", "tops_apb_merge_gate"])

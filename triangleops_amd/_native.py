@@ -85,6 +85,7 @@ _OTHER = {
     "tops_last_error": ([], ctypes.c_char_p),
     "tops_abi_version": ([], ctypes.c_int),
     "tops_apb_workspace_bytes": ([_i64, _i64, _i64], ctypes.c_int64),
+    "tops_apb_single_launch": ([_i64, _i64, _i64], ctypes.c_int),
     "tops_apb_gated_workspace_bytes": ([_i64, _i64, _i64], ctypes.c_int64),
     "tops_gate_generic_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64, _i32, _i32], ctypes.c_int64),
 }
@@ -141,6 +142,12 @@ def call(name: str, *args) -> None:
 def apb_workspace_bytes(M: int, H: int, D: int) -> int:
     lib = _lib if _lib is not None else load()
     return int(lib.tops_apb_workspace_bytes(M, H, D))
+
+
+@functools.lru_cache(maxsize=256)
+def apb_single_launch(M: int, H: int, D: int) -> bool:
+    lib = _lib if _lib is not None else load()
+    return bool(lib.tops_apb_single_launch(M, H, D))
 
 
 @functools.lru_cache(maxsize=256)

@@ -86,8 +86,9 @@ def gated_ok(X, Z, W_combined, W_g, W_o, residual=None):
 def apb_forward_gated(X, Z, W_combined, sum_W_combined, B_const, wqkv_hm, W_g, b_g, W_o, b_o, *, scale=1.0,
                       eps=1e-5, mask=None, residual=None):
     """out = ((Og * sigmoid(X W_g^T + b_g)) -> io) W_o^T + b_o (+ residual), Og = apb_forward(...):
-    the attention with the gate and output projection of attn_pair_bias/module.py:69-70 fused
-    (tops_apb_forward_gated).  Requires gated_ok(...); returns (M, 128)."""
+    the attention with the gate and output projection of attn_pair_bias/module.py:69-70 fused.  Few tokens,
+    or keys that are not split: tops_apb_forward_gated.  More: its launches as three calls, tops_apb_qkn_prep,
+    tops_apb_forward_qkv (Og = NULL) and tops_apb_merge_gate.  Requires gated_ok(...); returns (M, 128)."""
     assert gated_ok(X, Z, W_combined, W_g, W_o, residual) and wqkv_hm.shape[2] == 32
     return gated_forward(X, Z, W_combined, sum_W_combined, B_const, wqkv_hm, W_g, b_g, W_o, b_o, scale, eps, mask,
                          residual)
@@ -100,22 +101,19 @@ def _dense_as(t, dt):
     return _native.dense(t, dt)
 
 
-# Up to here the Q / K / V pre-pass is part of the attention's launch and the kernels take about as long as
-# their calls (M = 128: 16 us of GPU time); beyond, three C calls start the first kernel sooner.
-SINGLE_CALL_MAX_M = 512
-
-
 def gated_forward(X, Z, Wc, sWc, Bc, wqkv_hm, W_g, b_g, W_o, b_o, scale, eps, mask, residual):
-    """apb_forward_gated after gated_ok(...) has been established by the caller.  Few tokens: one C call that
-    issues every launch.  More: everything the first launch reads is checked and prepared before it, the
-    gate's operands (W_g, b_g, W_o, b_o, residual) while the attention runs."""
+    """apb_forward_gated after gated_ok(...) has been established by the caller.  Where the Q / K / V pre-pass is
+    part of the attention's launch (few tokens), the kernels take about as long as their calls (M = 128: 16 us
+    of GPU time), so one C call issues every launch.  Beyond, three C calls start the first kernel sooner:
+    everything it reads is checked and prepared before it, the gate's operands (W_g, b_g, W_o, b_o, residual)
+    while the attention runs."""
     M = X.shape[0]
     dt = X.dtype
     code = io_dtype_code(dt)
     f32 = torch.float32
     nqkv = (3 * M * 4 * 32 * 2 + 255) // 256 * 256
     nbytes = _native.apb_workspace_bytes(M, 4, 32)
-    if M > SINGLE_CALL_MAX_M and nbytes > nqkv:
+    if nbytes > nqkv and not _native.apb_single_launch(M, 4, 32):
         # split keys: three launches, each issued once its own operands are checked, the next one's
         # prepared while the previous runs: the Q / K / V pre-pass (tops_apb_qkn_prep without Q bias
         # or norm runs tops_apb_forward's first kernel), the attention (tops_apb_forward_qkv with

@@ -5,7 +5,8 @@ Drop-in for `triangle_ops/attn_pair_bias/module.py` of the reference: same `prec
 B_const), plus `wqkv_hm` (the head-major weight the kernel loads).  Three launches per call at the
 tuned shape (C_s = C_z = C_out = 128, H = 4, D = 32): the Q / K / V pre-pass, the LN(Z) bias +
 attention kernel, and the split merge fused with the gate + W_o (tops_apb_forward_gated; the gate
-kernel itself when the keys are not split); up to 512 tokens the first two are one; other shapes run `apb_forward` then the gate.
+kernel itself when the keys are not split).  With few tokens (up to 512 on 256 CUs) the first two are
+one launch.  Other shapes run `apb_forward` then the gate.
 
 Additive extension: `forward(..., mask=None)` / `attention_pair_bias(..., mask=None)` take an
 optional (M,) key mask (masked keys -> -inf, as the reference's K-Fold variant does at

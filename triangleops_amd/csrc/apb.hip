@@ -1,6 +1,7 @@
 // attention_pair_bias core on gfx950.
 //
-// Two kernels (three when the key range is split):
+// Few tokens (apb_small_queries: up to 512 on 256 CUs): apb_attn_small_kernel, the two kernels below in one
+// launch of smaller blocks.  Otherwise two kernels.  Either way one more where the key range is split:
 //   apb_qkv_kernel: Q = X.Wq^T (+ b_q, scaled), K = X.Wk^T, V = X.Wv^T for all M tokens once,
 //     (M, H*D) rows each, 32 tokens per block and one wave per head (MFMA, fp32 accumulation);
 //     the qk-norm variant (benchmarks/references.py:230-277) also takes the Q bias and a
@@ -1032,6 +1033,10 @@ static int apb_merge_gate_t(const float* part, const void* X, const void* Wg, co
     hipLaunchKernelGGL((apb_merge_gate_kernel<T, false>), dim3((unsigned)blocks), dim3(256), 0, st, part, (const T*)X,
                        (const T*)Wg, (const T*)bg, (const T*)Wo, (const T*)bo, (const T*)res, (T*)out, M, nsplit);
   return launched("apb_merge_gate_kernel");
+}
+
+extern "C" int tops_apb_single_launch(int64_t M, int64_t H, int64_t D) {
+  return M > 0 && H == 4 && D == 32 && apb_small_queries(M, apb_split(M)) != 0;
 }
 
 extern "C" int tops_apb_forward_gated(const void* X, const void* wqkv, const void* Z, int64_t sz0, int64_t sz1,
