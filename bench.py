@@ -411,16 +411,19 @@ def tri_work(N, c=C, h=H, dh=D):
 
 
 def apb_phases(d, pre):
-    """forward()'s three launches at the tuned shape (tops_apb_forward_gated), each as its own call on
-    the same workspace layout: the Q / K / V pre-pass (apb_qkv_kernel, which tops_apb_qkn_prep runs
-    at the tuned shape without a Q bias or qk-norm, exactly as the fused call does), the attention
-    kernel alone (tops_apb_forward_qkv with Og = NULL leaves the split partials in the workspace),
-    then the split merge fused with the gate and W_o (tops_apb_merge_gate)."""
+    """forward()'s launches at the tuned shape (tops_apb_forward_gated), each as its own call on the same
+    workspace layout: the Q / K / V pre-pass (apb_qkv_kernel, which tops_apb_qkn_prep runs at the tuned
+    shape without a Q bias or qk-norm), the attention kernel alone (tops_apb_forward_qkv with Og = NULL
+    leaves the split partials in the workspace), then the split merge fused with the gate and W_o
+    (tops_apb_merge_gate).  With few tokens (_native.apb_single_launch) the attention's launch contains the
+    pre-pass (tops_apb_forward with Og = NULL) and there are two phases."""
     st = {}
     M = d["X"].shape[0]
     dev, dt = d["X"].device, d["X"].dtype
     m8 = d["mask"].view(torch.int8) if d["mask"].dtype == torch.bool else d["mask"]
     work = torch.empty(max(_native.apb_workspace_bytes(M, H, D), 1), device=dev, dtype=torch.uint8)
+    single = _native.apb_single_launch(M, H, D)
+    part = work.data_ptr() + (apb_qkv_bytes(M) if single else 0)
     Wc, sWc, Bc = (pre[k].float().contiguous() for k in ("W_combined", "sum_W_combined", "B_const"))
     wg, bg, wo, bo = (d[k].to(dt).contiguous() for k in ("W_proj_g", "B_proj_g", "W_proj_o", "B_proj_o"))
     out = torch.empty(M, C, device=dev, dtype=dt)
@@ -435,20 +438,33 @@ def apb_phases(d, pre):
                      d["Z"].stride(0), d["Z"].stride(1), Wc.data_ptr(), sWc.data_ptr(), Bc.data_ptr(), m8.data_ptr(),
                      None, work.data_ptr(), M, H * D, C, H, D, 1.0, 1e-5, code, _native.stream_of(q))
 
+    def p_from_x():
+        _native.call("tops_apb_forward", d["X"].data_ptr(), pre["wqkv_hm"].data_ptr(), d["Z"].data_ptr(),
+                     d["Z"].stride(0), d["Z"].stride(1), Wc.data_ptr(), sWc.data_ptr(), Bc.data_ptr(), m8.data_ptr(),
+                     None, work.data_ptr(), M, C, C, H, D, D**-0.5, 1e-5, code, _native.stream_of(d["X"]))
+
     def p_mg():
-        _native.call("tops_apb_merge_gate", work.data_ptr(), d["X"].data_ptr(), wg.data_ptr(), bg.data_ptr(),
+        _native.call("tops_apb_merge_gate", part, d["X"].data_ptr(), wg.data_ptr(), bg.data_ptr(),
                      wo.data_ptr(), bo.data_ptr(), None, out.data_ptr(), M, H, D, code, _native.stream_of(out))
         st["out"] = out
 
-    return [p_qkv, p_att, p_mg]
+    return [p_from_x, p_mg] if single else [p_qkv, p_att, p_mg]
+
+
+def apb_qkv_bytes(M):
+    """Bytes of the workspace's Q / K / V region, after which the split partials start."""
+    return (3 * M * H * D * 2 + 255) // 256 * 256
 
 
 def apb_work(M):
-    """apb_attention: Z read once (2 M^2 C bytes) by apb_attn_kernel; apb_merge_gate reads the split
-    partials (nsplit M H (D + 2) fp32) and X and writes the output."""
-    part = _native.apb_workspace_bytes(M, H, D) - ((3 * M * H * D * 2 + 255) // 256 * 256)
-    return {"apb_qkv": ("hbm", 2 * M * C + 3 * 2 * M * H * D), "apb_attention": ("hbm", 2 * M * M * C),
+    """apb_attention: Z read once (2 M^2 C bytes); apb_merge_gate reads the split partials (nsplit M H (D + 2)
+    fp32) and X and writes the output.  One entry per phase of apb_phases."""
+    part = _native.apb_workspace_bytes(M, H, D) - apb_qkv_bytes(M)
+    work = {"apb_qkv": ("hbm", 2 * M * C + 3 * 2 * M * H * D), "apb_attention": ("hbm", 2 * M * M * C),
             "apb_merge_gate": ("hbm", part + 2 * 2 * M * C)}
+    if _native.apb_single_launch(M, H, D):
+        del work["apb_qkv"]
+    return work
 
 
 def apb_qkn_phases(d, pre, p):
