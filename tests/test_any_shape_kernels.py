@@ -1,8 +1,12 @@
 """The any-shape kernels at the edges of their tiles, against float64 with the same rounding points.
 
-Bounds: eps is one unit in the last place of the I/O type (relative); an operand rounded to the I/O
-type may fall on the neighbouring value, so a product over it may differ by eps times its absolute
-sum, and the result is rounded once more.
+Bounds: with 16-bit I/O, EPS is one unit in the last place of the type (relative): an operand rounded to
+it may fall on the neighbouring value, so a product over it may differ by EPS times its absolute sum, and
+the result is rounded once more.  Nothing is rounded in fp32 but the sums: each addition is off by up to
+2^-24 of its partial sum, and EPS, 2^-18, is the worst element with 64 of them all to one side, over sums of
+up to 1100 products.  Over all elements such errors have no common sign: the 2-norm of what an fp32 result
+is off by stays within one unit in the last place, 2^-23, of that of the absolute sums (the largest here is
+2/3 of it, in the attention, and 0.3 of it elsewhere).
 """
 
 import pytest
@@ -20,17 +24,22 @@ def _rnd(g, dtype, *shape, scale=1.0):
     return (torch.randn(*shape, generator=g, dtype=torch.float64) * scale).to(dtype)
 
 
-def _within(out, ref, bound, name):
+def _within(out, ref, bound, name, eps=EPS[torch.float32]):
+    """Every element within `bound`; fp32 results also in the 2-norm, where bound / eps is the absolute sums."""
     d = (out.double().cpu() - ref).abs()
     worst = (d / bound).max().item()
     assert worst <= 1.0, f"{name}: {worst:.2f} of the bound, max |d| {d.max().item():.2e}"
+    if out.dtype == torch.float32:
+        norm = (d.norm() / bound.norm()).item() * eps
+        assert norm <= 2.0**-23, f"{name}: 2-norm {norm * 2**23:.2f} units in the last place of the absolute sums"
 
 
 # tokens: one, one short of and past a 32-token tile and past two, past the one-tile-per-CU rule
 # (32 * 256 tokens), and thousands of blocks
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("M,Cin,HD,Cout", [(1, 64, 64, 64), (31, 384, 384, 384), (65, 33, 40, 7), (8225, 96, 72, 100),
-                                           (8225, 24, 24, 24), (131137, 32, 32, 32), (33, 512, 512, 130)])
+                                           (8225, 24, 24, 24), (131137, 32, 32, 32), (33, 512, 512, 130),
+                                           (33, 387, 390, 384)])
 @pytest.mark.parametrize("extras", ["", "bias", "ln"])
 def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
     """bias: both biases and a residual; ln: also LayerNorm of the gate input, and rows of o and of the
@@ -61,6 +70,40 @@ def test_gate_any_shape(device, dtype, M, Cin, HD, Cout, extras):
         ref = res.double() + ref
         bound = bound + EPS[dtype] * ref.abs()
     _within(out, ref, bound, f"gate {dtype} {M} {Cin} {HD} {Cout}")
+
+
+# few tokens with wide rows, the two launches' 16-byte and element-wise forms: rows that are column slices of
+# wider tensors, a residual and a destination with strides of their own (a transposed view's, odd, in place)
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("M,Cin,HD,Cout", [(33, 384, 384, 384), (70, 400, 392, 500), (33, 387, 390, 386)])
+@pytest.mark.parametrize("pad", [0, 3, 8])
+def test_gate_few_tokens_strided(device, dtype, M, Cin, HD, Cout, pad):
+    from triangleops_amd import _native
+    from triangleops_amd._common.dtype import any_shape_dtype_code
+    from triangleops_amd.triangle_attn.kernel import gate_out_forward
+
+    assert _native.gate_generic_workspace_bytes(M, 1, Cin, HD, Cout, 0, any_shape_dtype_code(dtype)) > 0
+    g = torch.Generator().manual_seed(M + pad)
+    o, gin, res = (_rnd(g, dtype, M, 1, c + pad) for c in (HD, Cin, Cout))
+    wg, wo, bg, bo = (_rnd(g, dtype, *s) for s in ((HD, Cin), (Cout, HD), (HD,), (Cout,)))
+    wg, wo = wg * Cin**-0.5, wo * HD**-0.5
+    od, gd, rd, *w = (t.to(device) for t in (o, gin, res, wg, bg, wo, bo))
+    big = torch.full((M, 3, Cout + 2 * pad), 7.0, device=device, dtype=dtype)
+    dst = big[:, 1:2, pad:pad + Cout]
+    out = gate_out_forward(od[..., :HD], gd[..., :Cin], *w, residual=rd[..., :Cout], out=dst)
+    assert out.data_ptr() == dst.data_ptr()
+    y = (o[..., :HD].double() * torch.sigmoid(gin[..., :Cin].double() @ wg.double().T + bg.double())).to(dtype).double()
+    ref = y @ wo.double().T + bo.double()
+    bound = EPS[dtype] * (ref.abs() + y.abs() @ wo.double().T.abs() + 1e-3)
+    ref = res[..., :Cout].double() + ref
+    _within(out, ref, bound + EPS[dtype] * ref.abs(), f"{dtype} {M} {Cin} {HD} {Cout} {pad}")
+    rest = torch.ones_like(big, dtype=torch.bool)
+    rest[:, 1:2, pad:pad + Cout] = False
+    assert (big[rest] == 7.0).all()
+    alone = gate_out_forward(od[..., :HD], gd[..., :Cin], *w, residual=rd[..., :Cout])
+    inplace = rd.clone()[..., :Cout]
+    gate_out_forward(od[..., :HD], gd[..., :Cin], *w, residual=inplace, out=inplace)
+    assert torch.equal(alone, out) and torch.equal(inplace, alone)
 
 
 # one launch and two; weights of another dtype, or transposed: the launcher makes copies
@@ -139,11 +182,11 @@ def test_apb_qkv_any_shape(device, dtype, M, C, H, D):
         _within(out[i], ref, EPS[dtype] * (ref.abs() + x.double().abs() @ wi.abs().T + 1e-3), name)
 
 
-# key chunks of 32: one key, one chunk less one, one, one more, several; 128-query blocks; D at and below
-# 32 and 64, with and without 16-byte rows; few blocks (keys split over the waves) and many
+# key chunks and query tiles of 32: one, one less one, one, one more, several; D at and below 16, 32 and 64, with
+# and without 16-byte rows; few query tiles (keys split over the waves) and many
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("N,H,D", [(1, 2, 32), (31, 3, 24), (32, 2, 64), (33, 1, 10), (129, 4, 32), (70, 9, 40),
-                                   (100, 8, 64), (160, 4, 6)])
+                                   (100, 8, 64), (160, 4, 6), (65, 4, 16), (100, 4, 8)])
 @pytest.mark.parametrize("mask", ["none", "random", "rows", "inf"])
 def test_attention_any_shape(device, dtype, N, H, D, mask):
     """Triangle attention (a random pair mask; whole rows masked) and attention over one row (mask
@@ -183,6 +226,13 @@ def test_attention_any_shape(device, dtype, N, H, D, mask):
     _within(out, ref, 0.5 * EPS[dtype] * ref.abs() + EPS[torch.float32] * size + 1e-7, f"{dtype} {N} {H} {D} {mask}")
 
 
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("N,D", [(400, 16), (391, 10), (400, 40)])
+def test_attention_one_row_many_heads(device, dtype, N, D):
+    """One row of queries whose 64 heads are tiles enough to leave the keys unsplit, some chunks wholly masked."""
+    test_attention_any_shape(device, dtype, N, 64, D, "inf")
+
+
 # keys split over the waves (H = 2) and not (H = 8); one and two 32-channel tiles
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("N,H,D", [(40, 2, 24), (40, 8, 24), (40, 2, 64), (40, 8, 64)])
@@ -220,7 +270,8 @@ def test_attention_weights_keep_fp32(device, dtype, N, H, D):
     ref = torch.einsum("hk,ikhd->ihd", p, v.double()).reshape(N, 1, H * D)
     size = torch.einsum("hk,ikhd->ihd", p, v.double().abs()).reshape(N, 1, H * D)
     ulp = torch.tensor([2.0**-21, 2.0**-18], dtype=torch.float64).repeat(N // 2)[:, None, None]
-    _within(out, ref.expand(out.shape), (0.5 * EPS[dtype] * ref.abs() + ulp * size).expand(out.shape), f"{dtype} {H} {D}")
+    bound = 0.5 * EPS[dtype] * ref.abs() + ulp * size
+    _within(out, ref.expand(out.shape), bound.expand(out.shape), f"{dtype} {H} {D}", eps=2.0**-21)
 
 
 @pytest.mark.parametrize("dtype", TYPES)
@@ -245,7 +296,8 @@ def test_attention_infinities_in_v(device, dtype, H, D):
     ref, size = ref.reshape(out.shape), size.reshape(out.shape)
     got, ok = out.double().cpu(), ref.isfinite()
     assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
-    _within(got[ok], ref[ok], 0.5 * EPS[dtype] * ref[ok].abs() + EPS[torch.float32] * size[ok] + 1e-7, f"{dtype} {H} {D}")
+    bound = 0.5 * EPS[dtype] * ref.abs() + EPS[torch.float32] * size + 1e-7
+    _within(got[ok], ref[ok], bound[ok], f"{dtype} {H} {D}")
 
 
 # pairs: one, below and past a 16-pair step, several steps per wave; C_z of every chunk count with tails;

@@ -49,6 +49,36 @@ def test_apb_few_tokens_from_x_and_from_qkv_bitwise(device, M):
     assert torch.equal(a, b)
 
 
+# every block shape; remainders of the query and key tiles
+@pytest.mark.parametrize("M", [33, 100, 127, 181, 200, 300, 400, 512])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mask", ["none", "random"])
+def test_apb_few_tokens_bits_of_the_general_kernel(device, M, dtype, mask):
+    """The few-token kernel leaves the bits of the pre-pass and the general kernel: the same tokens at the head of
+    the first size that has no such form, where the keys are split into steps of 32 as well and the tokens added
+    are masked keys (their steps end with an empty sum)."""
+    from triangleops_amd import _native
+    from triangleops_amd.attn_pair_bias.kernel import apb_forward
+
+    big = next(n for n in range(M, 2049) if not _native.apb_single_launch(n, 4, 32))
+    inp = apb_inputs(big, seed=M, mask="random", biases=True, dtype=dtype)
+    inp["mask"][M - 1] = True
+    inp["mask"][M:] = False
+    if mask == "none":
+        inp["mask"][:M] = True
+    d = to_dev(inp, device)
+    pre = tops.attn_pair_bias.precompute(*(d[k] for k in ("WQ", "WK", "WV", "W_ln", "B_ln", "W_proj_z", "B_proj_z")),
+                                         d["H"], d["D"])
+    outs = []
+    for n in (M, big):
+        assert _native.apb_single_launch(n, 4, 32) == (n == M)
+        out = torch.empty(n, 128, device=device, dtype=dtype)
+        apb_forward(d["X"][:n], pre["W_QKV"], d["Z"][:n, :n].contiguous(), pre["W_combined"], pre["sum_W_combined"],
+                    pre["B_const"], out, scale=d["scale"], mask=d["mask"][:n], wqkv_hm=pre["wqkv_hm"])
+        outs.append(out[:M])
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("M", [40, 300])
 def test_apb_few_tokens_qknorm(device, M):
     inp = apb_qkn_inputs(M, seed=M, mask="random")
