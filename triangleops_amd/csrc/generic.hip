@@ -210,8 +210,8 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // keys gives NaN, as torch's softmax does) and keys >= N left out, online softmax in fp32, and
 // O^T += V^T . P^T with the score registers as the operand.  fp32 I/O runs the fp32 MFMA throughout;
 // with 16-bit I/O each fp32 weight enters as three 16-bit terms that hold all its 24 bits (weight_terms).  Three
-// MFMAs: two terms, 16 to 22 bits, are 1-7 % faster in bf16 and 1-20 % in fp16 and lose weight bits (bf16 / fp16,
-// N = 500, 2 heads of 64: 246 / 244 -> 252 / 274 us; 600 tokens x 16 heads of 24: 11.6 / 12.2 -> 12.0 / 12.7);
+// MFMAs: two terms, 16 to 22 bits, are 1-6 % faster in bf16 and 3-25 % in fp16 and lose weight bits (bf16 / fp16,
+// N = 500, 2 heads of 64: 239 / 241 against 253 / 275 us; 600 tokens x 16 heads of 24: 11.5 / 12.2 and 11.7 / 12.6);
 // V and weights converted to the fp32 MFMA, as in fp32 I/O: 392 / 393 and 13.1 / 13.0.
 // K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
 // per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block's
@@ -300,110 +300,127 @@ __global__ __launch_bounds__(KSPL == 1 ? 64 : 256, DP <= 32 ? 4 : 2) void tri_ge
     vd[n] = 16 * hl * HDB + (d < D ? d : D - 1) * ES;  // channels past D are computed and not stored
   }
   const uint32_t bd = (uint32_t)(q - q0) * N * 4 + 64 * hl, kd = tile_perm(col) * HDB;
-  f32x16 o[ND];
-  float m, l;
+  f32x16 o[ND] = {};
+  float m = -INFINITY, l = 0.f;
   const int nch = (N + 31) / 32, c0 = KSPL == 1 ? 0 : wave;
-  auto walk = [&](auto full) __attribute__((always_inline)) {  // full: weights and V enter the products as fp32
+  int c = c0;
+  if (c < nch) load_row(kf, kr, kd + 32 * c * HDB);
+  for (; c < nch; c += KSPL) {
+    const int k0 = 32 * c;
+    // this chunk's V, bias and mask, used after the scores
+    V vf[ND][NV];
+    f32x16 b;
 #pragma unroll
-    for (int n = 0; n < ND; ++n) o[n] = f32x16{};
-    m = -INFINITY;
-    l = 0.f;
-    if (c0 < nch) load_row(kf, kr, kd + 32 * c0 * HDB);
-    for (int c = c0; c < nch; c += KSPL) {
-      const int k0 = 32 * c;
-      // this chunk's V, bias and mask, used after the scores
-      V vf[ND][NV];
-      f32x16 b;
+    for (int v = 0; v < 16; ++v)
 #pragma unroll
-      for (int v = 0; v < 16; ++v)
+      for (int n = 0; n < ND; ++n) vf[n][v / M::VE][v % M::VE] = buffer_load<T>(vr, vd[n] + (k0 + v) * HDB);
+    if (k0 + 32 <= N) {
 #pragma unroll
-        for (int n = 0; n < ND; ++n) vf[n][v / M::VE][v % M::VE] = buffer_load<T>(vr, vd[n] + (k0 + v) * HDB);
-      if (k0 + 32 <= N) {
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 t = buffer_load<f32x4>(br, bd + k0 * 4 + 16 * g);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 t = buffer_load<f32x4>(br, bd + k0 * 4 + 16 * g);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) b[4 * g + e] = t[e];
-        }
-      } else {  // (past the end of a row: the next row or 0, replaced by -inf below)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) b[v] = buffer_load<float>(br, bd + k0 * 4 + 4 * v);
+        for (int e = 0; e < 4; ++e) b[4 * g + e] = t[e];
       }
-      const bool in = k0 + col < N;
-      const bool on = in && (!mrow || mrow[(int64_t)(k0 + col) * sm1] != 0);
-      const uint32_t inb = (uint32_t)__builtin_amdgcn_ballot_w64(in), onb = (uint32_t)__builtin_amdgcn_ballot_w64(on);
-      f32x16 s = {};
+    } else {  // (past the end of a row: the next row or 0, replaced by -inf below)
 #pragma unroll
-      for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
-      if (c + KSPL < nch) load_row(kf, kr, kd + 32 * (c + KSPL) * HDB);
+      for (int v = 0; v < 16; ++v) b[v] = buffer_load<float>(br, bd + k0 * 4 + 4 * v);
+    }
+    const bool in = k0 + col < N;
+    const bool on = in && (!mrow || mrow[(int64_t)(k0 + col) * sm1] != 0);
+    const uint32_t inb = (uint32_t)__builtin_amdgcn_ballot_w64(in), onb = (uint32_t)__builtin_amdgcn_ballot_w64(on);
+    f32x16 s = {};
 #pragma unroll
-      for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], scale, b[v]);
-      if (onb != 0xffffffffu) {  // some key is masked or past the end
-        const uint32_t ib = inb >> (16 * hl), ob = onb >> (16 * hl);
+    for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
+    if (c + KSPL < nch) load_row(kf, kr, kd + 32 * (c + KSPL) * HDB);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          s[v] = (ob >> v) & 1 ? s[v] : (MASK_INF ? -INFINITY : s[v] - 1e9f);
-          s[v] = (ib >> v) & 1 ? s[v] : -INFINITY;
-        }
-      }
-      float cm = s[0];
-#pragma unroll
-      for (int v = 1; v < 16; ++v) cm = fmaxf(cm, s[v]);
-      const float mn = fmaxf(m, halves_max(cm));
-      // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
-      // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
-      const float sh = mn == -INFINITY ? 0.f : mn;
-      const float corr = fast_exp2((m - sh) * kLog2e);
-      m = mn;
-      float lc = 0.f;
+    for (int v = 0; v < 16; ++v) s[v] = fmaf(s[v], scale, b[v]);
+    if (onb != 0xffffffffu) {  // some key is masked or past the end
+      const uint32_t ib = inb >> (16 * hl), ob = onb >> (16 * hl);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        s[v] = fast_exp2(fmaf(s[v] - sh, kLog2e, kShift));
-        lc += s[v];
-      }
-      // the chunk's sums start at zero and are added to the running ones: a chain over all keys rounds
-      // against the whole sum at every key (fp32, N = 291: 18 % more error than sums over a quarter each)
-      l = fmaf(l, corr, lc);
-      auto add = [&](int n, const f32x16& t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[n][v] = fmaf(o[n][v], corr, t[v]);
-      };
-      if constexpr (!full) {
-        V p[3][NV];
-        weight_terms<T>(s, p);
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-          f32x16 t = {};
-#pragma unroll
-          for (int k = 2; k >= 0; --k) {  // the smallest terms first
-#pragma unroll
-            for (int j = 0; j < NV; ++j) t = M::mma(vf[n][j], p[k][j], t);
-            if (k > 0 && kTermScale<T> != 1) t *= 1.f / kTermScale<T>;
-          }
-          add(n, t);
-        }
-      } else {
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-          f32x16 t = {};
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            t = __builtin_amdgcn_mfma_f32_32x32x2f32((float)vf[n][v / M::VE][v % M::VE], s[v], t, 0, 0, 0);
-          add(n, t);
-        }
+        s[v] = (ob >> v) & 1 ? s[v] : (MASK_INF ? -INFINITY : s[v] - 1e9f);
+        s[v] = (ib >> v) & 1 ? s[v] : -INFINITY;
       }
     }
-  };
-  walk(std::bool_constant<sizeof(T) == 4>{});
+    float cm = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) cm = fmaxf(cm, s[v]);
+    const float mn = fmaxf(m, halves_max(cm));
+    // while every key so far is left out, m = mn = -inf: shift by 0 instead, so those keys get
+    // p = 0 and the state stays (m, l, o) = (-inf, 0, 0) instead of NaN
+    const float sh = mn == -INFINITY ? 0.f : mn;
+    const float corr = fast_exp2((m - sh) * kLog2e);
+    m = mn;
+    float lc = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] = fast_exp2(fmaf(s[v] - sh, kLog2e, kShift));
+      lc += s[v];
+    }
+    // the chunk's sums start at zero and are added to the running ones: a chain over all keys rounds
+    // against the whole sum at every key (fp32, N = 291: 18 % more error than sums over a quarter each)
+    l = fmaf(l, corr, lc);
+    auto add = [&](int n, const f32x16& t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[n][v] = fmaf(o[n][v], corr, t[v]);
+    };
+    if constexpr (sizeof(T) == 2) {
+      V p[3][NV];
+      weight_terms<T>(s, p);
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        f32x16 t = {};
+#pragma unroll
+        for (int k = 2; k >= 0; --k) {  // the smallest terms first
+#pragma unroll
+          for (int j = 0; j < NV; ++j) t = M::mma(vf[n][j], p[k][j], t);
+          if (k > 0 && kTermScale<T> != 1) t *= 1.f / kTermScale<T>;
+        }
+        add(n, t);
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        f32x16 t = {};
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          t = __builtin_amdgcn_mfma_f32_32x32x2f32((float)vf[n][v / M::VE][v % M::VE], s[v], t, 0, 0, 0);
+        add(n, t);
+      }
+    }
+  }
   if constexpr (sizeof(T) == 2) {
     // an infinity of V times a weight's zero term is NaN where the weight itself gives an infinity: a tile with an
-    // element that is not finite is done again in fp32 (twice the time for such a tile; 16 FMAs for the others)
+    // element that is not finite takes its products again in fp32, with the weights of the final maximum (some
+    // twice the time for such a tile; 16 FMAs per 32 channels for the others)
     float z = 0.f;
 #pragma unroll
     for (int n = 0; n < ND; ++n)
 #pragma unroll
       for (int v = 0; v < 16; ++v) z = fmaf(o[n][v], 0.f, z);
-    if (__builtin_amdgcn_ballot_w64(z != z) != 0) walk(std::true_type{});
+    if (__builtin_amdgcn_ballot_w64(z != z) != 0) {
+      const float sh = m == -INFINITY ? 0.f : m;
+#pragma unroll
+      for (int n = 0; n < ND; ++n) o[n] = f32x16{};
+      for (c = c0; c < nch; c += KSPL) {
+        const int k0 = 32 * c;
+        load_row(kf, kr, kd + k0 * HDB);
+        f32x16 s = {};
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) s = M::mma(kf[j], qf[j], s);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int key = k0 + 16 * hl + v;
+          s[v] = fmaf(s[v], scale, buffer_load<float>(br, bd + k0 * 4 + 4 * v));
+          if (mrow && key < N && mrow[(int64_t)key * sm1] == 0) s[v] = MASK_INF ? -INFINITY : s[v] - 1e9f;
+          s[v] = key < N ? fast_exp2(fmaf(s[v] - sh, kLog2e, kShift)) : 0.f;
+#pragma unroll
+          for (int n = 0; n < ND; ++n)
+            o[n] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)buffer_load<T>(vr, vd[n] + (k0 + v) * HDB), s[v], o[n],
+                                                        0, 0, 0);
+        }
+      }
+    }
   }
   l = halves_sum(l);
   if constexpr (KSPL == 1) {
