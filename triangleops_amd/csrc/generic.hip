@@ -106,7 +106,7 @@ static int qkv_piece(int D, const void* q, const void* k, const void* v) {
 // as xln), Q / K / V of all heads on the matrix cores (a wave takes 32-row chunks of the weight in
 // turn), the row-shared pair bias from the unrounded LN(x) in fp32 FMAs by the threads that normalise
 // the rows (H is small: an MFMA chunk of 32 features would be mostly empty).  Bound by the matrix
-// cores and the weight reads; N = 200, C = 128, H = 4, D = 32: fp32 130 -> 60 us, bf16 193 -> 29 us
+// cores and the weight reads; N = 200, C = 128, H = 4, D = 32: fp32 130 -> 57 us, bf16 193 -> 29 us
 // against VALU block products; N = 320, C = 256, H = 8 in bf16 3815 -> 210 us.  64 tokens per block
 // (each weight row read half as often) measured slower up to C = 128 (68 and 36 us) and 9 % faster
 // at C = 256.
@@ -214,11 +214,11 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // N = 500, 2 heads of 64: 239 / 241 against 253 / 275 us; 600 tokens x 16 heads of 24: 11.5 / 12.2 and 11.7 / 12.6);
 // V and weights converted to the fp32 MFMA, as in fp32 I/O: 392 / 393 and 13.1 / 13.0.
 // K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
-// per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block's
-// 4 waves take 4 query tiles and share the key reads through L1; with KSPL = 4 they take every 4th chunk
-// of one query tile and merge (m, l, o) through LDS.  Bound by the fp32 MFMAs in fp32 (N = 200, 4 heads
-// of 32: 247 -> 75 us against a query per lane on the VALU, half of the fp32 matrix rate), by the
-// exponentials and the split of the weights in 16 bits (the same in bf16: 245 -> 44 us).
+// per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block is one
+// wave and one query tile, and the tiles of a (row, head) share its key reads through their XCD's L2; with
+// KSPL = 4 a block's 4 waves take every 4th chunk of one query tile and merge (m, l, o) through LDS.  Bound by
+// the fp32 MFMAs in fp32 (N = 200, 4 heads of 32: 246 -> 62 us against a query per lane on the VALU, half of the
+// fp32 matrix rate), by the exponentials and the split of the weights in 16 bits (the same in bf16: 248 -> 37).
 // ---------------------------------------------------------------------------------------------
 // w[0 .. 15] as three terms of the I/O type that add up to all 24 bits: w = t[0] + (t[1] + t[2] / S) / S.  bf16 has
 // fp32's range: S = 1 and the terms are the first, second and last 8 bits.  fp16 has not: S = 2^11, a term's
@@ -692,9 +692,12 @@ static int generic_attention_t(const char* name, const void* q, const void* k, c
                                int64_t R, int64_t N, int H, int D, float scale, hipStream_t st) {
   if (R * N == 0) return TOPS_OK;
   const int64_t rh = R * H;
-  // keys split over the waves while 128-query blocks are fewer than the CUs (80 blocks, 600 tokens x 16
-  // heads of 24, bf16: 14 us against 31; 192 blocks, 1500 tokens: 41 against 75; 400 blocks, N = 100 x 4
-  // heads: 13 against 10; measured with 4 query tiles per block without the split)
+  // Keys split over a block's 4 waves while groups of 4 query tiles are fewer than the CUs: about where the
+  // tiles alone would give every SIMD one wave.  us with the split / without, D = 24, at so many tiles: 304 (600
+  // tokens x 16 heads) bf16 12 / 20, fp32 19 / 32; 752 (1500 x 16) 41 / 58, 54 / 91; 960 (1900 x 16) 63 / 73, 84 /
+  // 115; 576 (N = 96 x 2 heads) 5.4 / 5.6, 7.8 / 7.3.  Past the line: 1152 (N = 96 x 4) 9.4 / 6.9, 14 / 11; 2048
+  // (N = 128 x 4) 14 / 10, 23 / 16.  One long row still gains there up to 1264 tiles in bf16 (2500 x 16: 145 /
+  // 153; 3000 x 16: 217 / 207) and 1504 in fp32 (237 / 263): the line lies where pair rows need it.
   const bool split = rh * ((N + 127) / 128) < num_cus();
   const int64_t blocks = rh * ((N + 31) / 32);
   TOPS_REQUIRE(blocks < (1LL << 31), "%s: too many query blocks", name);
@@ -888,7 +891,7 @@ __global__ __launch_bounds__(256) void apb_generic_bias_kernel(const T* __restri
 // 16-byte chunks 4 j + qd of pair lane % 16, takes the two-pass LayerNorm in registers and feeds the
 // normalised fp32 values to v_mfma_f32_16x16x4_f32 against the fp32 folded weights, which stay in
 // registers over all steps.  The next step's loads are issued before this step's arithmetic.  Bound by
-// the read of Z and the matrix cores together (600 tokens, 16 heads, C_z = 128, bf16: 148 -> 38 us
+// the read of Z and the matrix cores together (600 tokens, 16 heads, C_z = 128, bf16: 148 -> 40 us
 // against LDS tiles and FMAs, 3 TB/s).
 template <typename T, int NKC, bool VEC>
 __global__ __launch_bounds__(256, NKC <= 4 ? 4 : 1) void apb_gen_bias_mma_kernel(const T* __restrict__ Z, int64_t sz0, int64_t sz1,
@@ -1056,9 +1059,9 @@ static int apb_generic_prep_t(const void* X, const void* wqkv, const void* Z, in
 //                 128 NB) pieces of the features' rows.
 //   output phase: tokens (b, i, j0 ..); y, channel-major, is transposed on its way into LDS.  Weights are
 //                 the A operand, so a lane holds 16 consecutive features of one token.
-// Bound by the fp32 MFMAs in fp32 (L = 256, C = 128: input / output phase 174 / 181 -> 91 / 66 us against
-// VALU block products, 94 and 65 TFLOP/s) and by memory and the weight reads in 16-bit types (bf16 L = 512,
-// C = 64: 174 / 320 -> 41 / 39 us, 2.5 TB/s).  Three waves per SIMD: left to itself the compiler takes the
+// Bound by the fp32 MFMAs in fp32 (L = 256, C = 128: input / output phase 174 / 181 -> 90 / 61 us against
+// VALU block products, 95 and 71 TFLOP/s) and by memory and the weight reads in 16-bit types (bf16 L = 512,
+// C = 64: 174 / 320 -> 40 / 41 us, 2.5 TB/s).  Three waves per SIMD: left to itself the compiler takes the
 // registers of one more (46 / 45 us), four spill (63 / 38).
 // ---------------------------------------------------------------------------------------------
 template <typename T, int NB, int NU, bool VEC>
