@@ -209,8 +209,8 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // "+ (-1e9)" in fp32 (triangle attention) or -inf (MASK_INF, attention_pair_bias: a row without valid
 // keys gives NaN, as torch's softmax does) and keys >= N left out, online softmax in fp32, and
 // O^T += V^T . P^T with the score registers as the operand.  fp32 I/O runs the fp32 MFMA throughout;
-// with 16-bit I/O each fp32 weight enters as three 16-bit terms that hold all its 24 bits (weight_terms).  Three
-// MFMAs: two terms, 16 to 22 bits, are 1-6 % faster in bf16 and 3-25 % in fp16 and lose weight bits (bf16 / fp16,
+// with 16-bit I/O each fp32 weight enters as three 16-bit terms that hold all its 24 bits (weight_terms).  Why
+// three: two hold 17 bits in bf16 and 22 down to 8 (small weights) in fp16, for 1-6 % and 3-25 % less time (bf16 / fp16,
 // N = 500, 2 heads of 64: 239 / 241 against 253 / 275 us; 600 tokens x 16 heads of 24: 11.5 / 12.2 and 11.7 / 12.6);
 // V and weights converted to the fp32 MFMA, as in fp32 I/O: 392 / 393 and 13.1 / 13.0.
 // K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
