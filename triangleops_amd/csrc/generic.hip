@@ -210,8 +210,8 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // keys gives NaN, as torch's softmax does) and keys >= N left out, online softmax in fp32, and
 // O^T += V^T . P^T with the score registers as the operand.  fp32 I/O runs the fp32 MFMA throughout;
 // with 16-bit I/O each fp32 weight enters as three 16-bit terms that hold all its 24 bits (weight_terms).  Why
-// three: two hold 17 bits in bf16 and 22 down to 8 (small weights) in fp16, for 1-6 % and 3-25 % less time (bf16 / fp16,
-// N = 500, 2 heads of 64: 239 / 241 against 253 / 275 us; 600 tokens x 16 heads of 24: 11.5 / 12.2 and 11.7 / 12.6);
+// three: two hold 17 bits in bf16 and 22 down to 8 (small weights) in fp16, for 1-6 % and 3-25 % less time (bf16 /
+// fp16, N = 500, 2 heads of 64: 239 / 241 against 253 / 275 us; 600 tokens x 16 heads of 24: 11.5 / 12.2 and 11.7 / 12.6);
 // V and weights converted to the fp32 MFMA, as in fp32 I/O: 392 / 393 and 13.1 / 13.0.
 // K, V and the bias rows come straight from L2 in operand order (K rows as 16-byte chunks, V an element
 // per key and lane, which is the transpose): no LDS and no barrier in the loop.  With KSPL = 1 a block is one
@@ -222,7 +222,8 @@ __global__ __launch_bounds__(256) void tri_generic_prep_kernel(const T* __restri
 // ---------------------------------------------------------------------------------------------
 // w[0 .. 15] as three terms of the I/O type that add up to all 24 bits: w = t[0] + (t[1] + t[2] / S) / S.  bf16 has
 // fp32's range: S = 1 and the terms are the first, second and last 8 bits.  fp16 has not: S = 2^11, a term's
-// width, keeps the rests clear of its denormals.
+// width, keeps the rests clear of its denormals (with the largest weight at 2^15, the others are whole down to
+// 2^-38 of it and off by less than 2^-61 of it below).
 template <typename T>
 constexpr int kTermScale = std::is_same<T, _Float16>::value ? 1 << 11 : 1;
 template <typename T, typename V, int NV>
